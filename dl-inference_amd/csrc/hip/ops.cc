@@ -4,6 +4,7 @@
 #include <string>
 
 #include "../kernels/conv_small.h"
+#include "../kernels/packed_attention.h"
 #include "runtime.h"
 
 namespace dli::hip {
@@ -74,6 +75,14 @@ FloatKernels k_kv_append("attention", "kv_append");
 FloatKernels k_conv2d("conv", "conv2d");
 DeviceKernel k_flash_attention("flash_attention", "flash_attention_bf16");
 DeviceKernel k_flash_attention_q32("flash_attention", "flash_attention_bf16_q32");
+DeviceKernel k_packed_paged64("packed_attention", "packed_attention_paged_d64");
+DeviceKernel k_packed_paged64_r128("packed_attention", "packed_attention_paged_d64_r128");
+DeviceKernel k_packed_paged128("packed_attention", "packed_attention_paged_d128");
+DeviceKernel k_packed_paged128_r128("packed_attention", "packed_attention_paged_d128_r128");
+DeviceKernel k_packed_dense128("packed_attention", "packed_attention_dense_d128");
+DeviceKernel k_packed_dense128_r128("packed_attention", "packed_attention_dense_d128_r128");
+DeviceKernel k_packed_merge64("packed_attention", "packed_attention_merge_d64");
+DeviceKernel k_packed_merge128("packed_attention", "packed_attention_merge_d128");
 DeviceKernel k_mfma_linear64("mfma_gemm", "mfma_linear_f32_t64");
 DeviceKernel k_mfma_linear128("mfma_gemm", "mfma_linear_f32_t128");
 DeviceKernel k_mfma_matmul64("mfma_gemm", "mfma_matmul_f32_t64");
@@ -133,6 +142,32 @@ int unary(FloatKernels& kernels, const char* op, int dtype, const void* x, void*
 }
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
+
+// ---- packed-row attention (packed_attention.hip) ------------------------------------------------
+// Rows (queries x heads of a KV group) per workgroup: 128, or 64 for units of at most 64 rows.
+int64_t packedTile(int64_t rows) { return rows > 64 ? 128 : 64; }
+
+// Key splits for `blocks` row tiles over all (sequence, KV head) pairs: about two workgroups per
+// CU, each with at least two 64-key tiles of the cache's capacity.
+int64_t packedSplits(int64_t blocks, int64_t capacity) {
+  const int64_t by_tiles = (capacity + dk::kPackedTileK - 1) / dk::kPackedTileK / 2;
+  int64_t splits = blocks > 0 ? 512 / blocks : 1;
+  if (splits > by_tiles) splits = by_tiles;
+  return splits < 1 ? 1 : (splits > 64 ? 64 : splits);
+}
+
+size_t packedPartialBytes(int64_t rows, int64_t head_dim, int64_t splits) {
+  return static_cast<size_t>(rows * splits * (head_dim + 2)) * sizeof(float);
+}
+
+// Forms that the packed kernels take (others run on the generic kernels).
+bool packedForm(int dtype, int64_t batch, int64_t q_heads, int64_t kv_heads, int64_t seq_q,
+                int64_t keys, const void* q, const void* k, const void* v, const void* out) {
+  const int64_t limit = int64_t{1} << 30;
+  return dtype == DLI_BF16 && batch * kv_heads <= 65535 && keys > 0 && keys < limit &&
+         seq_q < limit && seq_q * (q_heads / kv_heads) < limit && aligned16(q) && aligned16(k) &&
+         aligned16(v) && aligned16(out);
+}
 
 }  // namespace
 
@@ -577,6 +612,27 @@ static int attentionImpl(int dtype, const void* q, const void* k, const void* v,
                   {256}, 0, stream, q, k, v, out, q_heads, kv_heads, seq_q, seq_k, causal,
                   scale * log2e, out_bshd);
   }
+  // bf16 with head_dim 128: the packed-row MFMA kernel (fewer than 16 queries over long keys stay
+  // on the row kernel, whose waves split the heads; the packed kernel has no key splits here)
+  if (!out_bshd && head_dim == 128 && seq_q >= 16 &&
+      packedForm(dtype, batch, q_heads, kv_heads, seq_q, seq_k, q, k, v, out)) {
+    dk::PackedAttentionArgs a{};
+    a.q = static_cast<const uint16_t*>(q);
+    a.k = static_cast<const uint16_t*>(k);
+    a.v = static_cast<const uint16_t*>(v);
+    a.out = static_cast<uint16_t*>(out);
+    a.q_heads = static_cast<int32_t>(q_heads);
+    a.kv_heads = static_cast<int32_t>(kv_heads);
+    a.seq_q = static_cast<int32_t>(seq_q);
+    a.keys = static_cast<int32_t>(seq_k);
+    a.causal = causal;
+    a.splits = 1;
+    a.scale_log2 = scale * 1.4426950408889634f;
+    const int64_t unit_rows = seq_q * (q_heads / kv_heads), tile = packedTile(unit_rows);
+    return launch(tile == 128 ? k_packed_dense128_r128 : k_packed_dense128,
+                  {blocksFor(unit_rows, tile), static_cast<unsigned>(batch * kv_heads)}, {256}, 0,
+                  stream, a);
+  }
   if (out_bshd)
     return badArg("attention", "a [B, S, H, D] output needs bf16, head_dim 64, seq_k > 0 and "
                                "16-byte aligned tensors (the flash kernel)");
@@ -636,12 +692,14 @@ size_t dli_hip_paged_attention_workspace(int64_t batch, int64_t q_heads, int64_t
   return decodeAttentionWorkspace(batch, q_heads, seq_q, head_dim, max_tokens);
 }
 
-int dli_hip_paged_attention(int dtype, const void* q, const void* key_pool,
-                            const void* value_pool, const int32_t* block_table, void* out,
-                            int64_t batch, int64_t q_heads, int64_t kv_heads, int64_t seq_q,
-                            int64_t head_dim, int64_t block_size, int64_t max_blocks, int64_t past,
-                            const void* positions, int positions_dtype, int causal, float scale,
-                            int splits, void* workspace, size_t workspace_bytes, void* stream) {
+// workspace: the decode kernels' (one query per sequence); partials: the packed kernels' key splits
+static int pagedAttention(int dtype, const void* q, const void* key_pool, const void* value_pool,
+                          const int32_t* block_table, void* out, int64_t batch, int64_t q_heads,
+                          int64_t kv_heads, int64_t seq_q, int64_t head_dim, int64_t block_size,
+                          int64_t max_blocks, int64_t past, const void* positions,
+                          int positions_dtype, int causal, float scale, int splits,
+                          void* workspace, size_t workspace_bytes, void* partials,
+                          size_t partial_bytes, void* stream) {
   DeviceKernel* ka = k_paged_attention.pick(dtype);
   if (ka == nullptr) return badDtype("paged_attention", dtype);
   if (head_dim <= 0 || head_dim > 256) return badArg("paged_attention", "head_dim must be in [1, 256]");
@@ -664,9 +722,86 @@ int dli_hip_paged_attention(int dtype, const void* q, const void* key_pool,
     if (rc != 1) return rc;
   }
   const int pos64 = positions_dtype == DLI_I64 ? 1 : 0;
+  // several queries per sequence: the packed-row MFMA kernels (64-key tiles inside cache blocks)
+  if (seq_q > 1 && (head_dim == 64 || head_dim == 128) && block_size % dk::kPackedTileK == 0 &&
+      block_size < (int64_t{1} << 30) && max_blocks < (int64_t{1} << 30) &&
+      packedForm(dtype, batch, q_heads, kv_heads, seq_q, max_blocks * block_size, q, key_pool,
+                 value_pool, out)) {
+    const int64_t unit_rows = seq_q * (q_heads / kv_heads), tile = packedTile(unit_rows);
+    const int64_t units = batch * kv_heads, blocks = (unit_rows + tile - 1) / tile;
+    int64_t n = packedSplits(blocks * units, max_blocks * block_size);
+    while (n > 1 &&
+           (partials == nullptr || partial_bytes < packedPartialBytes(rows, head_dim, n)))
+      --n;
+    dk::PackedAttentionArgs a{};
+    a.q = static_cast<const uint16_t*>(q);
+    a.k = static_cast<const uint16_t*>(key_pool);
+    a.v = static_cast<const uint16_t*>(value_pool);
+    a.block_table = block_table;
+    a.positions = positions;
+    a.out = static_cast<uint16_t*>(out);
+    a.part_o = static_cast<float*>(partials);
+    a.part_ml = n > 1 ? a.part_o + rows * n * head_dim : nullptr;
+    a.past = past;
+    a.max_blocks = max_blocks;
+    a.pos64 = pos64;
+    a.block_size = static_cast<int32_t>(block_size);
+    a.q_heads = static_cast<int32_t>(q_heads);
+    a.kv_heads = static_cast<int32_t>(kv_heads);
+    a.seq_q = static_cast<int32_t>(seq_q);
+    a.keys = static_cast<int32_t>(max_blocks * block_size);
+    a.causal = causal;
+    a.splits = static_cast<int32_t>(n);
+    a.scale_log2 = scale * 1.4426950408889634f;
+    const bool d64 = head_dim == 64, big = tile == 128;
+    DeviceKernel& k = d64 ? (big ? k_packed_paged64_r128 : k_packed_paged64)
+                          : (big ? k_packed_paged128_r128 : k_packed_paged128);
+    if (int rc = launch(k, {static_cast<unsigned>(blocks), static_cast<unsigned>(units),
+                            static_cast<unsigned>(n)},
+                        {256}, 0, stream, a))
+      return rc;
+    if (n == 1) return 0;
+    return launch(d64 ? k_packed_merge64 : k_packed_merge128,
+                  {blocksFor(rows, 1024 / head_dim)}, {256}, 0, stream, a,
+                  static_cast<int>(units));
+  }
   return launch(*ka, {static_cast<unsigned>(rows)}, {64}, 0, stream, q, key_pool, value_pool,
                 block_table, out, batch, q_heads, kv_heads, seq_q, head_dim, block_size, max_blocks,
                 past, positions, pos64, causal, scale);
+}
+
+int dli_hip_paged_attention(int dtype, const void* q, const void* key_pool,
+                            const void* value_pool, const int32_t* block_table, void* out,
+                            int64_t batch, int64_t q_heads, int64_t kv_heads, int64_t seq_q,
+                            int64_t head_dim, int64_t block_size, int64_t max_blocks, int64_t past,
+                            const void* positions, int positions_dtype, int causal, float scale,
+                            int splits, void* workspace, size_t workspace_bytes, void* stream) {
+  return pagedAttention(dtype, q, key_pool, value_pool, block_table, out, batch, q_heads, kv_heads,
+                        seq_q, head_dim, block_size, max_blocks, past, positions, positions_dtype,
+                        causal, scale, splits, workspace, workspace_bytes, nullptr, 0, stream);
+}
+
+size_t dli_hip_chunk_attention_workspace(int dtype, int64_t batch, int64_t q_heads, int64_t seq_q,
+                                         int64_t head_dim, int64_t max_tokens) {
+  if (dtype != DLI_BF16 || batch <= 0 || q_heads <= 0 || seq_q <= 1 ||
+      (head_dim != 64 && head_dim != 128))
+    return 0;
+  // fewer splits than this holds are used when the KV heads cut the rows into more tiles
+  const int64_t rows = batch * q_heads * seq_q;
+  const int64_t splits = packedSplits((rows + 127) / 128, max_tokens);
+  return splits > 1 ? packedPartialBytes(rows, head_dim, splits) : 0;
+}
+
+int dli_hip_chunk_attention(int dtype, const void* q, const void* key_pool,
+                            const void* value_pool, const int32_t* block_table, void* out,
+                            int64_t batch, int64_t q_heads, int64_t kv_heads, int64_t seq_q,
+                            int64_t head_dim, int64_t block_size, int64_t max_blocks, int64_t past,
+                            const void* positions, int positions_dtype, int causal, float scale,
+                            void* workspace, size_t workspace_bytes, void* stream) {
+  if (seq_q == 1) return badArg("chunk_attention", "one query per sequence: paged_attention");
+  return pagedAttention(dtype, q, key_pool, value_pool, block_table, out, batch, q_heads, kv_heads,
+                        seq_q, head_dim, block_size, max_blocks, past, positions, positions_dtype,
+                        causal, scale, 0, nullptr, 0, workspace, workspace_bytes, stream);
 }
 
 int dli_hip_argmax(int dtype, const void* x, int64_t* ids, int64_t rows, int64_t width,

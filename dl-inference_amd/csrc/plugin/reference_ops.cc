@@ -281,12 +281,26 @@ class AttentionOp final : public Operator {
     }
     if (bshd) throw std::invalid_argument("attention output_layout \"bshd\" needs an empty cache");
     const KVCacheEntry& e = *cache.get(cache_name);
+    const auto* table = static_cast<const std::int32_t*>(ptr(e.block_table));
+    const void* pos = positions ? ptr(*positions) : nullptr;
+    const int pos_dt = positions ? hipDtype(positions->dtype()) : DLI_I64;
+    if (Sq > 1) {
+      const std::size_t bytes =
+          dli_hip_chunk_attention_workspace(dt, B, Hq, Sq, D, e.capacity());
+      Tensor ws;  // partial results of the key splits (from the caching allocator)
+      if (bytes > 0)
+        ws = allocLike(DType::Float32, {static_cast<std::int64_t>(bytes / sizeof(float))}, q);
+      check(dli_hip_chunk_attention(dt, ptr(q), ptr(e.key_pool), ptr(e.value_pool), table,
+                                    ptr(*out[0]), B, Hq, Hkv, Sq, D, e.block_size, e.max_blocks,
+                                    past, pos, pos_dt, causal ? 1 : 0, scale,
+                                    bytes > 0 ? ptr(ws) : nullptr, bytes, ctx.stream),
+            type());
+      return;
+    }
     const std::size_t ws_bytes = dli_hip_paged_attention_workspace(B, Hq, Sq, D, e.capacity());
     check(dli_hip_paged_attention(
-              dt, ptr(q), ptr(e.key_pool), ptr(e.value_pool),
-              static_cast<const std::int32_t*>(ptr(e.block_table)), ptr(*out[0]), B, Hq, Hkv, Sq,
-              D, e.block_size, e.max_blocks, past, positions ? ptr(*positions) : nullptr,
-              positions ? hipDtype(positions->dtype()) : DLI_I64, causal ? 1 : 0, scale, 0,
+              dt, ptr(q), ptr(e.key_pool), ptr(e.value_pool), table, ptr(*out[0]), B, Hq, Hkv, Sq,
+              D, e.block_size, e.max_blocks, past, pos, pos_dt, causal ? 1 : 0, scale, 0,
               workspace_.get(ws_bytes, q.deviceId(), ctx.stream), ws_bytes, ctx.stream),
           type());
   }

@@ -86,6 +86,9 @@ _SIGNATURES = {
     "dli_hip_paged_attention_workspace": [_i64] * 5,
     "dli_hip_paged_attention": [_int, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p]
     + [_i64] * 8 + [_c_void_p, _int, _int, _float, _int, _c_void_p, _size, _c_void_p],
+    "dli_hip_chunk_attention_workspace": [_int] + [_i64] * 5,
+    "dli_hip_chunk_attention": [_int, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p]
+    + [_i64] * 8 + [_c_void_p, _int, _int, _float, _c_void_p, _size, _c_void_p],
     "dli_hip_argmax": [_int, _c_void_p, _c_void_p, _i64, _i64, _c_void_p],
     "dli_hip_splitk_workspace": [_i64, _i64, _int],
     "dli_hip_qkv_rope_append": [_c_void_p] * 6 + [_i64, _c_void_p, _int] + [_c_void_p] * 4
@@ -120,6 +123,7 @@ _RESTYPES = {
     "dli_hip_linear_workspace": _size,
     "dli_hip_conv2d_workspace": _size,
     "dli_hip_paged_attention_workspace": _size,
+    "dli_hip_chunk_attention_workspace": _size,
     "dli_hip_splitk_workspace": _size,
     "dli_hip_qkv_rope_append_workspace": _size,
     "dli_hip_lm_head_argmax_workspace": _size,

@@ -277,6 +277,19 @@ int dli_hip_paged_attention(int dtype, const void* q, const void* key_pool,
                             int causal, float scale, int splits, void* workspace,
                             size_t workspace_bytes, void* stream);
 
+/* dli_hip_paged_attention for several queries per sequence (seq_q > 1), with scratch for the
+ * kernels' key splits: `workspace` of any content (size from dli_hip_chunk_attention_workspace; a
+ * smaller one or NULL means fewer splits), its content afterwards unspecified. */
+size_t dli_hip_chunk_attention_workspace(int dtype, int64_t batch, int64_t q_heads, int64_t seq_q,
+                                         int64_t head_dim, int64_t max_tokens);
+int dli_hip_chunk_attention(int dtype, const void* q, const void* key_pool,
+                            const void* value_pool, const int32_t* block_table, void* out,
+                            int64_t batch, int64_t q_heads, int64_t kv_heads, int64_t seq_q,
+                            int64_t head_dim, int64_t block_size, int64_t max_blocks,
+                            int64_t past, const void* positions, int positions_dtype,
+                            int causal, float scale, void* workspace, size_t workspace_bytes,
+                            void* stream);
+
 /* ids[r] = first index of the maximum of row r of x [rows, width] (torch.argmax rule). */
 int dli_hip_argmax(int dtype, const void* x, int64_t* ids, int64_t rows, int64_t width,
                    void* stream);

@@ -1,0 +1,121 @@
+"""Attention of several query tokens per sequence on the packed-row MFMA kernels (gfx950): over
+the paged cache and, for head_dim 128, over contiguous keys, against the float64 oracle."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import ops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+# bf16 output: 2^-9 of the value for its rounding, doubled for the fp32 sums before it
+REL = 4e-3
+
+
+def rand(shape, seed):
+    g = torch.Generator().manual_seed(seed)
+    return torch.randn(shape, generator=g).to(torch.bfloat16).to(DEV)
+
+
+def to_np(t):
+    return t.double().cpu().numpy()
+
+
+def run_attention(inputs, attrs, engine):
+    import json
+
+    import dli
+
+    names = list(inputs)
+    graph = dli.Graph.from_json(json.dumps({
+        "format": "dli.graph.v1", "model_type": "attention", "inputs": names, "outputs": ["out"],
+        "nodes": [{"name": "a", "op": "attention", "inputs": names, "outputs": ["out"],
+                   "attrs": attrs}]}))
+    return engine.run(graph, inputs)["out"]
+
+
+def check(out, ref):
+    out = to_np(out)
+    assert np.isfinite(out).all()
+    assert np.linalg.norm(out - ref) <= REL * np.linalg.norm(ref)
+    assert np.abs(out - ref).max() <= 2 * REL * max(1.0, np.abs(ref).max())
+
+
+def paged_case(hq, hkv, d, sq, past, causal, block_size=64, capacity=None, stale=0.0):
+    """Engine with `past[b]` random tokens cached per sequence, and the call's result next to the
+    oracle's inputs. stale: what unused cache slots hold."""
+    import dli
+
+    batch = len(past)
+    engine = dli.Engine().load_plugin()
+    engine.configure_kv_cache(block_size=block_size, max_seq_len=capacity or max(past) + sq)
+    engine.reserve_kv_cache("L", "bfloat16", batch, hkv, d)
+    entry = engine.kv_cache_entry("L")
+    entry["key_pool"].fill_(stale)
+    entry["value_pool"].fill_(stale)
+    hist_k, hist_v = rand((batch, hkv, max(past), d), 1), rand((batch, hkv, max(past), d), 2)
+    table = entry["block_table"].cpu().numpy()
+    for b in range(batch):
+        for j in range(past[b]):
+            blk, slot = table[b, j // block_size], j % block_size
+            entry["key_pool"][blk, :, slot] = hist_k[b, :, j]
+            entry["value_pool"][blk, :, :, slot] = hist_v[b, :, j]
+    q, k, v = (rand((batch, h, sq, d), 3 + i) for i, h in enumerate((hq, hkv, hkv)))
+    pos = torch.tensor(past, dtype=torch.int32, device=DEV)
+    return engine, {"q": q, "k": k, "v": v, "positions": pos}, hist_k, hist_v
+
+
+def check_paged(engine, inputs, hist_k, hist_v, past, causal):
+    out = run_attention(inputs, {"causal": causal, "kv_cache": "L"}, engine)
+    q, k, v = inputs["q"], inputs["k"], inputs["v"]
+    for b, n in enumerate(past):
+        keys = np.concatenate([to_np(hist_k[b:b + 1, :, :n]), to_np(k[b:b + 1])], 2)
+        vals = np.concatenate([to_np(hist_v[b:b + 1, :, :n]), to_np(v[b:b + 1])], 2)
+        check(out[b:b + 1], ops.attention(to_np(q[b:b + 1]), keys, vals, causal=causal))
+
+
+# rows per KV head (sq * group) on both sides of the 64- and 128-row tiles; contexts on both sides
+# of a 64-key tile, few enough for one key split and long enough for many
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("hq,hkv,sq,past,causal", [
+    (14, 2, 2, [64], True), (28, 4, 9, [63, 1], True), (28, 4, 10, [130, 257], True),
+    (4, 4, 64, [0, 65], True), (4, 4, 65, [5], True), (6, 1, 43, [127, 700], False),
+    (3, 3, 129, [1000, 500], True)])
+def test_paged_chunk(d, hq, hkv, sq, past, causal):
+    check_paged(*paged_case(hq, hkv, d, sq, past, causal), past, causal)
+
+
+def test_paged_chunk_large_blocks_and_spare_capacity():
+    """Cache blocks of two tiles; a capacity far above the tokens held (empty key splits)."""
+    check_paged(*paged_case(14, 2, 64, 5, [90, 30], True, block_size=128, capacity=4096), [90, 30],
+                True)
+
+
+@pytest.mark.parametrize("d", [64, 128])
+def test_paged_chunk_never_reads_hidden_values(d):
+    """NaN in unused cache slots, and infinite or NaN values of the chunk's last token: rows that
+    do not see them are unaffected."""
+    past, sq = [70, 200], 20
+    engine, inputs, hist_k, hist_v = paged_case(14, 2, d, sq, past, True, stale=float("nan"))
+    check_paged(engine, inputs, hist_k, hist_v, past, True)
+    clean = run_attention(inputs, {"causal": True, "kv_cache": "L"}, engine)
+    inputs["v"][:, :, -1, ::2] = float("inf")
+    inputs["v"][:, :, -1, 1::2] = float("nan")
+    out = run_attention(inputs, {"causal": True, "kv_cache": "L"}, engine)
+    err = (out[:, :, :-1].double() - clean[:, :, :-1].double()).norm()
+    assert err <= REL * clean[:, :, :-1].double().norm()
+    assert torch.isinf(out[:, :, -1, ::2]).all() and torch.isnan(out[:, :, -1, 1::2]).all()
+
+
+@pytest.mark.parametrize("sq,sk,hq,hkv,causal", [(16, 16, 4, 4, True), (18, 100, 28, 4, True),
+                                                 (77, 77, 7, 1, True), (40, 130, 6, 2, False),
+                                                 (130, 65, 2, 2, True)])
+def test_dense_head_dim_128(sq, sk, hq, hkv, causal):
+    import dli
+
+    q, k, v = rand((2, hq, sq, 128), 11), rand((2, hkv, sk, 128), 12), rand((2, hkv, sk, 128), 13)
+    out = run_attention({"q": q, "k": k, "v": v}, {"causal": causal}, dli.Engine().load_plugin())
+    if causal and sq > sk:  # queries before the first key: zeros
+        assert (out[:, :, :sq - sk] == 0).all()
+        out, q = out[:, :, sq - sk:], q[:, :, sq - sk:]
+    check(out, ops.attention(to_np(q), to_np(k), to_np(v), causal=causal))
