@@ -42,28 +42,15 @@ DeviceKernel k_res_norm("decode", "residual_rms_norm");
 DeviceKernel k_argmax_final("decode", "argmax_finalize");
 // many-row (prefill) forms of linear_residual and gate_up_silu: tiled MFMA GEMMs with the same
 // epilogues (mfma_gemm.hip)
-DeviceKernel k_mfma_linres64("mfma_gemm", "mfma_linear_residual_bf16_t64");
-DeviceKernel k_mfma_linres128("mfma_gemm", "mfma_linear_residual_bf16_t128");
-DeviceKernel k_mfma_gu64("mfma_gemm", "mfma_gate_up_silu_bf16_t64");
-DeviceKernel k_mfma_gu128("mfma_gemm", "mfma_gate_up_silu_bf16_t128");
-DeviceKernel k_mfma_gu_stream("mfma_gemm", "mfma_gate_up_silu_bf16_stream_t64");
-DeviceKernel k_mfma_qkvh64("mfma_gemm", "mfma_qkv_heads_bf16_t64");
-DeviceKernel k_mfma_qkvh128("mfma_gemm", "mfma_qkv_heads_bf16_t128");
-
-// Tiled launch of those: 128 x 128 tiles once they alone give every CU a workgroup, else 64 x 64;
-// grid (column tiles, row tiles).
-bool tiledGrid(int64_t rows, int64_t cols, bool* big, unsigned (&grid)[2]) {
-  // 128 x 128 tiles once there are enough of them to fill most of the 256 CUs (measured at
-  // 896 columns: 2048 rows / 112 tiles ran faster in 64 x 64 tiles, 4096 rows / 224 tiles in
-  // 128 x 128 tiles)
-  *big = ((rows + 127) / 128) * ((cols + 127) / 128) >= 168;
-  const int64_t tile = *big ? 128 : 64;
-  const int64_t gx = (cols + tile - 1) / tile, gy = (rows + tile - 1) / tile;
-  if (gy > 65535 || gx > (int64_t{1} << 31)) return false;
-  grid[0] = static_cast<unsigned>(gx);
-  grid[1] = static_cast<unsigned>(gy);
-  return true;
-}
+// (indexed by TileForm16)
+DeviceKernel k_mfma_gu[4] = {{"mfma_gemm", "mfma_gate_up_silu_bf16_t64"},
+                             {"mfma_gemm", "mfma_gate_up_silu_bf16_t64_g2"},
+                             {"mfma_gemm", "mfma_gate_up_silu_bf16_t64_stream"},
+                             {"mfma_gemm", "mfma_gate_up_silu_bf16_t128"}};
+DeviceKernel k_mfma_qkvh[4] = {{"mfma_gemm", "mfma_qkv_heads_bf16_t64"},
+                               {"mfma_gemm", "mfma_qkv_heads_bf16_t64_g2"},
+                               {"mfma_gemm", "mfma_qkv_heads_bf16_t64_stream"},
+                               {"mfma_gemm", "mfma_qkv_heads_bf16_t128"}};
 DeviceKernel k_dec_attn("attention", "decode_attention_d64");
 DeviceKernel k_dec_attn128("attention", "decode_attention_d128");
 
@@ -130,9 +117,6 @@ int partialThenResidual(const char* op, const void* x, const void* w, const void
 // ops.cc: the tiled bf16 GEMM for decode-sized m (K split into a workspace)
 bool tiledDecodeLinear(int64_t m, int64_t n);
 int64_t bf16Splits(int64_t m, int64_t n, int64_t k);
-int tiledBf16(const void* x, const void* w, const void* bias, const void* residual, void* out,
-              int64_t m, int64_t n, int64_t k, void* workspace, size_t workspace_bytes,
-              void* stream);
 int tiledBf16Parts(const void* x, const void* w, int64_t m, int64_t n, int64_t k,
                    void* workspace, size_t workspace_bytes, void* stream, int* parts_out);
 
@@ -296,6 +280,24 @@ int dli_hip_qkv_rope_append_ws(const void* hidden, const void* norm_weight, cons
                 static_cast<int>(head_dim));
 }
 
+size_t dli_hip_linear_residual_rows_workspace(int64_t m, int64_t n, int64_t k) {
+  return m > 64 && n > 0 && k > 0 ? tiled16Workspace(m, n, k) : 0;
+}
+
+int dli_hip_linear_residual_rows(const void* x, const void* w, const void* bias,
+                                 const void* residual, void* out, int64_t m, int64_t n, int64_t k,
+                                 void* workspace, size_t workspace_bytes, void* stream) {
+  const char* op = "linear_residual";
+  if (m <= 64) return bad(op, "linear_residual_rows is for more than 64 rows");
+  if (n <= 0) return bad(op, "n must be positive");
+  if (k <= 0 || k % 8 != 0) return bad(op, "k must be a positive multiple of 8");
+  if (!aligned16(x) || !aligned16(w)) return bad(op, "x and w must be 16-byte aligned");
+  Dim3 grid, block;
+  if (!tileLaunch16(tileForm16(m, n), m, n, &grid, &block)) return bad(op, "too many rows");
+  return tiled16(DLI_BF16, x, w, bias, residual, out, m, n, k, 0, 0, workspace, workspace_bytes,
+                 stream);
+}
+
 int dli_hip_linear_residual(const void* x, const void* w, const void* bias, const void* residual,
                             void* out, int64_t m, int64_t n, int64_t k, int splits,
                             void* workspace, size_t workspace_bytes, void* stream) {
@@ -306,18 +308,11 @@ int dli_hip_linear_residual(const void* x, const void* w, const void* bias, cons
   if (m > 8 && m <= 64 && n > 1024 && k % 8 == 0 && aligned16(x) && aligned16(w) &&
       tiledDecodeLinear(m, n)) {
     if (splits < 1) return bad(op, "splits must be positive");
-    return tiledBf16(x, w, bias, residual, out, m, n, k, workspace, workspace_bytes, stream);
+    return tiled16(DLI_BF16, x, w, bias, residual, out, m, n, k, 0, 0, workspace,
+                   workspace_bytes, stream);
   }
-  if (m > 64) {  // many rows (a prompt): one tiled MFMA GEMM, no split
-    if (n <= 0) return bad(op, "n must be positive");
-    if (k <= 0 || k % 8 != 0) return bad(op, "k must be a positive multiple of 8");
-    if (!aligned16(x) || !aligned16(w)) return bad(op, "x and w must be 16-byte aligned");
-    bool big = false;
-    unsigned grid[2];
-    if (!tiledGrid(m, n, &big, grid)) return bad(op, "too many rows");
-    return launch(big ? k_mfma_linres128 : k_mfma_linres64, {grid[0], grid[1]}, {256}, 0,
-                  stream, x, w, bias, residual, out, m, n, k);
-  }
+  if (m > 64)  // many rows (a prompt): one tiled MFMA GEMM, no split
+    return dli_hip_linear_residual_rows(x, w, bias, residual, out, m, n, k, nullptr, 0, stream);
   if (int rc = checkSkinny(op, m, k)) return rc;
   if (n <= 0) return bad(op, "n must be positive");
   if (splits < 1 || splits > k / 64 || splits > kMaxNormSplits)
@@ -385,14 +380,11 @@ int dli_hip_gate_up_silu(const void* hidden, const void* norm_weight, const void
       return bad(op, "the RMSNorm prologue is for at most 64 rows (normalize first)");
     if (!aligned16(hidden) || !aligned16(w_gate_up))
       return bad(op, "hidden and w_gate_up must be 16-byte aligned");
-    if (m <= 64)  // decode-sized rows: 64 x 64 tiles, 128-wide K slices
-      return launch(k_mfma_gu_stream, {static_cast<unsigned>((2 * ffn + 63) / 64), 1}, {256}, 0,
-                    stream, hidden, w_gate_up, out, m, ffn, hidden_size);
-    bool big = false;
-    unsigned grid[2];
-    if (!tiledGrid(m, 2 * ffn, &big, grid)) return bad(op, "too many rows");
-    return launch(big ? k_mfma_gu128 : k_mfma_gu64, {grid[0], grid[1]}, {256}, 0, stream, hidden,
-                  w_gate_up, out, m, ffn, hidden_size);
+    const TileForm16 form = tileForm16(m, 2 * ffn);
+    Dim3 grid, block;
+    if (!tileLaunch16(form, m, 2 * ffn, &grid, &block)) return bad(op, "too many rows");
+    return launch(k_mfma_gu[static_cast<int>(form)], grid, block, 0, stream, hidden, w_gate_up,
+                  out, m, ffn, hidden_size);
   }
   if (int rc = checkSkinny(op, m, hidden_size)) return rc;
   if (ffn <= 0 || ffn % 16 != 0) return bad(op, "ffn must be a positive multiple of 16");
@@ -431,10 +423,10 @@ int dli_hip_qkv_rope_heads(const void* x, const void* w_qkv, const void* b_qkv, 
   const int64_t n = (q_heads + 2 * kv_heads) * head_dim;
   if (m >= (int64_t{1} << 31) || n >= (int64_t{1} << 31))
     return bad(op, "batch * seq and the q|k|v width must be below 2^31");
-  bool big = false;
-  unsigned grid[2];
-  if (!tiledGrid(m, n, &big, grid)) return bad(op, "too many rows");
-  return launch(big ? k_mfma_qkvh128 : k_mfma_qkvh64, {grid[0], grid[1]}, {256}, 0, stream, x,
+  const TileForm16 form = tileForm16(m, n);
+  Dim3 grid, block;
+  if (!tileLaunch16(form, m, n, &grid, &block)) return bad(op, "too many rows");
+  return launch(k_mfma_qkvh[static_cast<int>(form)], grid, block, 0, stream, x,
                 w_qkv, b_qkv, cos, sin, max_pos, q_out, k_out, v_out, m, hidden_size, seq,
                 start_pos, static_cast<int>(q_heads), static_cast<int>(kv_heads),
                 static_cast<int>(head_dim));

@@ -66,9 +66,19 @@ FloatKernels k_rms_norm("norm", "rms_norm");
 DeviceKernel k_rms_norm_rows("norm", "rms_norm_rows_bf16_k");
 DeviceKernel k_kv_append_tiles("attention", "kv_append_tiles_bf16_k");
 FloatKernels k_gemm("gemm", "gemm_tiled");
-DeviceKernel k_skinny1("gemm", "skinny_linear_m1");
-DeviceKernel k_skinny2("gemm", "skinny_linear_m2");
-DeviceKernel k_skinny4("gemm", "skinny_linear_m4");
+// [16 waves][16 MB rows: MB = 1, 2, 4]
+DeviceKernel k_skinny_bf16[2][3] = {{{"gemm", "skinny_linear_bf16_m1"},
+                                     {"gemm", "skinny_linear_bf16_m2"},
+                                     {"gemm", "skinny_linear_bf16_m4"}},
+                                    {{"gemm", "skinny_linear_bf16_w16_m1"},
+                                     {"gemm", "skinny_linear_bf16_w16_m2"},
+                                     {"gemm", "skinny_linear_bf16_w16_m4"}}};
+DeviceKernel k_skinny_f16[2][3] = {{{"gemm", "skinny_linear_f16_m1"},
+                                    {"gemm", "skinny_linear_f16_m2"},
+                                    {"gemm", "skinny_linear_f16_m4"}},
+                                   {{"gemm", "skinny_linear_f16_w16_m1"},
+                                    {"gemm", "skinny_linear_f16_w16_m2"},
+                                    {"gemm", "skinny_linear_f16_w16_m4"}}};
 FloatKernels k_attention("attention", "attention");
 FloatKernels k_paged_attention("attention", "paged_attention");
 FloatKernels k_kv_append("attention", "kv_append");
@@ -91,12 +101,25 @@ DeviceKernel k_conv_small9("conv", "conv2d_small_f32_p9");
 DeviceKernel k_conv_small27("conv", "conv2d_small_f32_p27");
 DeviceKernel k_mfma_conv64("mfma_gemm", "mfma_conv2d_f32_t64");
 DeviceKernel k_mfma_conv128("mfma_gemm", "mfma_conv2d_f32_t128");
-DeviceKernel k_mfma_bf16_64("mfma_gemm", "mfma_linear_bf16_t64");
-DeviceKernel k_mfma_bf16_128("mfma_gemm", "mfma_linear_bf16_t128");
+// [tile form: TileForm16]
+DeviceKernel k_mfma_bf16[4] = {{"mfma_gemm", "mfma_linear_bf16_t64"},
+                               {"mfma_gemm", "mfma_linear_bf16_t64_g2"},
+                               {"mfma_gemm", "mfma_linear_bf16_t64_stream"},
+                               {"mfma_gemm", "mfma_linear_bf16_t128"}};
+DeviceKernel k_mfma_f16[4] = {{"mfma_gemm", "mfma_linear_f16_t64"},
+                              {"mfma_gemm", "mfma_linear_f16_t64_g2"},
+                              {"mfma_gemm", "mfma_linear_f16_t64_stream"},
+                              {"mfma_gemm", "mfma_linear_f16_t128"}};
+DeviceKernel k_mfma_linres[4] = {{"mfma_gemm", "mfma_linear_residual_bf16_t64"},
+                                 {"mfma_gemm", "mfma_linear_residual_bf16_t64_g2"},
+                                 {"mfma_gemm", "mfma_linear_residual_bf16_t64_stream"},
+                                 {"mfma_gemm", "mfma_linear_residual_bf16_t128"}};
 DeviceKernel k_mfma_bf16_splitk("mfma_gemm", "mfma_linear_bf16_splitk_t64");
+DeviceKernel k_mfma_bf16_rows("mfma_gemm", "mfma_linear_bf16_splitk_rows_t64");
 DeviceKernel k_splitk_reduce_bf16("mfma_gemm", "splitk_reduce_bf16");
-DeviceKernel k_mfma_bf16_stream("mfma_gemm", "mfma_linear_bf16_stream_t64");
-DeviceKernel k_mfma_linres_stream("mfma_gemm", "mfma_linear_residual_bf16_stream_t64");
+DeviceKernel k_mfma_f16_splitk("mfma_gemm", "mfma_linear_f16_splitk_t64");
+DeviceKernel k_mfma_f16_rows("mfma_gemm", "mfma_linear_f16_splitk_rows_t64");
+DeviceKernel k_splitk_reduce_f16("mfma_gemm", "splitk_reduce_f16");
 DeviceKernel k_mfma_splitk("mfma_gemm", "mfma_linear_f32_splitk_t64");
 DeviceKernel k_splitk_reduce("mfma_gemm", "splitk_reduce_f32");
 DeviceKernel k_mfma_conv_splitk("mfma_gemm", "mfma_conv2d_f32_splitk_t64");
@@ -188,32 +211,115 @@ int64_t bf16Splits(int64_t m, int64_t n, int64_t k) {
 // m = 32 on the wide ones, never at m <= 8)
 bool tiledDecodeLinear(int64_t m, int64_t n) { return m > 32 || (m > 8 && n >= 8192); }
 
-// The tiled bf16 GEMM over decode-sized m, K split when the workspace allows it: out =
-// bf16(x w^T + bias) or, with a residual, bf16(residual + bf16(x w^T + bias)).
-int tiledBf16(const void* x, const void* w, const void* bias,
-              const void* residual, void* out, int64_t m, int64_t n, int64_t k, void* workspace,
-              size_t workspace_bytes, void* stream) {
-  int64_t splits = bf16Splits(m, n, k);
-  const size_t part = static_cast<size_t>(m * n) * sizeof(float);
-  while (splits > 1 && (workspace == nullptr || workspace_bytes < part * splits)) splits /= 2;
-  const Dim3 grid{static_cast<unsigned>((n + 63) / 64), static_cast<unsigned>((m + 63) / 64)};
-  if (splits == 1) {
-    if (residual != nullptr)
-      return launch(k_mfma_linres_stream, grid, {256}, 0, stream, x, w, bias, residual, out, m,
-                    n, k);
-    return launch(k_mfma_bf16_stream, grid, {256}, 0, stream, x, w, bias, out, m, n, k, 0);
-  }
-  const int64_t per = ((k + splits - 1) / splits + 127) / 128 * 128;  // whole 128-wide slices
-  const int64_t parts = (k + per - 1) / per;
-  if (int rc = launch(k_mfma_bf16_splitk, {grid.x, grid.y, static_cast<unsigned>(parts)}, {256},
-                      0, stream, x, w, static_cast<float*>(workspace), m, n, k, per))
-    return rc;
-  return launch(k_splitk_reduce_bf16, {strideBlocks(m * n)}, {256}, 0, stream,
-                static_cast<const float*>(workspace), bias, residual, out, m, n,
-                static_cast<int>(parts));
+// Which kernels a 16-bit linear of m rows runs on: the skinny kernels (K over the 4 or the 16 waves
+// of a workgroup, no second launch) or the tiled GEMM.
+enum class Linear16 { kSkinny4, kSkinny16, kTiled };
+
+// Skinny needs m <= 64 and K % 64 == 0. Its waves load x themselves, 16 rows a fragment, which
+// costs more with every row and column of x; 16 waves of 16 weight rows up to one workgroup per CU
+// (n <= 4096), else 4 waves of 32 rows. Measured in us (4 waves / 16 waves / tiled with its parts),
+// n x k at m rows: 896 x 896 m = 1 4.3 / 3.3 / 8.6, m = 64 10.3 / 7.1 / 8.2; 896 x 4864 m = 8
+// 13 / 8.3 / 8.7, m = 16 15.2 / 10.7 / 8.9; 4096 x 1024 m = 64 11.4 / 8.7 / 9.8; 3584 x 3584 m = 17
+// 13.9 / 10.0 / 10.9, m = 32 16.5 / 12.6 / 11.4; 4864 x 896 m = 32 6.8 / 8.3 / 9.5, m = 50 10.0 /
+// 12.1 / 9.9; 18944 x 3584 m = 9 29 / 31 / 33, m = 17 42 / 43 / 33.
+Linear16 linear16Route(int64_t m, int64_t n, int64_t k) {
+  if (m > 64 || k % 64 != 0) return Linear16::kTiled;
+  const bool w16 = n <= 4096;
+  if (m > 8 && m * k > (w16 ? 65536 : 32768)) return Linear16::kTiled;
+  return w16 ? Linear16::kSkinny16 : Linear16::kSkinny4;
 }
 
-// The split GEMM of tiledBf16 alone: fp32 parts [parts, m, n] of x w^T in the workspace (K in
+// Output tiles of the 16-bit GEMM: 128 x 128 from about 168 of them (at 896 columns, 2048 rows /
+// 112 tiles ran faster in 64 x 64 tiles, 4096 rows / 224 tiles in 128 x 128 tiles); else 64 x 64,
+// with two K groups per workgroup where the tiles leave CUs with one workgroup (in us, one group /
+// two: 77 x 896 x 896 6.6 / 6.2, 1000 x 896 x 4864 19.9 / 18.7, 300 x 4864 x 896 (380 tiles) 9.2 /
+// 9.4). One row tile over more column tiles than CUs streams its weights past the caches: a large
+// weight that stays out of the memory-side cache leaves it to the rest of the layer (34 tokens
+// through a layer of hidden 3584, ffn 18944: 205 us, 212 with cached loads).
+TileForm16 tileForm16(int64_t m, int64_t n) {
+  const bool few = ((m + 63) / 64) * ((n + 63) / 64) <= 256;
+  if (m <= 64) return few ? TileForm16::k64Two : TileForm16::k64Stream;
+  if (((m + 127) / 128) * ((n + 127) / 128) >= 168) return TileForm16::k128;
+  return few ? TileForm16::k64Two : TileForm16::k64;
+}
+
+// Grid and threads of a tile form; false when the rows do not fit the grid.
+bool tileLaunch16(TileForm16 form, int64_t m, int64_t n, Dim3* grid, Dim3* block) {
+  const int64_t tile = form == TileForm16::k128 ? 128 : 64;
+  const int64_t gx = (n + tile - 1) / tile, gy = (m + tile - 1) / tile;
+  if (gy > kMaxGridY || gx > (int64_t{1} << 31)) return false;
+  *grid = Dim3{static_cast<unsigned>(gx), static_cast<unsigned>(gy)};
+  *block = Dim3{form == TileForm16::k64Two ? 512u : 256u};
+  return true;
+}
+
+// K parts of a 16-bit linear on the tiled GEMM: parts of `per` columns (whole slices).
+struct Parts16 {
+  int64_t parts, per;
+};
+Parts16 parts16(int64_t m, int64_t k, int64_t splits) {
+  const int64_t slice = m <= 64 ? 128 : 64;
+  const int64_t per = ((k + splits - 1) / splits + slice - 1) / slice * slice;
+  return Parts16{(k + per - 1) / per, per};
+}
+int64_t splits16(int64_t m, int64_t n, int64_t k) {
+  if (m <= 64) {
+    // two parts are not worth the second launch against two K groups in one workgroup
+    // (64 x 4864 x 896: 9.6 us in two parts, 6.3 unsplit)
+    const int64_t splits = bf16Splits(m, n, k);
+    return splits <= 2 ? 1 : splits;
+  }
+  // A workgroup walks its K one slice per LDS round trip: few tiles over a long K are split until
+  // about 224 workgroups walk at most 6 parts of at least 768 columns. Measured in us unsplit /
+  // split: 77 x 896 x 4864 16.0 / 9.4 (6 parts), 200 rows 16.6 / 12.3, 300 rows 17.6 / 13.7 (3
+  // parts); from 600 rows, and at K = 1024, the parts' fp32 traffic costs more than it gives
+  // (600 x 896 x 4864 18.6 / 21.6).
+  const int64_t tiles = ((m + 63) / 64) * ((n + 63) / 64);
+  if (tiles > 96) return 1;
+  int64_t splits = 224 / tiles;
+  if (splits > k / 768) splits = k / 768;
+  return splits < 1 ? 1 : (splits > 6 ? 6 : splits);
+}
+
+size_t tiled16Workspace(int64_t m, int64_t n, int64_t k) {
+  const int64_t parts = parts16(m, k, splits16(m, n, k)).parts;
+  return parts > 1 ? static_cast<size_t>(parts * m * n) * sizeof(float) : 0;
+}
+
+// out = T(x w^T + bias) (or fp32), optional ReLU, or with a residual (bf16) bf16(residual +
+// bf16(x w^T + bias)), for bf16 and f16 operands with K % 8 == 0 and 16-byte aligned x and w on the
+// tiled MFMA GEMM; K is split as far as the workspace holds the parts.
+int tiled16(int dtype, const void* x, const void* w, const void* bias, const void* residual,
+            void* out, int64_t m, int64_t n, int64_t k, int out_f32, int relu, void* workspace,
+            size_t workspace_bytes, void* stream) {
+  const bool h = dtype == DLI_F16;
+  Parts16 p = parts16(m, k, splits16(m, n, k));
+  while (p.parts > 1 && (workspace == nullptr ||
+                         workspace_bytes < static_cast<size_t>(p.parts * m * n) * sizeof(float)))
+    p = parts16(m, k, p.parts / 2);
+  if (p.parts == 1) {
+    const TileForm16 form = tileForm16(m, n);
+    Dim3 grid, block;
+    if (!tileLaunch16(form, m, n, &grid, &block)) return badArg("linear", "m too large");
+    const int f = static_cast<int>(form);
+    if (residual != nullptr)
+      return launch(k_mfma_linres[f], grid, block, 0, stream, x, w, bias, residual, out, m, n, k);
+    return launch((h ? k_mfma_f16 : k_mfma_bf16)[f], grid, block, 0, stream, x, w, bias, out, m, n,
+                  k, out_f32, relu);
+  }
+  DeviceKernel& kern = m <= 64 ? (h ? k_mfma_f16_splitk : k_mfma_bf16_splitk)
+                               : (h ? k_mfma_f16_rows : k_mfma_bf16_rows);
+  if (int rc = launch(kern,
+                      {static_cast<unsigned>((n + 63) / 64), static_cast<unsigned>((m + 63) / 64),
+                       static_cast<unsigned>(p.parts)},
+                      {256}, 0, stream, x, w, static_cast<float*>(workspace), m, n, k, p.per))
+    return rc;
+  return launch(h ? k_splitk_reduce_f16 : k_splitk_reduce_bf16, {strideBlocks((m * n + 3) / 4)},
+                {256}, 0, stream, static_cast<const float*>(workspace), bias, residual, out, m, n,
+                static_cast<int>(p.parts), out_f32, relu);
+}
+
+// The split GEMM alone: fp32 parts [parts, m, n] of x w^T in the workspace (K in
 // whole 128-wide slices over at most bf16Splits(m, n, k) parts, as many as the workspace holds,
 // at least one), for a caller's own reduce. *parts_out = the number of parts written.
 int tiledBf16Parts(const void* x, const void* w, int64_t m, int64_t n, int64_t k,
@@ -470,10 +576,9 @@ int dli_hip_linear(int dtype, int out_dtype, const void* x, const void* w, const
 
 size_t dli_hip_linear_workspace(int dtype, int64_t m, int64_t n, int64_t k) {
   if (m <= 0 || n <= 0 || k <= 0) return 0;
-  if (dtype == DLI_BF16) {  // decode-sized m on the tiled GEMM: K split over fp32 parts
-    if (m > 64 || !tiledDecodeLinear(m, n) || k % 8 != 0) return 0;  // (fp32-out calls ignore it)
-    const int64_t splits = bf16Splits(m, n, k);
-    return splits > 1 ? static_cast<size_t>(splits * m * n) * sizeof(float) : 0;
+  if (dtype == DLI_BF16 || dtype == DLI_F16) {  // the tiled GEMM's K parts
+    if (k % 8 != 0 || linear16Route(m, n, k) != Linear16::kTiled) return 0;
+    return tiled16Workspace(m, n, k);
   }
   if (dtype != DLI_F32) return 0;
   const int64_t splits = linearSplits(m, n, k);
@@ -514,26 +619,21 @@ int dli_hip_linear_act(int dtype, int out_dtype, const void* x, const void* w, c
                   out, m, n, k, relu);
   }
   int rc;
-  if (dtype == DLI_BF16 && m <= 64 && tiledDecodeLinear(m, n) && k % 8 == 0 && aligned16(x) &&
-      aligned16(w) && !relu) {
-    if (out_f32)  // fp32 logits: one pass, no split (the split reduce writes bf16)
-      return launch(k_mfma_bf16_stream,
-                    {static_cast<unsigned>((n + 63) / 64), static_cast<unsigned>((m + 63) / 64)},
-                    {256}, 0, stream, x, w, bias, out, m, n, k, out_f32);
-    return tiledBf16(x, w, bias, nullptr, out, m, n, k, workspace, workspace_bytes,
-                     stream);
-  } else if (dtype == DLI_BF16 && m <= 64 && k % 64 == 0 && aligned16(x) && aligned16(w)) {
-    // bf16 weight streaming for decode-sized m: MFMA skinny kernel.
-    DeviceKernel* sk = m <= 16 ? &k_skinny1 : (m <= 32 ? &k_skinny2 : &k_skinny4);
-    rc = launch(*sk, {blocksFor(n, 32)}, {256}, 0, stream, x, w, bias, out, m, n, k, out_f32);
-  } else if (dtype == DLI_BF16 && k % 8 == 0 && aligned16(x) && aligned16(w) &&
-             (m + 63) / 64 <= kMaxGridY) {
-    // the bf16 GEMM's own tile rule (its 128 x 128 tiles pay off from about 168 of them)
-    const bool b128 = ((m + 127) / 128) * ((n + 127) / 128) >= 168;
-    const int64_t bt = b128 ? 128 : 64;
-    return launch(b128 ? k_mfma_bf16_128 : k_mfma_bf16_64,
-                  {static_cast<unsigned>((n + bt - 1) / bt), static_cast<unsigned>((m + bt - 1) / bt)},
-                  {256}, 0, stream, x, w, bias, out, m, n, k, out_f32, relu);
+  const bool h16 = dtype == DLI_BF16 || dtype == DLI_F16;
+  const bool wide = h16 && k > 0 && k % 8 == 0 && aligned16(x) && aligned16(w);
+  const Linear16 route = wide ? linear16Route(m, n, k) : Linear16::kTiled;
+  // without the workspace for its K parts, the tiled GEMM of few rows is slower than the skinny
+  // kernels up to 32 rows
+  const bool no_parts = m <= 32 && k % 64 == 0 &&
+                        workspace_bytes < dli_hip_linear_workspace(dtype, m, n, k);
+  if (wide && (route != Linear16::kTiled || no_parts)) {
+    const int w16 = route == Linear16::kSkinny16 ? 1 : 0;
+    auto& kernels = (dtype == DLI_F16 ? k_skinny_f16 : k_skinny_bf16)[w16];
+    rc = launch(kernels[m <= 16 ? 0 : (m <= 32 ? 1 : 2)], {blocksFor(n, w16 ? 16 : 32)},
+                {w16 ? 1024u : 256u}, 0, stream, x, w, bias, out, m, n, k, out_f32);
+  } else if (wide && (m + 63) / 64 <= kMaxGridY) {
+    return tiled16(dtype, x, w, bias, nullptr, out, m, n, k, out_f32, relu, workspace,
+                   workspace_bytes, stream);
   } else {
     DeviceKernel* kt = k_gemm.pick(dtype);
     if (kt == nullptr) return badDtype("linear", dtype);

@@ -30,6 +30,17 @@ int computeUnits(int* count);
 // groups of wph cache blocks (wph: waves per kv head); `requested` > 0 (the caller's count)
 // replaces the per-CU choice. Never fewer splits than the per-lane block ids of a wave allow.
 int decodeAttentionSplits(int64_t units, int64_t max_blocks, int cus, int wph, int requested);
+// Tile forms of the 16-bit tiled GEMM (mfma_gemm.hip): 64 x 64, the same with two K groups per
+// workgroup, 64 x 64 with 128-wide slices and nontemporal weight loads (one row tile), 128 x 128 (the
+// index of the kernel tables).
+enum class TileForm16 { k64 = 0, k64Two = 1, k64Stream = 2, k128 = 3 };
+TileForm16 tileForm16(int64_t m, int64_t n);
+bool tileLaunch16(TileForm16 form, int64_t m, int64_t n, Dim3* grid, Dim3* block);
+// A 16-bit linear on the tiled GEMM and its workspace for K parts (of any content).
+size_t tiled16Workspace(int64_t m, int64_t n, int64_t k);
+int tiled16(int dtype, const void* x, const void* w, const void* bias, const void* residual,
+            void* out, int64_t m, int64_t n, int64_t k, int out_f32, int relu, void* workspace,
+            size_t workspace_bytes, void* stream);
 constexpr int kMaxDecodeSplits = 32;  // key-range splits a decode-attention call may use
 
 // A kernel by name inside one embedded code object; resolved once per device.

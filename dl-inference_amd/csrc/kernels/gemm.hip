@@ -88,25 +88,25 @@ __device__ void gemm_tiled_impl(const void* a_, const void* b_, const void* bias
   }
 }
 
-// Skinny linear: grid (ceil(N / 32), 1), 256 threads. Requires K % 64 == 0 and 16-byte aligned
-// rows (checked on the host).
-template <int MB>
-__device__ void skinny_linear_impl(const uint16_t* x, const uint16_t* w, const uint16_t* bias,
-                                   void* out, int64_t M, int64_t N, int64_t K, int out_f32) {
-  using Core = SkinnyCore<2, MB, 4>;
+// Skinny linear: grid (ceil(N / (16 NF)), 1), 64 kWaves threads. Requires K % 64 == 0 and 16-byte
+// aligned rows (checked on the host).
+template <class Core, typename T>
+__device__ __forceinline__ void skinny_linear_impl(const uint16_t* x, const uint16_t* w,
+                                                   const T* bias, void* out, int64_t M, int64_t N,
+                                                   int64_t K, int out_f32) {
   __shared__ float lds[Core::kLdsFloats];
   const int64_t n0 = static_cast<int64_t>(blockIdx.x) * Core::kTileN;
   Core::run(w, XGlobal{x, K}, N, K, static_cast<int>(M), n0, 0, static_cast<int>(K / 64), lds);
-  for (int idx = threadIdx.x; idx < Core::kTileN * Core::kTileM; idx += 4 * kWave) {
+  for (int idx = threadIdx.x; idx < Core::kTileN * Core::kTileM; idx += blockDim.x) {
     const int nl = idx / Core::kTileM, m = idx % Core::kTileM;
     const int64_t n = n0 + nl;
     if (m >= M || n >= N) continue;
     float v = lds[idx];
-    if (bias != nullptr) v += bf16ToFloat(bias[n]);
+    if (bias != nullptr) v += ld(bias + n);
     if (out_f32)
       static_cast<float*>(out)[m * N + n] = v;
     else
-      static_cast<uint16_t*>(out)[m * N + n] = floatToBf16(v);
+      st(static_cast<T*>(out) + m * N + n, v);
   }
 }
 
@@ -117,12 +117,24 @@ DK_FLOAT_KERNELS(gemm_tiled, 256,
                   int64_t K, int b_is_nk, int out_f32),
                  (a, b, bias, out, M, N, K, b_is_nk, out_f32))
 
-#define DK_SKINNY_LINEAR(MB)                                                                \
-  extern "C" __global__ void __launch_bounds__(256)                                         \
-      skinny_linear_m##MB(const uint16_t* x, const uint16_t* w, const uint16_t* bias,       \
-                          void* out, int64_t M, int64_t N, int64_t K, int out_f32) {        \
-    skinny_linear_impl<MB>(x, w, bias, out, M, N, K, out_f32);                              \
+// _m<MB>: 32 weight rows per workgroup, K over 4 waves. _w16_m<MB>: 16 weight rows, K over 16
+// waves, for long K (a wave of the 4 walks K / 256 steps, one load round trip per batch).
+#define DK_SKINNY_LINEAR(name, NF, MB, WAVES, UNROLL, E, T)                                     \
+  extern "C" __global__ void __launch_bounds__(64 * WAVES)                                      \
+      name##_m##MB(const uint16_t* x, const uint16_t* w, const T* bias, void* out, int64_t M,   \
+                   int64_t N, int64_t K, int out_f32) {                                         \
+    skinny_linear_impl<SkinnyCore<NF, MB, WAVES, UNROLL, 0, E>, T>(x, w, bias, out, M, N, K,    \
+                                                                   out_f32);                    \
   }
-DK_SKINNY_LINEAR(1)
-DK_SKINNY_LINEAR(2)
-DK_SKINNY_LINEAR(4)
+DK_SKINNY_LINEAR(skinny_linear_bf16, 2, 1, 4, 4, Bf16, bf16)
+DK_SKINNY_LINEAR(skinny_linear_bf16, 2, 2, 4, 4, Bf16, bf16)
+DK_SKINNY_LINEAR(skinny_linear_bf16, 2, 4, 4, 4, Bf16, bf16)
+DK_SKINNY_LINEAR(skinny_linear_f16, 2, 1, 4, 4, F16, f16)
+DK_SKINNY_LINEAR(skinny_linear_f16, 2, 2, 4, 4, F16, f16)
+DK_SKINNY_LINEAR(skinny_linear_f16, 2, 4, 4, 4, F16, f16)
+DK_SKINNY_LINEAR(skinny_linear_bf16_w16, 1, 1, 16, 2, Bf16, bf16)
+DK_SKINNY_LINEAR(skinny_linear_bf16_w16, 1, 2, 16, 1, Bf16, bf16)
+DK_SKINNY_LINEAR(skinny_linear_bf16_w16, 1, 4, 16, 1, Bf16, bf16)
+DK_SKINNY_LINEAR(skinny_linear_f16_w16, 1, 1, 16, 2, F16, f16)
+DK_SKINNY_LINEAR(skinny_linear_f16_w16, 1, 2, 16, 1, F16, f16)
+DK_SKINNY_LINEAR(skinny_linear_f16_w16, 1, 4, 16, 1, F16, f16)

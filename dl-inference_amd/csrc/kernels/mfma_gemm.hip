@@ -8,8 +8,9 @@
 //  mfma_conv2d_f32          im2col-free conv2d (conv2d/kernel.py:6-49): A = weight [OC, C*KH*KW]
 //                           rows, B = the input patch of each output pixel, gathered from NCHW
 //                           x while staging (never materialised); out NCHW, optional fused ReLU
-//  mfma_linear_bf16_<t>     bf16 x, w (K % 8 == 0), bf16 MFMA 16x16x32, fp32 accumulation,
-//                           bf16 or fp32 out, optional ReLU
+//  mfma_linear_bf16_<t>, mfma_linear_f16_<t>  16-bit x, w (K % 8 == 0), MFMA 16x16x32, fp32
+//                           accumulation, 16-bit or fp32 out, optional ReLU. (f16, 1000 x 4864 x
+//                           896: 252 us on the general kernel of gemm.hip, 19 us here)
 //  mfma_linear_residual_bf16_<t>  the same plus a residual add (bf16 out)
 //  mfma_gate_up_silu_bf16_<t>     the same over an interleaved gate/up weight, SwiGLU epilogue
 //  mfma_linear_f32_splitk   fp32 linear / conv2d with K split over grid.z into a workspace,
@@ -296,8 +297,8 @@ __device__ __forceinline__ void gemmF32(ASrc A, BSrc B, int64_t R, int64_t Cn, i
   }
 }
 
-// ---- bf16 core ---------------------------------------------------------------------------------
-// v_mfma_f32_16x16x32_bf16: lane l supplies A[l % 16][(l / 16) * 8 + j] and
+// ---- 16-bit core ---------------------------------------------------------------------------------
+// v_mfma_f32_16x16x32_bf16 / _f16 (E = Bf16 / F16): lane l supplies A[l % 16][(l / 16) * 8 + j] and
 // B[(l / 16) * 8 + j][l % 16], j < 8. Operands are [rows, K] row-major with K % 8 == 0 and
 // 16-byte aligned rows, loaded 8 elements at a time.
 //
@@ -322,9 +323,13 @@ __device__ __forceinline__ void gemmF32(ASrc A, BSrc B, int64_t R, int64_t Cn, i
 // Each load instruction covers whole 128-byte lines (16 lanes per 256-byte row slice of a
 // 128-wide slice); a streaming probe over 1 GiB read 6.5-6.9 TB/s that way against 5.8-6.0 with
 // cached loads.
-template <int BM, int BN, int BK = 64, bool kStreamB = false, class Epi>
-__device__ __forceinline__ void gemmBf16(const uint16_t* a, const uint16_t* b, int64_t R,
-                                         int64_t Cn, int64_t K, int64_t ld, const Epi& epi) {
+// G: groups of 256 threads that take equal runs of K slices of the same tile, each with operand
+// buffers of its own; the epilogue adds the groups' sums in group order. One group walks K one slice
+// per load and LDS round trip (about 550 cycles for 64 x 64, of which 256 are the slice's 16 KB at
+// 64 bytes a cycle), so a grid that leaves CUs with one workgroup gains from a second group.
+template <int BM, int BN, int BK = 64, bool kStreamB = false, class E = Bf16, int G = 1, class Epi>
+__device__ __forceinline__ void gemm16(const uint16_t* a, const uint16_t* b, int64_t R,
+                                       int64_t Cn, int64_t K, int64_t ld, const Epi& epi) {
   static_assert(BK == 64 || BK == 128, "slice width");
   constexpr int TM = BM / 32, TN = BN / 32;
   constexpr int VPR = BK / 8;  // 16-byte chunks per tile row
@@ -333,16 +338,32 @@ __device__ __forceinline__ void gemmBf16(const uint16_t* a, const uint16_t* b, i
   // epilogue, row pitch BN + 4 floats (the 4 row groups of an MFMA tile store land 16 banks apart)
   constexpr int CP = BN + 4;
   constexpr int kOperandBytes = 2 * (BM + BN) * BK * 2, kTileBytes = BM * CP * 4;
-  __shared__ __attribute__((aligned(16)))
-  uint8_t smem[kOperandBytes > kTileBytes ? kOperandBytes : kTileBytes];
-  uint16_t* const As0 = reinterpret_cast<uint16_t*>(smem);
+  constexpr int kGroupBytes = kOperandBytes > kTileBytes ? kOperandBytes : kTileBytes;
+  constexpr int kThreads = G * kGemmThreads;
+  __shared__ __attribute__((aligned(16))) uint8_t smem[G * kGroupBytes];
+  const int t = threadIdx.x % kGemmThreads, lane = t % kWave;
+  // uniform over the wave
+  const int wave = __builtin_amdgcn_readfirstlane(t / kWave);
+  const int grp = G == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / kGemmThreads);
+  uint16_t* const As0 = reinterpret_cast<uint16_t*>(smem + grp * kGroupBytes);
   uint16_t* const Bs0 = As0 + BM * BK;
   uint16_t* const As1 = Bs0 + BN * BK;
   uint16_t* const Bs1 = As1 + BM * BK;
-  const int t = threadIdx.x, lane = t % kWave, wave = t / kWave;
   const int wr = wave / 2, wc = wave % 2;
   int64_t r0, c0;
   groupedTile(BM, BN, r0, c0);
+  // the group's slices; every group makes the same number of steps (and barriers), the last one's
+  // steps past K multiply zeros
+  const int64_t slices = (K + BK - 1) / BK, nk = (slices + G - 1) / G;
+  int64_t whole = K;  // columns that every group has
+  if constexpr (G > 1) {
+    const int64_t per = nk * BK;
+    whole = K - (G - 1) * per;
+    a += grp * per;
+    b += grp * per;
+    K -= grp * per;
+    K = K < per ? K : per;
+  }
   // 64-wide slices: rows of 128 bytes, two rows fill the 64 banks, chunk c at c ^ ((r >> 1) & 7);
   // 128-wide: rows of 256 bytes, chunk c of 16 at c ^ (r & 15)
   auto at = [](int row, int c) {
@@ -421,8 +442,7 @@ __device__ __forceinline__ void gemmBf16(const uint16_t* a, const uint16_t* b, i
     for (int i = 0; i < TM; ++i)
 #pragma unroll
       for (int j = 0; j < TN; ++j)
-        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(asBf16x8(fa[i]), asBf16x8(fb[j]),
-                                                            acc[i][j], 0, 0, 0);
+        acc[i][j] = E::mma(fa[i], fb[j], acc[i][j]);
   };
   constexpr int kMm = TM * TN, kRd = TM + TN, kWr = AV + BV;
   static_assert(kMm >= kRd && (BK == 128 ? 2 * kMm >= kWr : kMm >= kWr),
@@ -502,14 +522,13 @@ __device__ __forceinline__ void gemmBf16(const uint16_t* a, const uint16_t* b, i
   };
   // slice j lives in registers j % 2 and LDS buffer j % 2
   U128 ra0[AV], rb0[BV], ra1[AV], rb1[BV];
-  const int64_t nk = (K + BK - 1) / BK;
   fetch(ra0, rb0, 0);
   if (nk > 1) fetch(ra1, rb1, BK);
   stash(ra0, rb0, As0, Bs0);
   __syncthreads();
   if (nk > 2) fetch(ra0, rb0, 2 * BK);
   int64_t s = 0;
-  for (; (s + 5) * BK <= K; s += 2) {  // steps s, s + 1 fetch slices s + 3, s + 4: all whole
+  for (; (s + 5) * BK <= whole; s += 2) {  // steps s, s + 1 fetch slices s + 3, s + 4: all whole
     wholeStep(As0, Bs0, ra1, rb1, As1, Bs1, (s + 3) * BK);
     wholeStep(As1, Bs1, ra0, rb0, As0, Bs0, (s + 4) * BK);
   }
@@ -523,24 +542,33 @@ __device__ __forceinline__ void gemmBf16(const uint16_t* a, const uint16_t* b, i
   // right edge, and outputs the vector forms cannot address, go element by element through the
   // same arithmetic.
   float* const ct = reinterpret_cast<float*>(smem);
+  constexpr int kNextGroup = kGroupBytes / 4;
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
     for (int j = 0; j < TN; ++j)
 #pragma unroll
       for (int v = 0; v < 4; ++v)
-        ct[(wr * (BM / 2) + i * 16 + fk * 4 + v) * CP + wc * (BN / 2) + j * 16 + fr] =
-            acc[i][j][v];
+        ct[grp * kNextGroup + (wr * (BM / 2) + i * 16 + fk * 4 + v) * CP + wc * (BN / 2) + j * 16 +
+           fr] = acc[i][j][v];
   __syncthreads();
+  auto sum = [&](int at) {
+    float v = ct[at];
+#pragma unroll
+    for (int q = 1; q < G; ++q) v += ct[q * kNextGroup + at];
+    return v;
+  };
+  const int te = threadIdx.x;
   const bool vec = epi.vectorOk();
   if constexpr (Epi::kPairs) {
     // [gate 16 | up 16] column groups: run h (0, 1) of group b pairs gate columns 32 b + 8 h ..
     // with up columns 32 b + 16 + 8 h ..
     constexpr int kRuns = BM * BN / 16;
-    static_assert(BN % 32 == 0 && kRuns % kGemmThreads == 0, "pair runs");
+    static_assert(BN % 32 == 0, "pair runs");
 #pragma unroll
-    for (int q = 0; q < kRuns / kGemmThreads; ++q) {
-      const int e = t + q * kGemmThreads;
+    for (int q = 0; q < (kRuns + kThreads - 1) / kThreads; ++q) {
+      const int e = te + q * kThreads;
+      if (kRuns % kThreads != 0 && e >= kRuns) break;
       const int row = e / (BN / 16), p = e % (BN / 16);
       const int cg = (p / 2) * 32 + (p % 2) * 8;
       const int64_t grow = r0 + row, gcol = c0 + cg;
@@ -548,8 +576,8 @@ __device__ __forceinline__ void gemmBf16(const uint16_t* a, const uint16_t* b, i
       float g[8], u[8];
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
-        g[k] = ct[row * CP + cg + k];
-        u[k] = ct[row * CP + cg + 16 + k];
+        g[k] = sum(row * CP + cg + k);
+        u[k] = sum(row * CP + cg + 16 + k);
       }
       if (vec && gcol + 24 <= Cn) {
         epi.pair8(grow, gcol, g, u);
@@ -560,13 +588,14 @@ __device__ __forceinline__ void gemmBf16(const uint16_t* a, const uint16_t* b, i
       }
     }
   } else {
-    // thread t's runs: rows t / (BN / 8) + q * (256 / (BN / 8)), all at column run c8. The
+    // a thread's runs: rows row0 + q * kRowStep, all at column run c8. The
     // loads of every run go out before any result is stored: the compiler must assume a store
     // may alias a later run's input, so a load-compute-store loop per run waited for each load.
-    constexpr int kRuns = BM * BN / 8, kPer = kRuns / kGemmThreads;
-    static_assert(kRuns % kGemmThreads == 0 && kGemmThreads % (BN / 8) == 0, "runs");
-    const int c8 = (t % (BN / 8)) * 8, row0 = t / (BN / 8);
-    constexpr int kRowStep = kGemmThreads / (BN / 8);
+    constexpr int kRuns = BM * BN / 8, kPer = (kRuns + kThreads - 1) / kThreads;
+    static_assert(kThreads % (BN / 8) == 0, "runs");
+    const int c8 = (te % (BN / 8)) * 8, row0 = te / (BN / 8);
+    constexpr int kRowStep = kThreads / (BN / 8);
+    if (kRuns < kThreads && row0 >= BM) return;  // more threads than runs
     const int64_t gcol = c0 + c8;
     if (Epi::kVectorOnly || (vec && gcol + 8 <= Cn)) {
       const auto cd = epi.column(gcol);
@@ -583,7 +612,7 @@ __device__ __forceinline__ void gemmBf16(const uint16_t* a, const uint16_t* b, i
         if (grow >= R) continue;
         float v[8];
 #pragma unroll
-        for (int k = 0; k < 8; ++k) v[k] = ct[row * CP + c8 + k];
+        for (int k = 0; k < 8; ++k) v[k] = sum(row * CP + c8 + k);
         epi.vec8(grow, gcol, v, cd, rd[q]);
       }
     } else if constexpr (!Epi::kVectorOnly) {
@@ -594,7 +623,7 @@ __device__ __forceinline__ void gemmBf16(const uint16_t* a, const uint16_t* b, i
         if (grow >= R) continue;
 #pragma unroll
         for (int k = 0; k < 8; ++k)
-          if (gcol + k < Cn) epi(grow, gcol + k, ct[row * CP + c8 + k]);
+          if (gcol + k < Cn) epi(grow, gcol + k, sum(row * CP + c8 + k));
       }
     }
   }
@@ -636,13 +665,40 @@ struct RowMajorOut {
   }
 };
 
-// RowMajorOut with the output type chosen at run time (one copy of the GEMM per kernel: two
-// inlined copies, one per output type, took the kernel past 256 registers)
-struct RowMajorOutBf16OrF32 {
+__device__ __forceinline__ void unpack16x8(const U128& w, float (&f)[8], bf16) {
+  unpackBf16x8(w, f);
+}
+__device__ __forceinline__ void unpack16x8(const U128& w, float (&f)[8], f16) {
+  const f16x8 h = __builtin_bit_cast(f16x8, w);
+#pragma unroll
+  for (int k = 0; k < 8; ++k) f[k] = static_cast<float>(h[k]);
+}
+__device__ __forceinline__ U128 pack16x8(const float (&f)[8], bf16) { return packBf16x8(f); }
+__device__ __forceinline__ U128 pack16x8(const float (&f)[8], f16) {
+  f16x8 h;
+#pragma unroll
+  for (int k = 0; k < 8; ++k) h[k] = static_cast<f16>(f[k]);
+  return __builtin_bit_cast(U128, h);
+}
+
+__device__ __forceinline__ uint2 pack16x4(const float (&f)[4], bf16) {
+  return uint2{packBf16x2(f[0], f[1]), packBf16x2(f[2], f[3])};
+}
+__device__ __forceinline__ uint2 pack16x4(const float (&f)[4], f16) {
+  typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
+  return __builtin_bit_cast(uint2, f16x4{static_cast<f16>(f[0]), static_cast<f16>(f[1]),
+                                         static_cast<f16>(f[2]), static_cast<f16>(f[3])});
+}
+
+// RowMajorOut of 16-bit operands (T = bf16 or f16) with the output type chosen at run time (one
+// copy of the GEMM per kernel: two inlined copies, one per output type, took the kernel past 256
+// registers)
+template <typename T>
+struct RowMajorOut16OrF32 {
   static constexpr bool kPairs = false;
   static constexpr bool kVectorOnly = false;
   void* out;
-  const bf16* bias;
+  const T* bias;
   int64_t ldo;
   int relu, out_f32;
   __device__ __forceinline__ void operator()(int64_t row, int64_t col, float v) const {
@@ -651,7 +707,7 @@ struct RowMajorOutBf16OrF32 {
     if (out_f32)
       st(static_cast<float*>(out) + row * ldo + col, v);
     else
-      st(static_cast<bf16*>(out) + row * ldo + col, v);
+      st(static_cast<T*>(out) + row * ldo + col, v);
   }
   __device__ __forceinline__ bool vectorOk() const {
     return ldo % 8 == 0 && aligned16(out) && aligned16(bias);
@@ -665,7 +721,7 @@ struct RowMajorOutBf16OrF32 {
                                        const Run&) const {
     if (bias != nullptr) {
       float b[8];
-      unpackBf16x8(bw, b);
+      unpack16x8(bw, b, T{});
 #pragma unroll
       for (int k = 0; k < 8; ++k) v[k] += b[k];
     }
@@ -679,10 +735,12 @@ struct RowMajorOutBf16OrF32 {
       *gp(reinterpret_cast<U128*>(o + 4)) = U128{__float_as_uint(v[4]), __float_as_uint(v[5]),
                                                  __float_as_uint(v[6]), __float_as_uint(v[7])};
     } else {
-      *gp(reinterpret_cast<U128*>(static_cast<bf16*>(out) + row * ldo + col)) = packBf16x8(v);
+      *gp(reinterpret_cast<U128*>(static_cast<T*>(out) + row * ldo + col)) = pack16x8(v, T{});
     }
   }
 };
+
+using RowMajorOutBf16OrF32 = RowMajorOut16OrF32<bf16>;
 
 // out[row, col] = bf16(residual[row, col] + bf16(v + bias[col])): a linear whose output is
 // added to the residual stream, rounded where the unfused graph rounds (linear, then add).
@@ -952,61 +1010,72 @@ extern "C" __global__ void __launch_bounds__(kGemmThreads)
 // fragments room without spilling.
 #define DK_BF16_OCCUPANCY __attribute__((amdgpu_waves_per_eu(2)))
 
-#define DK_MFMA_BF16(BM, BN)                                                                    \
-  extern "C" __global__ void __launch_bounds__(kGemmThreads) DK_BF16_OCCUPANCY                   \
-      mfma_linear_bf16_t##BM(                                                                  \
-      const uint16_t* x, const uint16_t* w, const uint16_t* bias, void* out, int64_t M,        \
-      int64_t N, int64_t K, int out_f32, int relu) {                                           \
-    gemmBf16<BM, BN>(x, w, M, N, K, K,                                                         \
-                     RowMajorOutBf16OrF32{out, reinterpret_cast<const bf16*>(bias), N, relu,   \
-                                          out_f32});                                           \
+// Names: _t64 and _t128 tiles, _t64_g2 with two K groups per workgroup (gemm16's G), _t64_stream
+// with 128-wide slices and nontemporal weight loads (one row tile over a large weight).
+#define DK_MFMA_LINEAR16(name, T, E, TILE, G, S)                                                  \
+  extern "C" __global__ void __launch_bounds__(G* kGemmThreads) DK_BF16_OCCUPANCY               \
+      name(const uint16_t* x, const uint16_t* w, const uint16_t* bias, void* out, int64_t M,    \
+           int64_t N, int64_t K, int out_f32, int relu) {                                       \
+    gemm16<TILE, TILE, S ? 128 : 64, S, E, G>(                                                            \
+        x, w, M, N, K, K,                                                                       \
+        RowMajorOut16OrF32<T>{out, reinterpret_cast<const T*>(bias), N, relu, out_f32});        \
   }
 
-DK_MFMA_BF16(64, 64)
-DK_MFMA_BF16(128, 128)
+DK_MFMA_LINEAR16(mfma_linear_bf16_t64, bf16, Bf16, 64, 1, false)
+DK_MFMA_LINEAR16(mfma_linear_bf16_t64_g2, bf16, Bf16, 64, 2, false)
+DK_MFMA_LINEAR16(mfma_linear_bf16_t64_stream, bf16, Bf16, 64, 1, true)
+DK_MFMA_LINEAR16(mfma_linear_bf16_t128, bf16, Bf16, 128, 1, false)
+DK_MFMA_LINEAR16(mfma_linear_f16_t64, f16, F16, 64, 1, false)
+DK_MFMA_LINEAR16(mfma_linear_f16_t64_g2, f16, F16, 64, 2, false)
+DK_MFMA_LINEAR16(mfma_linear_f16_t64_stream, f16, F16, 64, 1, true)
+DK_MFMA_LINEAR16(mfma_linear_f16_t128, f16, F16, 128, 1, false)
 
 // bf16 linear + residual (bf16 out) and SwiGLU of an interleaved gate/up weight (N = 2 * ffn,
 // ffn % 16 == 0): the ResidualOut and SwiGluOut epilogues above.
-#define DK_MFMA_BF16_FUSED(BM, BN)                                                              \
-  extern "C" __global__ void __launch_bounds__(kGemmThreads) DK_BF16_OCCUPANCY                   \
-      mfma_linear_residual_bf16_t##BM(                                                         \
+#define DK_MFMA_BF16_FUSED(SUFFIX, TILE, G, S)                                                  \
+  extern "C" __global__ void __launch_bounds__(G* kGemmThreads) DK_BF16_OCCUPANCY               \
+      mfma_linear_residual_bf16_##SUFFIX(                                                      \
       const uint16_t* x, const uint16_t* w, const uint16_t* bias, const uint16_t* residual,    \
       uint16_t* out, int64_t M, int64_t N, int64_t K) {                                        \
-    gemmBf16<BM, BN>(x, w, M, N, K, K,                                                         \
-                     ResidualOut{reinterpret_cast<bf16*>(out),                                  \
-                                 reinterpret_cast<const bf16*>(residual),                      \
-                                 reinterpret_cast<const bf16*>(bias), N});                     \
+    gemm16<TILE, TILE, S ? 128 : 64, S, Bf16, G>(x, w, M, N, K, K,                                       \
+                                       ResidualOut{reinterpret_cast<bf16*>(out),               \
+                                                   reinterpret_cast<const bf16*>(residual),    \
+                                                   reinterpret_cast<const bf16*>(bias), N});   \
   }                                                                                            \
-  extern "C" __global__ void __launch_bounds__(kGemmThreads) DK_BF16_OCCUPANCY                   \
-      mfma_gate_up_silu_bf16_t##BM(                                                            \
+  extern "C" __global__ void __launch_bounds__(G* kGemmThreads) DK_BF16_OCCUPANCY               \
+      mfma_gate_up_silu_bf16_##SUFFIX(                                                         \
       const uint16_t* x, const uint16_t* w_gate_up, uint16_t* out, int64_t M, int64_t ffn,      \
       int64_t K) {                                                                             \
-    gemmBf16<BM, BN>(x, w_gate_up, M, 2 * ffn, K, K,                                           \
-                     SwiGluOut{reinterpret_cast<bf16*>(out), ffn});                             \
+    gemm16<TILE, TILE, S ? 128 : 64, S, Bf16, G>(x, w_gate_up, M, 2 * ffn, K, K,                         \
+                                       SwiGluOut{reinterpret_cast<bf16*>(out), ffn});           \
   }
 
-DK_MFMA_BF16_FUSED(64, 64)
-DK_MFMA_BF16_FUSED(128, 128)
+DK_MFMA_BF16_FUSED(t64, 64, 1, false)
+DK_MFMA_BF16_FUSED(t64_g2, 64, 2, false)
+DK_MFMA_BF16_FUSED(t64_stream, 64, 1, true)
+DK_MFMA_BF16_FUSED(t128, 128, 1, false)
 
 // q|k|v projection + RoPE + head layout of a prefill prompt (QkvHeadsOut): x [B * S, K],
 // w_qkv [(Hq + 2 Hkv) D, K], b_qkv [(Hq + 2 Hkv) D].
-#define DK_MFMA_QKV_HEADS(BM, BN)                                                               \
-  extern "C" __global__ void __launch_bounds__(kGemmThreads) DK_BF16_OCCUPANCY                 \
-      mfma_qkv_heads_bf16_t##BM(const uint16_t* x, const uint16_t* w_qkv, const uint16_t* b_qkv, \
+#define DK_MFMA_QKV_HEADS(SUFFIX, TILE, G, S)                                                      \
+  extern "C" __global__ void __launch_bounds__(G* kGemmThreads) DK_BF16_OCCUPANCY              \
+      mfma_qkv_heads_bf16_##SUFFIX(const uint16_t* x, const uint16_t* w_qkv, const uint16_t* b_qkv, \
                                 const float* cos, const float* sin, int64_t max_pos,           \
                                 uint16_t* q, uint16_t* k, uint16_t* v, int64_t M, int64_t K,   \
                                 int64_t seq, int64_t start_pos, int q_heads, int kv_heads,     \
                                 int head_dim) {                                                \
     const int64_t n = static_cast<int64_t>(q_heads + 2 * kv_heads) * head_dim;                 \
-    gemmBf16<BM, BN>(x, w_qkv, M, n, K, K,                                                     \
+    gemm16<TILE, TILE, S ? 128 : 64, S, Bf16, G>(x, w_qkv, M, n, K, K,                                                     \
                      QkvHeadsOut{reinterpret_cast<bf16*>(q), reinterpret_cast<bf16*>(k),       \
                                  reinterpret_cast<bf16*>(v),                                   \
                                  reinterpret_cast<const bf16*>(b_qkv), cos, sin, seq, max_pos, \
                                  start_pos, q_heads, kv_heads, head_dim});                     \
   }
 
-DK_MFMA_QKV_HEADS(64, 64)
-DK_MFMA_QKV_HEADS(128, 128)
+DK_MFMA_QKV_HEADS(t64, 64, 1, false)
+DK_MFMA_QKV_HEADS(t64_g2, 64, 2, false)
+DK_MFMA_QKV_HEADS(t64_stream, 64, 1, true)
+DK_MFMA_QKV_HEADS(t128, 128, 1, false)
 
 // bf16 linear with K split over grid.z (decode-sized m with few output tiles): part z covers
 // columns [z * per, min(K, (z + 1) * per)) (per % 64 == 0) and writes its fp32 sums to
@@ -1017,51 +1086,86 @@ extern "C" __global__ void __launch_bounds__(kGemmThreads) DK_BF16_OCCUPANCY
   const int64_t k0 = static_cast<int64_t>(blockIdx.z) * per;
   const int64_t len = K - k0 < per ? K - k0 : per;
   float* const out = part + static_cast<int64_t>(blockIdx.z) * M * N;
-  gemmBf16<64, 64, 128, true>(x + k0, w + k0, M, N, len, K,
+  gemm16<64, 64, 128, true>(x + k0, w + k0, M, N, len, K,
                               RowMajorOutBf16OrF32{out, nullptr, N, 0, 1});
 }
 
-// The same tile and slice shape without a split: decode-sized m (at most 64 rows), bias, bf16 or
-// fp32 out; and with a residual (bf16 out).
-extern "C" __global__ void __launch_bounds__(kGemmThreads) DK_BF16_OCCUPANCY
-    mfma_linear_bf16_stream_t64(const uint16_t* x, const uint16_t* w, const uint16_t* bias,
-                                void* out, int64_t M, int64_t N, int64_t K, int out_f32) {
-  gemmBf16<64, 64, 128, true>(x, w, M, N, K, K,
-                              RowMajorOutBf16OrF32{out, reinterpret_cast<const bf16*>(bias), N, 0,
-                                                   out_f32});
-}
-extern "C" __global__ void __launch_bounds__(kGemmThreads) DK_BF16_OCCUPANCY
-    mfma_linear_residual_bf16_stream_t64(const uint16_t* x, const uint16_t* w,
-                                         const uint16_t* bias, const uint16_t* residual,
-                                         uint16_t* out, int64_t M, int64_t N, int64_t K) {
-  gemmBf16<64, 64, 128, true>(x, w, M, N, K, K,
-                              ResidualOut{reinterpret_cast<bf16*>(out),
-                                          reinterpret_cast<const bf16*>(residual),
-                                          reinterpret_cast<const bf16*>(bias), N});
-}
+// The same for more than 64 rows: several row tiles read each weight (cached loads).
+#define DK_MFMA_SPLITK16(name, E, T)                                                            \
+  extern "C" __global__ void __launch_bounds__(kGemmThreads) DK_BF16_OCCUPANCY                  \
+      name(const uint16_t* x, const uint16_t* w, float* part, int64_t M, int64_t N, int64_t K,  \
+           int64_t per) {                                                                       \
+    const int64_t k0 = static_cast<int64_t>(blockIdx.z) * per;                                  \
+    const int64_t len = K - k0 < per ? K - k0 : per;                                            \
+    float* const out = part + static_cast<int64_t>(blockIdx.z) * M * N;                         \
+    gemm16<64, 64, 64, false, E>(x + k0, w + k0, M, N, len, K,                                  \
+                                 RowMajorOut16OrF32<T>{out, nullptr, N, 0, 1});                 \
+  }
+DK_MFMA_SPLITK16(mfma_linear_bf16_splitk_rows_t64, Bf16, bf16)
+DK_MFMA_SPLITK16(mfma_linear_f16_splitk_rows_t64, F16, f16)
 
 extern "C" __global__ void __launch_bounds__(kGemmThreads) DK_BF16_OCCUPANCY
-    mfma_gate_up_silu_bf16_stream_t64(const uint16_t* x, const uint16_t* w_gate_up, uint16_t* out,
-                                      int64_t M, int64_t ffn, int64_t K) {
-  gemmBf16<64, 64, 128, true>(x, w_gate_up, M, 2 * ffn, K, K,
-                              SwiGluOut{reinterpret_cast<bf16*>(out), ffn});
+    mfma_linear_f16_splitk_t64(const uint16_t* x, const uint16_t* w, float* part, int64_t M,
+                               int64_t N, int64_t K, int64_t per) {
+  const int64_t k0 = static_cast<int64_t>(blockIdx.z) * per;
+  const int64_t len = K - k0 < per ? K - k0 : per;
+  float* const out = part + static_cast<int64_t>(blockIdx.z) * M * N;
+  gemm16<64, 64, 128, true, F16>(x + k0, w + k0, M, N, len, K,
+                                 RowMajorOut16OrF32<f16>{out, nullptr, N, 0, 1});
 }
 
-// out[m, n] = bf16(v + bias[n]), or with a residual bf16(residual[m, n] + bf16(v + bias[n])),
-// v = the sum of the split parts in split order: the rounding points of RowMajorOut and
-// ResidualOut.
-extern "C" __global__ void __launch_bounds__(256)
-    splitk_reduce_bf16(const float* part, const uint16_t* bias, const uint16_t* residual,
-                       uint16_t* out, int64_t M, int64_t N, int splits) {
+// out[m, n] = T(v + bias[n]) (or fp32, optional ReLU), or with a residual T(residual[m, n] +
+// T(v + bias[n])), v = the sum of the split parts in split order: the rounding points of
+// RowMajorOut16OrF32 and ResidualOut. Four columns per thread where the rows allow it.
+template <typename T>
+__device__ __forceinline__ void splitkReduce16(const float* part, const T* bias, const T* residual,
+                                               void* out, int64_t M, int64_t N, int splits,
+                                               int out_f32, int relu) {
   const int64_t total = M * N;
-  for (int64_t e = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; e < total;
-       e += static_cast<int64_t>(gridDim.x) * blockDim.x) {
+  auto finish = [&](int64_t e, int64_t col, float v) {
+    if (bias != nullptr) v += ld(bias + col);
+    if (residual != nullptr) v = ld(residual + e) + Num<T>::round(v);
+    return relu ? fmaxf(v, 0.f) : v;
+  };
+  const int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
+  const int64_t first = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (N % 4 == 0 && aligned16(part) && aligned16(out)) {
+    for (int64_t e = first * 4; e < total; e += stride * 4) {
+      f32x4 v = *gp(reinterpret_cast<const f32x4*>(part + e));
+#pragma unroll 4
+      for (int z = 1; z < splits; ++z)
+        v += *gp(reinterpret_cast<const f32x4*>(part + z * total + e));
+      const int64_t col = e % N;
+      float r[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) r[k] = finish(e + k, col + k, v[k]);
+      if (out_f32) {
+        *gp(reinterpret_cast<f32x4*>(static_cast<float*>(out) + e)) = f32x4{r[0], r[1], r[2], r[3]};
+      } else {
+        *gp(reinterpret_cast<uint2*>(static_cast<T*>(out) + e)) = pack16x4(r, T{});
+      }
+    }
+    return;
+  }
+  for (int64_t e = first; e < total; e += stride) {
     float v = gp(part)[e];
     for (int z = 1; z < splits; ++z) v += gp(part)[z * total + e];
-    if (bias != nullptr) v += bf16ToFloat(gp(bias)[e % N]);
-    if (residual != nullptr) v = bf16ToFloat(gp(residual)[e]) + Num<bf16>::round(v);
-    gp(out)[e] = floatToBf16(v);
+    v = finish(e, e % N, v);
+    if (out_f32)
+      st(static_cast<float*>(out) + e, v);
+    else
+      st(static_cast<T*>(out) + e, v);
   }
+}
+extern "C" __global__ void __launch_bounds__(256)
+    splitk_reduce_bf16(const float* part, const bf16* bias, const bf16* residual, void* out,
+                       int64_t M, int64_t N, int splits, int out_f32, int relu) {
+  splitkReduce16(part, bias, residual, out, M, N, splits, out_f32, relu);
+}
+extern "C" __global__ void __launch_bounds__(256)
+    splitk_reduce_f16(const float* part, const f16* bias, const f16* residual, void* out,
+                      int64_t M, int64_t N, int splits, int out_f32, int relu) {
+  splitkReduce16(part, bias, residual, out, M, N, splits, out_f32, relu);
 }
 
 // The split parts of the [q | k | v] projection of decode rows (one new token per row): each

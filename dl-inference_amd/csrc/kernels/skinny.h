@@ -33,6 +33,20 @@ typedef uint32_t U128 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ bf16x8 asBf16x8(const U128& v) { return __builtin_bit_cast(bf16x8, v); }
 
+// The 16-bit element types of the matrix products: D = A B + C of v_mfma_f32_16x16x32_<type>.
+struct Bf16 {
+  __device__ __forceinline__ static f32x4 mma(const U128& a, const U128& b, const f32x4& c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(asBf16x8(a), asBf16x8(b), c, 0, 0, 0);
+  }
+};
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+struct F16 {
+  __device__ __forceinline__ static f32x4 mma(const U128& a, const U128& b, const f32x4& c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a),
+                                                  __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
+  }
+};
+
 __device__ __forceinline__ U128 load16(const void* p) {
   return *reinterpret_cast<const U128*>(p);
 }
@@ -113,8 +127,8 @@ struct XFrag {
 };
 
 // kUnroll: 64-column steps per batch and wave (two batches are in flight); kIdle: leading waves
-// without steps (their partial tiles are zero).
-template <int NF, int MB, int kWaves, int kUnroll = 4, int kIdle = 0>
+// without steps (their partial tiles are zero); E: the operands' type.
+template <int NF, int MB, int kWaves, int kUnroll = 4, int kIdle = 0, class E = Bf16>
 struct SkinnyCore {
   static_assert(kIdle >= 0 && kIdle < kWaves, "at least one wave takes steps");
   static constexpr int kCW = kWaves - kIdle;  // waves that take steps
@@ -225,9 +239,7 @@ struct SkinnyCore {
         for (int f = 0; f < NF; ++f)
 #pragma unroll
           for (int b = 0; b < MB; ++b)
-            acc[f][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(asBf16x8(wb.a[u][f][h]),
-                                                                asBf16x8(xb.x[u][b][h]), acc[f][b],
-                                                                0, 0, 0);
+            acc[f][b] = E::mma(wb.a[u][f][h], xb.x[u][b][h], acc[f][b]);
     }
   }
 

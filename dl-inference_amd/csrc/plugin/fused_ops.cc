@@ -171,6 +171,18 @@ class LinearResidualOp final : public Operator {
       throw std::invalid_argument("linear_residual bias size mismatch");
     const auto splits = static_cast<int>(attrs.value_or<std::int64_t>("splits", 1));
     *out[0] = Tensor::cuda(DType::BFloat16, res.shape(), x.deviceId());
+    if (m > 64) {  // a prompt: K parts of the tiled GEMM, scratch from the caching allocator
+      const std::size_t bytes = dli_hip_linear_residual_rows_workspace(m, n, k);
+      Tensor ws;
+      if (bytes > 0)
+        ws = Tensor::cuda(DType::Float32, {static_cast<std::int64_t>(bytes / sizeof(float))},
+                          x.deviceId());
+      check(dli_hip_linear_residual_rows(ptr(x), ptr(w), in.size() == 4 ? ptr(*in[3]) : nullptr,
+                                         ptr(res), ptr(*out[0]), m, n, k,
+                                         bytes > 0 ? ptr(ws) : nullptr, bytes, ctx.stream),
+            type());
+      return;
+    }
     const std::size_t ws_bytes = dli_hip_splitk_workspace(n, m, splits);
     check(dli_hip_linear_residual(ptr(x), ptr(w), in.size() == 4 ? ptr(*in[3]) : nullptr, ptr(res),
                                   ptr(*out[0]), m, n, k, splits,

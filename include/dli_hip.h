@@ -355,6 +355,14 @@ int dli_hip_qkv_rope_append_ws(const void* hidden, const void* norm_weight, cons
 int dli_hip_linear_residual(const void* x, const void* w, const void* bias, const void* residual,
                             void* out, int64_t m, int64_t n, int64_t k, int splits,
                             void* workspace, size_t workspace_bytes, void* stream);
+/* dli_hip_linear_residual for more than 64 rows, with scratch for K parts: `workspace` of any
+ * content (size from dli_hip_linear_residual_rows_workspace; a smaller one or NULL means fewer
+ * parts), its content afterwards unspecified. k % 8 == 0, x and w 16-byte aligned. */
+size_t dli_hip_linear_residual_rows_workspace(int64_t m, int64_t n, int64_t k);
+int dli_hip_linear_residual_rows(const void* x, const void* w, const void* bias,
+                                 const void* residual, void* out, int64_t m, int64_t n, int64_t k,
+                                 void* workspace, size_t workspace_bytes, void* stream);
+
 
 /* h_out = residual + (x W^T + b) as above, and xn_out = rms_norm(h_out) * norm_weight, both
  * [m, n]. Replaces o_proj + attention_residual + post_attention_layernorm, and down_proj +
