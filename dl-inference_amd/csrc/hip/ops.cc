@@ -220,13 +220,16 @@ enum class Linear16 { kSkinny4, kSkinny16, kTiled };
 // (n <= 4096), else 4 waves of 32 rows. Measured in us (4 waves / 16 waves / tiled with its parts),
 // n x k at m rows: 896 x 896 m = 1 4.3 / 3.3 / 8.6, m = 64 10.3 / 7.1 / 8.2; 896 x 4864 m = 8
 // 13 / 8.3 / 8.7, m = 16 15.2 / 10.7 / 8.9; 4096 x 1024 m = 64 11.4 / 8.7 / 9.8; 3584 x 3584 m = 17
-// 13.9 / 10.0 / 10.9, m = 32 16.5 / 12.6 / 11.4; 4864 x 896 m = 32 6.8 / 8.3 / 9.5, m = 50 10.0 /
-// 12.1 / 9.9; 18944 x 3584 m = 9 29 / 31 / 33, m = 17 42 / 43 / 33.
+// 13.9 / 10.0 / 10.9, m = 32 16.5 / 12.6 / 11.4; 10 x 4096 m = 32 13.1 / 11.6 / 12.4; 4864 x 896
+// m = 32 6.8 / 8.3 / 9.5, m = 50 10.0 / 12.1 / 9.9. From 8192 columns a weight streams from memory,
+// where the tiled kernel is ahead as soon as more than 8 rows share it (a step of 9 rows with a head
+// of 152064 x 3584: 615 us, 639 with the skinny kernel).
 Linear16 linear16Route(int64_t m, int64_t n, int64_t k) {
   if (m > 64 || k % 64 != 0) return Linear16::kTiled;
-  const bool w16 = n <= 4096;
-  if (m > 8 && m * k > (w16 ? 65536 : 32768)) return Linear16::kTiled;
-  return w16 ? Linear16::kSkinny16 : Linear16::kSkinny4;
+  if (n > 4096)
+    return m <= 8 || (n < 8192 && m * k <= 32768) ? Linear16::kSkinny4 : Linear16::kTiled;
+  return m <= 8 || m * k <= 65536 || (n <= 64 && m <= 32) ? Linear16::kSkinny16
+                                                          : Linear16::kTiled;
 }
 
 // Output tiles of the 16-bit GEMM: 128 x 128 from about 168 of them (at 896 columns, 2048 rows /
