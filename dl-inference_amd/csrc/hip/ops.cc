@@ -42,6 +42,8 @@ int badArg(const char* op, const char* what) {
 
 bool validIndexDtype(int dtype) { return dtype == DLI_I64 || dtype == DLI_I32; }
 
+bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
+
 // Grid-stride launches: enough blocks to fill 256 CUs several times over, capped.
 unsigned strideBlocks(int64_t work) {
   const int64_t blocks = (work + 255) / 256;
@@ -93,14 +95,8 @@ DeviceKernel k_packed_dense128("packed_attention", "packed_attention_dense_d128"
 DeviceKernel k_packed_dense128_r128("packed_attention", "packed_attention_dense_d128_r128");
 DeviceKernel k_packed_merge64("packed_attention", "packed_attention_merge_d64");
 DeviceKernel k_packed_merge128("packed_attention", "packed_attention_merge_d128");
-DeviceKernel k_mfma_linear64("mfma_gemm", "mfma_linear_f32_t64");
-DeviceKernel k_mfma_linear128("mfma_gemm", "mfma_linear_f32_t128");
-DeviceKernel k_mfma_matmul64("mfma_gemm", "mfma_matmul_f32_t64");
-DeviceKernel k_mfma_matmul128("mfma_gemm", "mfma_matmul_f32_t128");
 DeviceKernel k_conv_small9("conv", "conv2d_small_f32_p9");
 DeviceKernel k_conv_small27("conv", "conv2d_small_f32_p27");
-DeviceKernel k_mfma_conv64("mfma_gemm", "mfma_conv2d_f32_t64");
-DeviceKernel k_mfma_conv128("mfma_gemm", "mfma_conv2d_f32_t128");
 // [tile form: TileForm16]
 DeviceKernel k_mfma_bf16[4] = {{"mfma_gemm", "mfma_linear_bf16_t64"},
                                {"mfma_gemm", "mfma_linear_bf16_t64_g2"},
@@ -120,25 +116,76 @@ DeviceKernel k_splitk_reduce_bf16("mfma_gemm", "splitk_reduce_bf16");
 DeviceKernel k_mfma_f16_splitk("mfma_gemm", "mfma_linear_f16_splitk_t64");
 DeviceKernel k_mfma_f16_rows("mfma_gemm", "mfma_linear_f16_splitk_rows_t64");
 DeviceKernel k_splitk_reduce_f16("mfma_gemm", "splitk_reduce_f16");
-DeviceKernel k_mfma_splitk("mfma_gemm", "mfma_linear_f32_splitk_t64");
-DeviceKernel k_splitk_reduce("mfma_gemm", "splitk_reduce_f32");
-DeviceKernel k_mfma_conv_splitk("mfma_gemm", "mfma_conv2d_f32_splitk_t64");
-DeviceKernel k_conv_splitk_reduce("mfma_gemm", "conv_splitk_reduce_f32");
+// fp32 GEMMs by K groups per workgroup (FormF32)
+constexpr const char* kF32 = "mfma_gemm_f32";
+DeviceKernel k_f32_linear[5] = {{kF32, "mfma_linear_f32_g1"},
+                                {kF32, "mfma_linear_f32_g2"},
+                                {kF32, "mfma_linear_f32_scalar"},
+                                {kF32, "mfma_linear_f32_stream"},
+                                {kF32, "mfma_linear_f32_m16"}};
+DeviceKernel k_f32_matmul[3] = {{kF32, "mfma_matmul_f32_g1"},
+                                {kF32, "mfma_matmul_f32_g2"},
+                                {kF32, "mfma_matmul_f32_scalar"}};
+DeviceKernel k_f32_conv[3] = {{kF32, "mfma_conv2d_f32_g1"},
+                              {kF32, "mfma_conv2d_f32_g2"},
+                              {kF32, "mfma_conv2d_f32_scalar"}};
+DeviceKernel k_splitk_reduce(kF32, "splitk_reduce_f32");
+DeviceKernel k_conv_splitk_reduce(kF32, "conv_splitk_reduce_f32");
 
-// Split count of an fp32 linear: 64 x 64 tiles are split over K (chunks of at least 256, eight
-// 32-wide slices) until there are about 512 workgroups (two per CU); 1 = no split. A workgroup
-// walks its K chunk one slice per load round trip, so a few tiles over a long K would otherwise
-// take that many round trips.
-int64_t linearSplits(int64_t m, int64_t n, int64_t k) {
-  const int64_t tiles = ((m + 63) / 64) * ((n + 63) / 64);
-  int64_t splits = 1;
-  while (splits < 16 && tiles * splits * 2 <= 512 && k / (splits * 2) >= 256) splits *= 2;
-  return splits;
+// Form of an fp32 GEMM (mfma_gemm_f32.hip): kernel index, threads, K parts of `per` columns.
+enum FormF32 { kG1 = 0, kG2 = 1, kScalar = 2, kStream = 3, kM16 = 4 };
+struct PlanF32 {
+  int form;
+  unsigned threads;
+  int64_t tile_rows, parts, per;
+};
+// `vec`: rows of 16-byte chunks (K % 4 == 0, aligned); `linear`: the forms of a few rows exist; at
+// most max_parts parts.
+//
+// Three workgroups of one K group (_g1) fit a CU and overlap each other's loads, staging and matrix
+// instructions; where the tiles alone are fewer, K parts make up for it, or, where the parts' traffic
+// would cost more, a second K group in the workgroup. In us: conv 384 x 4096 pixels x 1728 (384
+// tiles) 104 in one part, 68 + 5 for the sum in two; 256 x 4096 x 3456 (256 tiles) 108 with two
+// groups, 87 + 5 in three parts of one; linear 1000 x 896 x 4864 (224 tiles) 65 with two groups, 68
+// to 72 in parts; 1000 x 896 x 896 17 with two groups, 21 with one, 23 in two parts; a conv of 3
+// images (24 tiles) 12 + 4 with two groups and 11 to 16 parts, 14 + 4 with one.
+constexpr int64_t kMaxPartsF32 = 16;
+PlanF32 planF32(int64_t rows, int64_t cols, int64_t k, bool vec, bool linear, int64_t max_parts) {
+  PlanF32 p{kG1, 256, 64, 1, k};
+  const int64_t tiles = ((rows + 63) / 64) * ((cols + 63) / 64);
+  const int64_t slices = (k + 31) / 32;
+  const bool many = !linear && tiles >= 128 && vec;  // parts of one group
+  int groups = 1;
+  if (!vec) {
+    p.form = kScalar;
+  } else if (linear && rows <= 16) {
+    p.form = kM16, p.tile_rows = 16, groups = 4;
+  } else if (linear && rows <= 64) {
+    p.form = kStream, groups = 2;
+  } else if (tiles <= 256 && !many) {
+    p.form = kG2, groups = 2;
+  }
+  p.threads = 256u * groups;
+  // at least two slices per group (six where a workgroup has one)
+  int64_t s = (many ? 768 : 256) / tiles;
+  const int64_t least = many ? 6 : 2 * groups;
+  if (s > slices / least) s = slices / least;
+  if (s > max_parts) s = max_parts;
+  if (s > 1) {
+    p.per = (slices + s - 1) / s * 32;
+    p.parts = (k + p.per - 1) / p.per;
+  } else if (many && tiles <= 256) {
+    p.form = kG2, p.threads = 512;
+  }
+  return p;
 }
-
-// MFMA GEMM tiles: 128 x 128 once those alone give every CU a workgroup, else 64 x 64.
-bool bigTiles(int64_t rows, int64_t cols) {
-  return ((rows + 127) / 128) * ((cols + 127) / 128) >= 256;
+// parts that a workspace holds
+int64_t partsHeldF32(const void* workspace, size_t bytes, int64_t rows, int64_t cols) {
+  const auto held = static_cast<int64_t>(bytes / sizeof(float)) / (rows * cols);
+  return workspace == nullptr || held < 1 ? 1 : (held < kMaxPartsF32 ? held : kMaxPartsF32);
+}
+size_t partBytesF32(const PlanF32& p, int64_t rows, int64_t cols) {
+  return p.parts > 1 ? static_cast<size_t>(p.parts * rows * cols) * sizeof(float) : 0;
 }
 
 constexpr int64_t kMaxGridY = 65535;
@@ -163,8 +210,6 @@ int unary(FloatKernels& kernels, const char* op, int dtype, const void* x, void*
   if (x == nullptr || out == nullptr) return badArg(op, "NULL pointer");
   return launch(*k, {strideBlocks(total)}, {256}, 0, stream, x, out, total);
 }
-
-bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 // ---- packed-row attention (packed_attention.hip) ------------------------------------------------
 // Rows (queries x heads of a KV group) per workgroup: 128, or 64 for units of at most 64 rows.
@@ -488,10 +533,8 @@ size_t dli_hip_conv2d_workspace(int dtype, int64_t n, int64_t in_c, int64_t out_
   if (dtype != DLI_F32 || n <= 0 || in_c <= 0 || out_c <= 0 || kernel_h <= 0 || kernel_w <= 0 ||
       out_h <= 0 || out_w <= 0)
     return 0;
-  const int64_t pixels = n * out_h * out_w;
-  if (bigTiles(out_c, pixels)) return 0;
-  const int64_t splits = linearSplits(out_c, pixels, in_c * kernel_h * kernel_w);
-  return splits > 1 ? static_cast<size_t>(splits * out_c * pixels) * sizeof(float) : 0;
+  const int64_t pixels = n * out_h * out_w, patch = in_c * kernel_h * kernel_w;
+  return partBytesF32(planF32(out_c, pixels, patch, patch % 4 == 0, false, kMaxPartsF32), out_c, pixels);
 }
 
 int dli_hip_conv2d_act(int dtype, const void* x, const void* weight, const void* bias, void* out,
@@ -536,31 +579,21 @@ int dli_hip_conv2d_act(int dtype, const void* x, const void* weight, const void*
                     i32(out_c), i32(out_h), i32(out_w), i32(stride_h), i32(stride_w), i32(pad_h),
                     i32(pad_w), relu, tab);
     }
-    const bool big = bigTiles(out_c, pixels);
-    const int64_t tile = big ? 128 : 64;
-    const int64_t splits = big ? 1 : linearSplits(out_c, pixels, patch);
-    const size_t need = static_cast<size_t>(splits * out_c * pixels) * sizeof(float);
-    if (splits > 1 && workspace != nullptr && workspace_bytes >= need &&
-        (out_c + 63) / 64 <= kMaxGridY) {
-      const int64_t per = (patch + splits - 1) / splits;
-      int rc = launch(k_mfma_conv_splitk,
-                      {static_cast<unsigned>((pixels + 63) / 64),
-                       static_cast<unsigned>((out_c + 63) / 64), static_cast<unsigned>(splits)},
-                      {256}, 0, stream, x, weight, workspace, i32(n), i32(in_c), i32(h), i32(w),
-                      i32(out_c), i32(kernel_h), i32(kernel_w), i32(out_h), i32(out_w),
-                      i32(stride_h), i32(stride_w), i32(pad_h), i32(pad_w), i32(per));
-      if (rc != 0) return rc;
-      return launch(k_conv_splitk_reduce, {strideBlocks(out_c * pixels)}, {256}, 0, stream,
-                    workspace, bias, out, out_c, pixels, out_h * out_w,
-                    static_cast<int>(splits), relu);
-    }
-    if ((out_c + tile - 1) / tile <= kMaxGridY) {
-      return launch(big ? k_mfma_conv128 : k_mfma_conv64,
-                    {static_cast<unsigned>((pixels + tile - 1) / tile),
-                     static_cast<unsigned>((out_c + tile - 1) / tile)},
-                    {256}, 0, stream, x, weight, bias, out, i32(n), i32(in_c), i32(h), i32(w),
-                    i32(out_c), i32(kernel_h), i32(kernel_w), i32(out_h), i32(out_w),
-                    i32(stride_h), i32(stride_w), i32(pad_h), i32(pad_w), relu);
+    const bool vec = patch % 4 == 0 && aligned16(weight);
+    const PlanF32 p = planF32(out_c, pixels, patch, vec, false,
+                              partsHeldF32(workspace, workspace_bytes, out_c, pixels));
+    if ((out_c + 63) / 64 <= kMaxGridY) {
+      const int rc =
+          launch(k_f32_conv[p.form],
+                 {static_cast<unsigned>((pixels + 63) / 64), static_cast<unsigned>((out_c + 63) / 64),
+                  static_cast<unsigned>(p.parts)},
+                 {p.threads}, 0, stream, x, weight, bias, out, workspace, i32(n), i32(in_c), i32(h),
+                 i32(w), i32(out_c), i32(kernel_h), i32(kernel_w), i32(out_h), i32(out_w),
+                 i32(stride_h), i32(stride_w), i32(pad_h), i32(pad_w), i32(p.per), relu);
+      if (rc != 0 || p.parts == 1) return rc;
+      return launch(k_conv_splitk_reduce, {strideBlocks((out_c * pixels + 3) / 4)}, {256}, 0,
+                    stream, workspace, bias, out, out_c, pixels, out_h * out_w,
+                    static_cast<int>(p.parts), relu);
     }
   }
   DeviceKernel* k = k_conv2d.pick(dtype);
@@ -584,8 +617,7 @@ size_t dli_hip_linear_workspace(int dtype, int64_t m, int64_t n, int64_t k) {
     return tiled16Workspace(m, n, k);
   }
   if (dtype != DLI_F32) return 0;
-  const int64_t splits = linearSplits(m, n, k);
-  return splits > 1 ? static_cast<size_t>(splits * m * n) * sizeof(float) : 0;
+  return partBytesF32(planF32(m, n, k, k % 4 == 0, true, kMaxPartsF32), m, n);
 }
 
 int dli_hip_linear_act(int dtype, int out_dtype, const void* x, const void* w, const void* bias,
@@ -600,26 +632,18 @@ int dli_hip_linear_act(int dtype, int out_dtype, const void* x, const void* w, c
   if (x == nullptr || w == nullptr || out == nullptr) return badArg("linear", "NULL pointer");
   const int out_f32 = out_dtype == DLI_F32 ? 1 : 0;
   const int relu = activation == DLI_ACT_RELU ? 1 : 0;
-  const bool big = bigTiles(m, n);
-  const int64_t tile = big ? 128 : 64;
-  const Dim3 grid{static_cast<unsigned>((n + tile - 1) / tile),
-                  static_cast<unsigned>((m + tile - 1) / tile)};
-  const bool grid_ok = (m + tile - 1) / tile <= kMaxGridY;
-  if (dtype == DLI_F32 && grid_ok) {
-    const int64_t splits = linearSplits(m, n, k);
-    const size_t need = static_cast<size_t>(splits * m * n) * sizeof(float);
-    if (splits > 1 && workspace != nullptr && workspace_bytes >= need) {
-      const int64_t per = (k + splits - 1) / splits;
-      int rc = launch(k_mfma_splitk,
-                      {static_cast<unsigned>((n + 63) / 64), static_cast<unsigned>((m + 63) / 64),
-                       static_cast<unsigned>(splits)},
-                      {256}, 0, stream, x, w, workspace, m, n, k, per);
-      if (rc != 0) return rc;
-      return launch(k_splitk_reduce, {strideBlocks(m * n)}, {256}, 0, stream, workspace, bias,
-                    out, m, n, static_cast<int>(splits), relu);
-    }
-    return launch(big ? k_mfma_linear128 : k_mfma_linear64, grid, {256}, 0, stream, x, w, bias,
-                  out, m, n, k, relu);
+  if (dtype == DLI_F32 && (m + 63) / 64 <= kMaxGridY) {
+    const bool vec = k > 0 && k % 4 == 0 && aligned16(x) && aligned16(w);
+    const PlanF32 p =
+        planF32(m, n, k, vec, true, partsHeldF32(workspace, workspace_bytes, m, n));
+    const int rc = launch(k_f32_linear[p.form],
+                          {static_cast<unsigned>((n + 63) / 64),
+                           static_cast<unsigned>((m + p.tile_rows - 1) / p.tile_rows),
+                           static_cast<unsigned>(p.parts)},
+                          {p.threads}, 0, stream, x, w, bias, out, workspace, m, n, k, p.per, relu);
+    if (rc != 0 || p.parts == 1) return rc;
+    return launch(k_splitk_reduce, {strideBlocks((m * n + 3) / 4)}, {256}, 0, stream, workspace,
+                  bias, out, m, n, static_cast<int>(p.parts), relu);
   }
   int rc;
   const bool h16 = dtype == DLI_BF16 || dtype == DLI_F16;
@@ -653,13 +677,13 @@ int dli_hip_matmul(int dtype, const void* a, const void* b, void* out, int64_t m
   if (m < 0 || n < 0 || k < 0) return badArg("matmul", "negative size");
   if (m == 0 || n == 0) return 0;
   if (a == nullptr || b == nullptr || out == nullptr) return badArg("matmul", "NULL pointer");
-  const bool big = bigTiles(m, n);
-  const int64_t tile = big ? 128 : 64;
-  if (dtype == DLI_F32 && (m + tile - 1) / tile <= kMaxGridY)
-    return launch(big ? k_mfma_matmul128 : k_mfma_matmul64,
-                  {static_cast<unsigned>((n + tile - 1) / tile),
-                   static_cast<unsigned>((m + tile - 1) / tile)},
-                  {256}, 0, stream, a, b, out, m, n, k);
+  if (dtype == DLI_F32 && (m + 63) / 64 <= kMaxGridY) {
+    const bool vec = k > 0 && k % 4 == 0 && aligned16(a);
+    const PlanF32 p = planF32(m, n, k, vec, false, 1);
+    return launch(k_f32_matmul[p.form],
+                  {static_cast<unsigned>((n + 63) / 64), static_cast<unsigned>((m + 63) / 64)},
+                  {p.threads}, 0, stream, a, b, out, m, n, k);
+  }
   DeviceKernel* kt = k_gemm.pick(dtype);
   if (kt == nullptr) return badDtype("matmul", dtype);
   if ((m + 63) / 64 > kMaxGridY) return badArg("matmul", "m too large");

@@ -1,301 +1,28 @@
-// MFMA GEMMs of the generic operators on gfx950 (linear, matmul and conv2d for many rows; decode
-// sizes use the weight-streaming kernels of gemm.hip / decode.hip).
+// 16-bit MFMA GEMMs on gfx950 (linears and the fused projections of many rows; decode sizes use the
+// weight-streaming kernels of gemm.hip / decode.hip; fp32: mfma_gemm_f32.hip).
 //
 //   C[r, c] = sum_k A(r, k) * B(c, k), then an epilogue per output element (bias, ReLU, layout)
 //
-//  mfma_linear_f32_<t>      fp32: A = x [M, K], B = w [N, K] (linear/kernel.py:6-44), or
-//  mfma_matmul_f32          B = b [K, N] (matmul/kernel.py:6-40); fp32 MFMA 16x16x4
-//  mfma_conv2d_f32          im2col-free conv2d (conv2d/kernel.py:6-49): A = weight [OC, C*KH*KW]
-//                           rows, B = the input patch of each output pixel, gathered from NCHW
-//                           x while staging (never materialised); out NCHW, optional fused ReLU
-//  mfma_linear_bf16_<t>, mfma_linear_f16_<t>  16-bit x, w (K % 8 == 0), MFMA 16x16x32, fp32
-//                           accumulation, 16-bit or fp32 out, optional ReLU. (f16, 1000 x 4864 x
-//                           896: 252 us on the general kernel of gemm.hip, 19 us here)
+//  mfma_linear_bf16_<t>, mfma_linear_f16_<t>  16-bit x, w (K % 8 == 0; linear/kernel.py:6-44), MFMA
+//                           16x16x32, fp32 accumulation, 16-bit or fp32 out, optional ReLU. (f16,
+//                           1000 x 4864 x 896: 252 us on the general kernel of gemm.hip, 19 us here)
 //  mfma_linear_residual_bf16_<t>  the same plus a residual add (bf16 out)
 //  mfma_gate_up_silu_bf16_<t>     the same over an interleaved gate/up weight, SwiGLU epilogue
-//  mfma_linear_f32_splitk   fp32 linear / conv2d with K split over grid.z into a workspace,
-//  mfma_conv2d_f32_splitk   then a fixed-order sum with bias and ReLU (splitk_reduce_f32,
-//                           conv_splitk_reduce_f32)
+//  mfma_qkv_heads_bf16_<t>        q|k|v projection with RoPE into attention's layout
+//  *_splitk*                K split over grid.z into a workspace, then a fixed-order sum
 //
-// Work split: a 256-thread workgroup owns a BM x BN tile of C (4 waves, 2 x 2, each BM/2 x BN/2
-// as 16 x 16 MFMA tiles) and walks K in BK-wide slices. A slice of A and B is loaded from global
-// memory into registers (coalesced: consecutive lanes take consecutive k of a row, or
-// consecutive rows/pixels when those are contiguous in memory), written to LDS as [row][k] with
-// a padded row pitch, and read back as MFMA fragments; the next slice's loads are in flight
-// while the current one is multiplied (the bf16 GEMM keeps two slices in flight and two LDS
-// buffers, and orders its tiles by XCD: see the bf16 core). Rows, columns and k past the ends
-// load zeros (or, in the bf16 GEMM, clamped rows whose results are dropped), so any shape works.
-// Every output is a fixed-order sum: results do not depend on timing.
-//
-// Conv output pixels are the C columns, so the 16 lanes that share an output row of an MFMA
-// tile store 16 consecutive pixels of one channel (coalesced NCHW stores).
+// Work split: 256 threads own a BM x BN tile of C (4 waves, 2 x 2, each BM/2 x BN/2 as 16 x 16 MFMA
+// tiles) and walk K in BK-wide slices, two slices in flight in registers and two LDS buffers, tiles
+// ordered by XCD (gemm_tiles.h). Rows and columns past the ends load clamped rows whose results are
+// dropped and k past the end loads zeros, so any shape works. Every output is a fixed-order sum:
+// results do not depend on timing.
 #include "common.h"
+#include "gemm_tiles.h"
 #include "skinny.h"
 
 using namespace dk;
 
 namespace {
-
-constexpr int kGemmThreads = 256;
-
-// ---- operand sources -------------------------------------------------------------------------
-// load(row, k): element (row, k) as fp32, zero outside [0, rows) x [0, K). kFastK: consecutive k
-// of a row are adjacent in memory (else consecutive rows are).
-
-struct RowsK {  // p[row * ld + k]
-  static constexpr bool kFastK = true;
-  const float* p;
-  int64_t rows, K, ld;
-  __device__ __forceinline__ float load(int64_t row, int64_t k) const {
-    return row < rows && k < K ? gp(p)[row * ld + k] : 0.f;
-  }
-};
-
-struct KRows {  // p[k * ld + row] (matmul's b [K, N])
-  static constexpr bool kFastK = false;
-  const float* p;
-  int64_t rows, K, ld;
-  __device__ __forceinline__ float load(int64_t row, int64_t k) const {
-    return row < rows && k < K ? gp(p)[k * ld + row] : 0.f;
-  }
-};
-
-// Source hooks used by gemmF32 (no-ops for the plain layouts): begin() once per workgroup,
-// prepare() for every K slice before it is fetched (threads < BK fill a per-slice table),
-// load(row, k, kl, tab) with kl = k - slice start.
-struct NoTable {
-  __device__ __forceinline__ void begin(int64_t, int, int) {}
-  template <int BK>
-  __device__ __forceinline__ void prepareT(int64_t, int, int2*) const {}
-};
-
-struct RowsKT : RowsK, NoTable {
-  __device__ __forceinline__ float load(int64_t row, int64_t k, int, const int2*) const {
-    return RowsK::load(row, k);
-  }
-};
-
-struct KRowsT : KRows, NoTable {
-  __device__ __forceinline__ float load(int64_t row, int64_t k, int, const int2*) const {
-    return KRows::load(row, k);
-  }
-};
-
-// Input patch of a zero-padded NCHW conv: column `row` = output pixel (n, oy, ox), k = (c, ky,
-// kx) over k_base + [0, K). The tile's columns are fixed per thread (row = c0 + t % BN), so
-// begin() decomposes the pixel once; prepare() tabulates (c * H * W + ky * W + kx, ky, kx) for
-// the BK k of a slice, and a load is a table read, two bounds checks and one gather. 32-bit
-// index math (the host checks that every index fits).
-struct ConvPatch {
-  static constexpr bool kFastK = false;
-  const float* x;
-  int rows, K, k_base, C, H, W, KH, KW, OH, OW, SH, SW, PH, PW;
-  bool valid = false;
-  int iy0 = 0, ix0 = 0, base = 0;
-  __device__ __forceinline__ void begin(int64_t c0, int t, int bn) {
-    const int pixel = static_cast<int>(c0) + t % bn;
-    valid = pixel < rows;
-    const int ox = pixel % OW, q = pixel / OW;
-    const int oy = q % OH, n = q / OH;
-    iy0 = oy * SH - PH;
-    ix0 = ox * SW - PW;
-    base = n * C * H * W + iy0 * W + ix0;
-  }
-  template <int BK>
-  __device__ __forceinline__ void prepareT(int64_t k0, int t, int2* tab) const {
-    const int k = static_cast<int>(k0) + t;
-    if (t < BK && k < K) {
-      const int kk = k_base + k, khw = KH * KW;
-      const int c = kk / khw, rem = kk - c * khw;
-      const int ky = rem / KW, kx = rem - ky * KW;
-      tab[t] = int2{(c * H + ky) * W + kx, (ky << 16) | kx};
-    }
-  }
-  __device__ __forceinline__ float load(int64_t, int64_t k, int kl, const int2* tab) const {
-    if (!valid || k >= K) return 0.f;
-    const int2 e = tab[kl];
-    const int iy = iy0 + (e.y >> 16), ix = ix0 + (e.y & 0xFFFF);
-    if (iy < 0 || iy >= H || ix < 0 || ix >= W) return 0.f;
-    return gp(x)[base + e.x];
-  }
-};
-
-// ---- tile order ----------------------------------------------------------------------------------
-// Workgroups are handed to the 8 XCDs round robin by linear id, so XCD x gets the x-th contiguous
-// range of tiles of a grouped order (kGroupRows row blocks per group, row blocks fastest): the
-// tiles one XCD runs at once share A row blocks and B column blocks in its L2. (gridDim.x, y) =
-// (column tiles, row tiles); each blockIdx.z slice (a K split) is mapped the same way. At
-// 8192 x 896 x 4864 (down_proj over a 4 x 2048 prompt) this took the bf16 GEMM from 110 to
-// 79 us; with the plain order, the 7 column tiles of a row block ran on 7 XCDs, each fetching
-// the row block from memory.
-constexpr int kGroupRows = 8;
-
-__device__ __forceinline__ void groupedTile(int BM, int BN, int64_t& r0, int64_t& c0) {
-  const uint64_t nn = gridDim.x, nm = gridDim.y, T = nn * nm;
-  const uint64_t L = blockIdx.x + nn * blockIdx.y;
-  const uint64_t x = L % 8, l = L / 8;
-  const uint64_t g = x * (T / 8) + (x < T % 8 ? x : T % 8) + l;  // a bijection of [0, T)
-  const uint64_t per = kGroupRows * nn, grp = g / per, first = grp * kGroupRows;
-  const uint64_t gs = nm - first < kGroupRows ? nm - first : kGroupRows;
-  const uint64_t in = g - grp * per;
-  r0 = static_cast<int64_t>(first + in % gs) * BM;
-  c0 = static_cast<int64_t>(in / gs) * BN;
-}
-
-// ---- fp32 core ---------------------------------------------------------------------------------
-// v_mfma_f32_16x16x4_f32: lane l supplies A[l % 16][kk] and B[kk][l % 16] for the step's k
-// index kk = l / 16 and receives D[(l / 16) * 4 + i][l % 16], i < 4.
-// LDS layout of one operand's K slice, chosen by how the source is staged:
-//   kFastK (lanes take consecutive k of a row): [row][k], pitch BK + 4 floats (16-byte aligned
-//     rows whose starts fall in distinct banks for the 16 rows of a fragment read), and a
-//     lane's 4 consecutive k come in one 16-byte read;
-//   otherwise (lanes take consecutive rows): [k][row], pitch ROWS + 2, so the stash writes
-//     consecutive words and the four lane groups of a fragment read (k 8 apart) start 16
-//     banks apart; 4 single reads.
-template <bool kFastK, int ROWS, int BK>
-struct SliceLayout {
-  static constexpr int kPitch = kFastK ? BK + 4 : ROWS + 2;
-  static constexpr int kFloats = kFastK ? ROWS * kPitch : BK * kPitch;
-  __device__ __forceinline__ static int at(int row, int k) {
-    return kFastK ? row * kPitch + k : k * kPitch + row;
-  }
-  // x[row][k .. k + 3], k a multiple of 4
-  __device__ __forceinline__ static float4 four(const float* x, int row, int k) {
-    if constexpr (kFastK) {
-      return *reinterpret_cast<const float4*>(&x[at(row, k)]);
-    } else {
-      return float4{x[at(row, k)], x[at(row, k + 1)], x[at(row, k + 2)], x[at(row, k + 3)]};
-    }
-  }
-};
-
-template <int BM, int BN, class ASrc, class BSrc, class Epi>
-__device__ __forceinline__ void gemmF32(ASrc A, BSrc B, int64_t R, int64_t Cn, int64_t K,
-                                        const Epi& epi) {
-  // 32-wide K slices (64 measured no faster on the CNN layers and wastes half a slice when K is
-  // small).
-  constexpr int BK = 32;
-  using LA = SliceLayout<ASrc::kFastK, BM, BK>;
-  using LB = SliceLayout<BSrc::kFastK, BN, BK>;
-  constexpr int TM = BM / 32, TN = BN / 32;
-  constexpr int AE = BM * BK / kGemmThreads, BE = BN * BK / kGemmThreads;
-  __shared__ __attribute__((aligned(16))) float As[LA::kFloats];
-  __shared__ __attribute__((aligned(16))) float Bs[LB::kFloats];
-  const int t = threadIdx.x, lane = t % kWave, wave = t / kWave;
-  const int wr = wave / 2, wc = wave % 2;
-  int64_t r0, c0;
-  groupedTile(BM, BN, r0, c0);
-  __shared__ int2 ktab[2][BK];  // per-slice k table of a source that has one (double-buffered)
-  float ra[AE], rb[BE];
-  auto slot = [&](int e, int rows_in_tile, bool fast_k, int& row, int& k) {
-    if (fast_k) {
-      row = e / BK;
-      k = e % BK;
-    } else {
-      row = e % rows_in_tile;
-      k = e / rows_in_tile;
-    }
-  };
-  auto fetch = [&](int64_t k0, const int2* tab) {
-#pragma unroll
-    for (int i = 0; i < AE; ++i) {
-      int row, k;
-      slot(t + i * kGemmThreads, BM, ASrc::kFastK, row, k);
-      ra[i] = A.load(r0 + row, k0 + k, k, tab);
-    }
-#pragma unroll
-    for (int i = 0; i < BE; ++i) {
-      int row, k;
-      slot(t + i * kGemmThreads, BN, BSrc::kFastK, row, k);
-      rb[i] = B.load(c0 + row, k0 + k, k, tab);
-    }
-  };
-  auto prepare = [&](int64_t k0, int2* tab) { B.template prepareT<BK>(k0, t, tab); };
-  auto stash = [&] {
-#pragma unroll
-    for (int i = 0; i < AE; ++i) {
-      int row, k;
-      slot(t + i * kGemmThreads, BM, ASrc::kFastK, row, k);
-      As[LA::at(row, k)] = ra[i];
-    }
-#pragma unroll
-    for (int i = 0; i < BE; ++i) {
-      int row, k;
-      slot(t + i * kGemmThreads, BN, BSrc::kFastK, row, k);
-      Bs[LB::at(row, k)] = rb[i];
-    }
-  };
-  f32x4 acc[TM][TN];
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int fr = lane % 16, fk = lane / 16;
-  A.begin(r0, t, BM);
-  B.begin(c0, t, BN);
-  prepare(0, ktab[0]);
-  __syncthreads();
-  fetch(0, ktab[0]);
-  int slice = 0;
-  for (int64_t k0 = 0; k0 < K; k0 += BK, ++slice) {
-    // the table of slice + 1 goes to the buffer that slice - 1's fetch read two barriers ago
-    if (k0 + BK < K) prepare(k0 + BK, ktab[(slice + 1) & 1]);
-    __syncthreads();  // every wave is done reading the previous slice
-    stash();
-    __syncthreads();
-    if (k0 + BK < K) fetch(k0 + BK, ktab[(slice + 1) & 1]);
-    // In each 32-k half of a slice, MFMA step s uses k = fk * 8 + s for lane group fk (A and B
-    // alike, so each step is still a 4-term slice of the dot products).
-#pragma unroll
-    for (int kh = 0; kh < BK / 32; ++kh) {
-      float4 a4[TM][2], b4[TN][2];
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-          a4[i][h] = LA::four(As, wr * (BM / 2) + i * 16 + fr, kh * 32 + fk * 8 + h * 4);
-#pragma unroll
-      for (int j = 0; j < TN; ++j)
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-          b4[j][h] = LB::four(Bs, wc * (BN / 2) + j * 16 + fr, kh * 32 + fk * 8 + h * 4);
-#pragma unroll
-      for (int s = 0; s < 8; ++s)
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-          for (int j = 0; j < TN; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(
-                a4[i][s / 4][s % 4], b4[j][s / 4][s % 4], acc[i][j], 0, 0, 0);
-    }
-  }
-  if constexpr (Epi::kPairs) {
-    // column blocks 2 p and 2 p + 1 (16 wide) of a wave's tile go to one epi.pair call: the
-    // C columns of an interleaved [gate 16 | up 16] weight pair up in the same lane
-    static_assert(TN % 2 == 0, "column block pairs");
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; j += 2)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int64_t row = r0 + wr * (BM / 2) + i * 16 + fk * 4 + v;
-          const int64_t col = c0 + wc * (BN / 2) + j * 16 + fr;
-          if (row < R && col + 16 < Cn) epi.pair(row, col, acc[i][j][v], acc[i][j + 1][v]);
-        }
-  } else {
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-      for (int j = 0; j < TN; ++j)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int64_t row = r0 + wr * (BM / 2) + i * 16 + fk * 4 + v;
-          const int64_t col = c0 + wc * (BN / 2) + j * 16 + fr;
-          if (row < R && col < Cn) epi(row, col, acc[i][j][v]);
-        }
-  }
-}
 
 // ---- 16-bit core ---------------------------------------------------------------------------------
 // v_mfma_f32_16x16x32_bf16 / _f16 (E = Bf16 / F16): lane l supplies A[l % 16][(l / 16) * 8 + j] and
@@ -650,21 +377,6 @@ __device__ __forceinline__ U128 packBf16x8(const float (&f)[8]) {
               packBf16x2(f[6], f[7])};
 }
 
-// out[row * ldo + col] = act(v + bias[col]) as T
-template <typename T, typename BiasT>
-struct RowMajorOut {
-  static constexpr bool kPairs = false;
-  T* out;
-  const BiasT* bias;
-  int64_t ldo;
-  int relu;
-  __device__ __forceinline__ void operator()(int64_t row, int64_t col, float v) const {
-    if (bias != nullptr) v += ld(bias + col);
-    if (relu) v = fmaxf(v, 0.f);
-    st(out + row * ldo + col, v);
-  }
-};
-
 __device__ __forceinline__ void unpack16x8(const U128& w, float (&f)[8], bf16) {
   unpackBf16x8(w, f);
 }
@@ -690,8 +402,8 @@ __device__ __forceinline__ uint2 pack16x4(const float (&f)[4], f16) {
                                          static_cast<f16>(f[2]), static_cast<f16>(f[3])});
 }
 
-// RowMajorOut of 16-bit operands (T = bf16 or f16) with the output type chosen at run time (one
-// copy of the GEMM per kernel: two inlined copies, one per output type, took the kernel past 256
+// out[row * ldo + col] = act(v + bias[col]) of 16-bit operands (T = bf16 or f16), the output type
+// chosen at run time (one copy of the GEMM per kernel: two inlined copies, one per output type, took the kernel past 256
 // registers)
 template <typename T>
 struct RowMajorOut16OrF32 {
@@ -904,106 +616,7 @@ struct QkvHeadsOut {
   }
 };
 
-// out[n, oc, oy, ox] = act(v + bias[oc]) for C row oc and C column pixel (n, oy, ox)
-struct ConvOut {
-  static constexpr bool kPairs = false;
-  float* out;
-  const float* bias;
-  int64_t OC, OHW;
-  int relu;
-  __device__ __forceinline__ void operator()(int64_t oc, int64_t pixel, float v) const {
-    if (bias != nullptr) v += gp(bias)[oc];
-    if (relu) v = fmaxf(v, 0.f);
-    const int64_t n = pixel / OHW, p = pixel - n * OHW;
-    gp(out)[(n * OC + oc) * OHW + p] = v;
-  }
-};
-
 }  // namespace
-
-// Tile sizes: _t64 for C up to a few hundred tiles of 64 x 64, _t128 for larger ones.
-#define DK_MFMA_F32(BM, BN)                                                                     \
-  extern "C" __global__ void __launch_bounds__(kGemmThreads)                                   \
-      mfma_linear_f32_t##BM(const float* x, const float* w, const float* bias, float* out,     \
-                            int64_t M, int64_t N, int64_t K, int relu) {                       \
-    gemmF32<BM, BN>(RowsKT{{x, M, K, K}}, RowsKT{{w, N, K, K}}, M, N, K,                       \
-                    RowMajorOut<float, float>{out, bias, N, relu});                            \
-  }                                                                                            \
-  extern "C" __global__ void __launch_bounds__(kGemmThreads)                                   \
-      mfma_matmul_f32_t##BM(const float* a, const float* b, float* out, int64_t M, int64_t N,  \
-                            int64_t K) {                                                       \
-    gemmF32<BM, BN>(RowsKT{{a, M, K, K}}, KRowsT{{b, N, K, N}}, M, N, K,                       \
-                    RowMajorOut<float, float>{out, nullptr, N, 0});                            \
-  }                                                                                            \
-  extern "C" __global__ void __launch_bounds__(kGemmThreads) mfma_conv2d_f32_t##BM(            \
-      const float* x, const float* weight, const float* bias, float* out, int N, int C, int H, \
-      int W, int OC, int KH, int KW, int OH, int OW, int SH, int SW, int PH, int PW, int relu) { \
-    const int K = C * KH * KW, pixels = N * OH * OW;                                           \
-    gemmF32<BM, BN>(RowsKT{{weight, OC, K, K}},                                                \
-                    ConvPatch{x, pixels, K, 0, C, H, W, KH, KW, OH, OW, SH, SW, PH, PW}, OC,   \
-                    pixels, K, ConvOut{out, bias, OC, static_cast<int64_t>(OH) * OW, relu});   \
-  }
-
-DK_MFMA_F32(64, 64)
-DK_MFMA_F32(128, 128)
-
-// Split-K conv2d for layers whose output tiles leave CUs with one workgroup: split z takes the
-// patch elements [z * k_per_split, ...) and writes its partial [OC][pixels] tile to part[z];
-// conv_splitk_reduce_f32 sums the splits in order, adds the bias, applies ReLU, writes NCHW.
-extern "C" __global__ void __launch_bounds__(kGemmThreads) mfma_conv2d_f32_splitk_t64(
-    const float* x, const float* weight, float* part, int N, int C, int H, int W, int OC, int KH,
-    int KW, int OH, int OW, int SH, int SW, int PH, int PW, int k_per_split) {
-  const int K = C * KH * KW, pixels = N * OH * OW;
-  const int kb = static_cast<int>(blockIdx.z) * k_per_split;
-  const int kl = K - kb < k_per_split ? K - kb : k_per_split;
-  gemmF32<64, 64>(RowsKT{{weight + kb, OC, kl, K}},
-                  ConvPatch{x, pixels, kl, kb, C, H, W, KH, KW, OH, OW, SH, SW, PH, PW}, OC,
-                  pixels, kl,
-                  RowMajorOut<float, float>{part + static_cast<int64_t>(blockIdx.z) * OC * pixels,
-                                            nullptr, pixels, 0});
-}
-
-extern "C" __global__ void __launch_bounds__(kGemmThreads)
-    conv_splitk_reduce_f32(const float* part, const float* bias, float* out, int64_t OC,
-                           int64_t pixels, int64_t OHW, int splits, int relu) {
-  const int64_t total = OC * pixels;
-  for (int64_t e = static_cast<int64_t>(blockIdx.x) * kGemmThreads + threadIdx.x; e < total;
-       e += static_cast<int64_t>(gridDim.x) * kGemmThreads) {
-    float v = gp(part)[e];
-    for (int z = 1; z < splits; ++z) v += gp(part)[z * total + e];
-    const int64_t oc = e / pixels, pixel = e - oc * pixels;
-    if (bias != nullptr) v += gp(bias)[oc];
-    if (relu) v = fmaxf(v, 0.f);
-    const int64_t n = pixel / OHW, q = pixel - n * OHW;
-    gp(out)[(n * OC + oc) * OHW + q] = v;
-  }
-}
-
-// Split-K fp32 linear for few output tiles and a long K (fully connected layers at small batch):
-// split z = blockIdx.z takes k in [z * k_per_split, (z + 1) * k_per_split) and writes its
-// partial tile to part[z][M][N]; splitk_reduce_f32 sums the splits in order (deterministic).
-extern "C" __global__ void __launch_bounds__(kGemmThreads)
-    mfma_linear_f32_splitk_t64(const float* x, const float* w, float* part, int64_t M, int64_t N,
-                               int64_t K, int64_t k_per_split) {
-  const int64_t kb = static_cast<int64_t>(blockIdx.z) * k_per_split;
-  const int64_t kl = K - kb < k_per_split ? K - kb : k_per_split;
-  gemmF32<64, 64>(RowsKT{{x + kb, M, kl, K}}, RowsKT{{w + kb, N, kl, K}}, M, N, kl,
-                  RowMajorOut<float, float>{part + blockIdx.z * M * N, nullptr, N, 0});
-}
-
-extern "C" __global__ void __launch_bounds__(kGemmThreads)
-    splitk_reduce_f32(const float* part, const float* bias, float* out, int64_t M, int64_t N,
-                      int splits, int relu) {
-  const int64_t total = M * N;
-  for (int64_t e = static_cast<int64_t>(blockIdx.x) * kGemmThreads + threadIdx.x; e < total;
-       e += static_cast<int64_t>(gridDim.x) * kGemmThreads) {
-    float v = gp(part)[e];
-    for (int z = 1; z < splits; ++z) v += gp(part)[z * total + e];
-    if (bias != nullptr) v += gp(bias)[e % N];
-    if (relu) v = fmaxf(v, 0.f);
-    gp(out)[e] = v;
-  }
-}
 
 // Two workgroups per CU (the LDS of two fits) and at most 256 VGPRs a lane: the compiler then
 // keeps the accumulators in VGPRs and gives the two register stages and both sub-slices'

@@ -1,0 +1,103 @@
+"""fp32 linear, matmul and conv2d over the edges of their forms (few rows, K groups, K parts, unaligned
+rows), against float64, and the operands that the three-term products hand to the fp32 instruction."""
+import json
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+pytestmark = pytest.mark.gpu
+
+
+def rand(shape, seed, scale=1.0):
+    return (torch.randn(shape, generator=torch.Generator().manual_seed(seed)) * scale).cuda()
+
+
+def run(op, inputs, attrs):
+    import dli
+
+    graph = dli.Graph.from_json(json.dumps({
+        "format": "dli.graph.v1", "model_type": op, "inputs": list(inputs), "outputs": ["out"],
+        "nodes": [{"name": "n", "op": op, "inputs": list(inputs), "outputs": ["out"],
+                   "attrs": attrs}]}))
+    return dli.Engine().load_plugin().run(graph, inputs)["out"]
+
+
+def close(out, ref, terms, k):
+    """Each product within 2^-22 of its value (what the split leaves out, the output's rounding) and
+    at most one rounding of the partial sums per product."""
+    assert ((out.double() - ref).abs() <= (k + 4) * 2.0 ** -23 * terms).all()
+    assert (out.double() - ref).norm() <= 1e-6 * terms.norm()
+
+
+def check_linear(x, w, b, relu=False):
+    out = run("linear", {"x": x, "w": w, "b": b}, {"activation": "relu"} if relu else {})
+    ref = x.double() @ w.double().t() + b.double()
+    terms = x.double().abs() @ w.double().abs().t() + b.double().abs()
+    close(out, ref.clamp_min(0) if relu else ref, terms, x.shape[1])
+
+
+@pytest.mark.parametrize("m,n,k", [
+    (1, 64, 4), (16, 65, 32), (16, 4096, 1024), (3, 10, 4096), (5, 896, 4864),  # 16-row tiles
+    (17, 63, 36), (64, 4096, 1024), (64, 10, 4096), (40, 130, 4100),  # one row tile
+    (65, 64, 64), (77, 128, 896), (256, 1024, 100), (200, 896, 2000),  # K groups, parts
+    (1000, 1100, 260), (513, 2050, 32),  # one group
+    (7, 9, 3), (70, 100, 33), (100, 70, 1001)])  # K % 4 != 0
+def test_linear_f32_forms(m, n, k):
+    x, w, b = rand((m, k), 1), rand((n, k), 2, 0.05), rand((n,), 3)
+    check_linear(x, w, b)
+    check_linear(x, w, b, relu=True)
+
+
+def test_linear_f32_unaligned_rows():
+    """A weight that does not start on 16 bytes takes the 4-byte loads."""
+    base = rand((100 * 64 + 1,), 4, 0.1)
+    w = base[1:].view(100, 64)
+    assert w.data_ptr() % 16 != 0
+    check_linear(rand((70, 64), 5), w, rand((100,), 6))
+
+
+@pytest.mark.parametrize("m", [4, 40, 100, 300])
+@pytest.mark.parametrize("scale", [2.0 ** 60, 2.0 ** -60])
+def test_linear_f32_magnitudes(m, scale):
+    x, w, b = rand((m, 256), 7) * scale, rand((80, 256), 8), rand((80,), 9) * scale
+    check_linear(x, w, b)
+
+
+@pytest.mark.parametrize("m", [4, 40, 100, 300])
+def test_linear_f32_infinities_and_nan(m):
+    """Infinite and NaN operands, and sums past the fp32 range, give what fp32 arithmetic gives; the
+    other rows keep their values."""
+    x, w, b = rand((m, 512), 10), rand((72, 512), 11).abs() + 0.5, rand((72,), 12)
+    clean = run("linear", {"x": x, "w": w, "b": b}, {})
+    x[0, 3] = float("inf")
+    x[1, 500] = float("nan")
+    x[2, :] = 3e38
+    x[3, 8], x[3, 9] = float("inf"), float("-inf")
+    out = run("linear", {"x": x, "w": w, "b": b}, {})
+    assert (out[0] == float("inf")).all() and (out[2] == float("inf")).all()
+    assert torch.isnan(out[1]).all() and torch.isnan(out[3]).all()
+    err = (out[4:] - clean[4:]).abs()
+    assert (err <= 512 * 2.0 ** -23 * (x[4:].abs() @ w.abs().t())).all()
+
+
+def test_matmul_f32_forms():
+    for m, n, k in ((5, 70, 64), (100, 65, 260), (600, 1100, 96), (33, 40, 7)):
+        a, b = rand((m, k), 13), rand((k, n), 14, 0.1)
+        close(run("matmul", {"a": a, "b": b}, {}), a.double() @ b.double(),
+              a.double().abs() @ b.double().abs(), k)
+
+
+@pytest.mark.parametrize("n,c,h,w,oc,kern,stride,pad", [
+    (1, 64, 16, 16, 192, 3, 1, 1), (3, 192, 8, 8, 384, 3, 1, 1),  # K groups and parts
+    (40, 64, 8, 8, 256, 3, 1, 1),  # parts of one group
+    (64, 16, 16, 16, 192, 3, 1, 1),  # one group, one part
+    (2, 5, 9, 7, 33, 3, 2, 1), (2, 7, 11, 11, 10, 5, 2, 2), (3, 12, 5, 5, 65, 1, 1, 0)])
+def test_conv2d_f32_forms(n, c, h, w, oc, kern, stride, pad):
+    x, k, b = rand((n, c, h, w), 15), rand((oc, c, kern, kern), 16, 0.1), rand((oc,), 17)
+    attrs = {"stride": [stride, stride], "padding": [pad, pad], "activation": "relu"}
+    out = run("conv2d", {"x": x, "w": k, "b": b}, attrs)
+    ref, terms = (F.conv2d(p.double().cpu(), q.double().cpu(), r.double().cpu(), stride=stride,
+                           padding=pad).cuda()
+                  for p, q, r in ((x, k, b), (x.abs(), k.abs(), b.abs())))
+    close(out, ref.clamp_min(0), terms, c * kern * kern)
