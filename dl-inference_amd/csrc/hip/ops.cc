@@ -93,6 +93,8 @@ DeviceKernel k_packed_paged128("packed_attention", "packed_attention_paged_d128"
 DeviceKernel k_packed_paged128_r128("packed_attention", "packed_attention_paged_d128_r128");
 DeviceKernel k_packed_dense128("packed_attention", "packed_attention_dense_d128");
 DeviceKernel k_packed_dense128_r128("packed_attention", "packed_attention_dense_d128_r128");
+DeviceKernel k_packed_f32_64("packed_attention", "packed_attention_f32_d64");
+DeviceKernel k_packed_f32_128("packed_attention", "packed_attention_f32_d128");
 DeviceKernel k_packed_merge64("packed_attention", "packed_attention_merge_d64");
 DeviceKernel k_packed_merge128("packed_attention", "packed_attention_merge_d128");
 DeviceKernel k_conv_small9("conv", "conv2d_small_f32_p9");
@@ -232,7 +234,7 @@ size_t packedPartialBytes(int64_t rows, int64_t head_dim, int64_t splits) {
 bool packedForm(int dtype, int64_t batch, int64_t q_heads, int64_t kv_heads, int64_t seq_q,
                 int64_t keys, const void* q, const void* k, const void* v, const void* out) {
   const int64_t limit = int64_t{1} << 30;
-  return dtype == DLI_BF16 && batch * kv_heads <= 65535 && keys > 0 && keys < limit &&
+  return (dtype == DLI_BF16 || dtype == DLI_F32) && batch * kv_heads <= 65535 && keys > 0 && keys < limit &&
          seq_q < limit && seq_q * (q_heads / kv_heads) < limit && aligned16(q) && aligned16(k) &&
          aligned16(v) && aligned16(out);
 }
@@ -741,13 +743,15 @@ static int attentionImpl(int dtype, const void* q, const void* k, const void* v,
   }
   // bf16 with head_dim 128: the packed-row MFMA kernel (fewer than 16 queries over long keys stay
   // on the row kernel, whose waves split the heads; the packed kernel has no key splits here)
-  if (!out_bshd && head_dim == 128 && seq_q >= 16 &&
+  // fp32 with head_dim 64 or 128: the same on the fp32 matrix instruction.
+  const bool f32 = dtype == DLI_F32;
+  if (!out_bshd && (head_dim == 128 || (f32 && head_dim == 64)) && seq_q >= 16 &&
       packedForm(dtype, batch, q_heads, kv_heads, seq_q, seq_k, q, k, v, out)) {
     dk::PackedAttentionArgs a{};
-    a.q = static_cast<const uint16_t*>(q);
-    a.k = static_cast<const uint16_t*>(k);
-    a.v = static_cast<const uint16_t*>(v);
-    a.out = static_cast<uint16_t*>(out);
+    a.q = q;
+    a.k = k;
+    a.v = v;
+    a.out = out;
     a.q_heads = static_cast<int32_t>(q_heads);
     a.kv_heads = static_cast<int32_t>(kv_heads);
     a.seq_q = static_cast<int32_t>(seq_q);
@@ -755,8 +759,11 @@ static int attentionImpl(int dtype, const void* q, const void* k, const void* v,
     a.causal = causal;
     a.splits = 1;
     a.scale_log2 = scale * 1.4426950408889634f;
-    const int64_t unit_rows = seq_q * (q_heads / kv_heads), tile = packedTile(unit_rows);
-    return launch(tile == 128 ? k_packed_dense128_r128 : k_packed_dense128,
+    const int64_t unit_rows = seq_q * (q_heads / kv_heads);
+    const int64_t tile = f32 ? 64 : packedTile(unit_rows);
+    DeviceKernel& kern = f32 ? (head_dim == 64 ? k_packed_f32_64 : k_packed_f32_128)
+                             : (tile == 128 ? k_packed_dense128_r128 : k_packed_dense128);
+    return launch(kern,
                   {blocksFor(unit_rows, tile), static_cast<unsigned>(batch * kv_heads)}, {256}, 0,
                   stream, a);
   }
@@ -850,8 +857,8 @@ static int pagedAttention(int dtype, const void* q, const void* key_pool, const 
   }
   const int pos64 = positions_dtype == DLI_I64 ? 1 : 0;
   // several queries per sequence: the packed-row MFMA kernels (64-key tiles inside cache blocks)
-  if (seq_q > 1 && (head_dim == 64 || head_dim == 128) && block_size % dk::kPackedTileK == 0 &&
-      block_size < (int64_t{1} << 30) && max_blocks < (int64_t{1} << 30) &&
+  if (dtype == DLI_BF16 && seq_q > 1 && (head_dim == 64 || head_dim == 128) &&
+      block_size % dk::kPackedTileK == 0 && block_size < (int64_t{1} << 30) && max_blocks < (int64_t{1} << 30) &&
       packedForm(dtype, batch, q_heads, kv_heads, seq_q, max_blocks * block_size, q, key_pool,
                  value_pool, out)) {
     const int64_t unit_rows = seq_q * (q_heads / kv_heads), tile = packedTile(unit_rows);
@@ -861,12 +868,12 @@ static int pagedAttention(int dtype, const void* q, const void* key_pool, const 
            (partials == nullptr || partial_bytes < packedPartialBytes(rows, head_dim, n)))
       --n;
     dk::PackedAttentionArgs a{};
-    a.q = static_cast<const uint16_t*>(q);
-    a.k = static_cast<const uint16_t*>(key_pool);
-    a.v = static_cast<const uint16_t*>(value_pool);
+    a.q = q;
+    a.k = key_pool;
+    a.v = value_pool;
     a.block_table = block_table;
     a.positions = positions;
-    a.out = static_cast<uint16_t*>(out);
+    a.out = out;
     a.part_o = static_cast<float*>(partials);
     a.part_ml = n > 1 ? a.part_o + rows * n * head_dim : nullptr;
     a.past = past;

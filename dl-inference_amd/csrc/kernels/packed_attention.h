@@ -9,12 +9,12 @@ namespace dk {
 constexpr int kPackedTileK = 64;  // keys per tile
 
 struct PackedAttentionArgs {
-  const uint16_t* q;  // [B, Hq, Sq, D]
-  const uint16_t* k;  // [B, Hkv, keys, D], or the key pool [block, Hkv, block_size, D]
-  const uint16_t* v;  // [B, Hkv, keys, D], or the value pool [block, Hkv, D, block_size]
+  const void* q;  // [B, Hq, Sq, D]
+  const void* k;  // [B, Hkv, keys, D], or the key pool [block, Hkv, block_size, D]
+  const void* v;  // [B, Hkv, keys, D], or the value pool [block, Hkv, D, block_size]
   const int32_t* block_table;  // paged: [B, max_blocks]
   const void* positions;       // paged: tokens cached before the queries, per sequence, or NULL
-  uint16_t* out;               // [B, Hq, Sq, D]
+  void* out;                   // [B, Hq, Sq, D]
   float* part_ml;              // splits > 1: [splits][B Hkv][rows] of (max, sum)
   float* part_o;               // splits > 1: [splits][B Hkv][rows][D]
   int64_t past;                // paged: tokens cached before the queries when positions is NULL

@@ -89,23 +89,23 @@ __device__ __forceinline__ int64_t partIndex(const PackedAttentionArgs& a, int u
   return (static_cast<int64_t>(blockIdx.z) * gridDim.y + unit) * rows + p;
 }
 
-template <int D>
-__device__ __forceinline__ uint16_t* outRow(const PackedAttentionArgs& a, int b, int kvh,
+template <int D, typename T>
+__device__ __forceinline__ T* outRow(const PackedAttentionArgs& a, int b, int kvh,
                                             int group, int p) {
   const int i = p / group, h = kvh * group + p - i * group;
-  return a.out + ((static_cast<int64_t>(b) * a.q_heads + h) * a.seq_q + i) * D;
+  return static_cast<T*>(a.out) + ((static_cast<int64_t>(b) * a.q_heads + h) * a.seq_q + i) * D;
 }
 
 // Row p over the keys [j0, j1) that it sees, by one wave without the matrix cores: lane j scores
 // a key, then owns the outputs lane + 64 u. Keys that the row does not see are never touched.
-template <int D, bool kPaged>
+template <int D, bool kPaged, typename T>
 __device__ __forceinline__ void rowByKeys(const PackedAttentionArgs& a, int unit, int rows, int p,
                                        int j0, int j1) {
   const int lane = threadIdx.x % kWave, group = a.q_heads / a.kv_heads;
   const int b = unit / a.kv_heads, kvh = unit % a.kv_heads, i = p / group;
   const int lim = visibleKeys<kPaged>(a, pastOf<kPaged>(a, b), i);
-  const uint16_t* q =
-      a.q + ((static_cast<int64_t>(b) * a.q_heads + kvh * group + p % group) * a.seq_q + i) * D;
+  const T* q = static_cast<const T*>(a.q) +
+               ((static_cast<int64_t>(b) * a.q_heads + kvh * group + p % group) * a.seq_q + i) * D;
   auto block = [&](int j) {  // first element of the key's (block, head), or of the (b, head)
     if constexpr (kPaged) {
       const int64_t blk = gp(a.block_table)[b * a.max_blocks + j / a.block_size];
@@ -121,9 +121,9 @@ __device__ __forceinline__ void rowByKeys(const PackedAttentionArgs& a, int unit
     const int j = j0 + lane;
     float s = -INFINITY;
     if (j < j1) {
-      const uint16_t* k = a.k + block(j) + static_cast<int64_t>(j % size) * D;
+      const T* k = static_cast<const T*>(a.k) + block(j) + static_cast<int64_t>(j % size) * D;
       float dot = 0.f;
-      for (int d = 0; d < D; ++d) dot = fmaf(bf16ToFloat(gp(q)[d]), bf16ToFloat(gp(k)[d]), dot);
+      for (int d = 0; d < D; ++d) dot = fmaf(ld(q + d), ld(k + d), dot);
       s = dot * a.scale_log2;
     }
     const float next = fmaxf(m, waveMax(s));
@@ -136,11 +136,11 @@ __device__ __forceinline__ void rowByKeys(const PackedAttentionArgs& a, int unit
     for (int u = 0; u < D / kWave; ++u) acc[u] *= alpha;
     for (int jj = j0; jj < j1 && jj < j0 + kWave; ++jj) {
       const float pj = __shfl(w, jj - j0, kWave);
-      const uint16_t* v = a.v + block(jj);
+      const T* v = static_cast<const T*>(a.v) + block(jj);
 #pragma unroll
       for (int u = 0; u < D / kWave; ++u) {
         const int64_t d = lane + u * kWave, at = jj % size;
-        acc[u] = fmaf(pj, bf16ToFloat(gp(v)[kPaged ? d * size + at : at * D + d]), acc[u]);
+        acc[u] = fmaf(pj, ld(v + (kPaged ? d * size + at : at * D + d)), acc[u]);
       }
     }
   }
@@ -155,9 +155,9 @@ __device__ __forceinline__ void rowByKeys(const PackedAttentionArgs& a, int unit
     return;
   }
   const float inv = lim > 0 ? 1.f / l : 0.f;
-  uint16_t* out = outRow<D>(a, b, kvh, group, p);
+  T* out = outRow<D, T>(a, b, kvh, group, p);
 #pragma unroll
-  for (int u = 0; u < D / kWave; ++u) gp(out)[lane + u * kWave] = floatToBf16(acc[u] * inv);
+  for (int u = 0; u < D / kWave; ++u) st(out + lane + u * kWave, acc[u] * inv);
 }
 
 template <int D, int QB, bool kPaged>
@@ -192,8 +192,8 @@ __device__ __forceinline__ void packedAttention(const PackedAttentionArgs& a) {
   for (int qb = 0; qb < QB; ++qb) {
     const int p = pw + qb * 16 + r < rows ? pw + qb * 16 + r : rows - 1;  // clamped: not stored
     const int i = p / group, h = kvh * group + p - i * group;
-    const uint16_t* qp =
-        a.q + ((static_cast<int64_t>(b) * a.q_heads + h) * a.seq_q + i) * D + g * 8;
+    const uint16_t* qp = static_cast<const uint16_t*>(a.q) +
+                         ((static_cast<int64_t>(b) * a.q_heads + h) * a.seq_q + i) * D + g * 8;
 #pragma unroll
     for (int c = 0; c < DK; ++c) qf[qb][c] = gload16(qp + c * 32);
     lim[qb] = visibleKeys<kPaged>(a, past, i);
@@ -218,8 +218,8 @@ __device__ __forceinline__ void packedAttention(const PackedAttentionArgs& a) {
       const int64_t blk = gp(a.block_table)[b * a.max_blocks + k0 / a.block_size];
       const int slot = k0 % a.block_size;
       const int64_t base = (blk * a.kv_heads + kvh) * a.block_size * D;
-      const uint16_t* kq = a.k + base + static_cast<int64_t>(slot) * D;
-      const uint16_t* vq = a.v + base + slot;
+      const uint16_t* kq = static_cast<const uint16_t*>(a.k) + base + static_cast<int64_t>(slot) * D;
+      const uint16_t* vq = static_cast<const uint16_t*>(a.v) + base + slot;
 #pragma unroll
       for (int i = 0; i < kPer; ++i) {
         const int c = t + i * kThreads;
@@ -227,8 +227,9 @@ __device__ __forceinline__ void packedAttention(const PackedAttentionArgs& a) {
         vr[i] = gload16(vq + static_cast<int64_t>(c / 8) * a.block_size + (c % 8) * 8);
       }
     } else {
-      const uint16_t* kq = a.k + dense_base + static_cast<int64_t>(k0) * D;
-      const uint16_t* vq = a.v + dense_base + static_cast<int64_t>(k0) * D;
+      const int64_t at = dense_base + static_cast<int64_t>(k0) * D;
+      const uint16_t* kq = static_cast<const uint16_t*>(a.k) + at;
+      const uint16_t* vq = static_cast<const uint16_t*>(a.v) + at;
 #pragma unroll
       for (int i = 0; i < kPer; ++i) {
         const int c = t + i * kThreads;
@@ -416,7 +417,7 @@ __device__ __forceinline__ void packedAttention(const PackedAttentionArgs& a) {
 
   if (special != 0) {  // uniform
     for (int q = wave; q < kTileQ && p0 + q < rows; q += kThreads / kWave)
-      rowByKeys<D, kPaged>(a, unit, rows, p0 + q, kt0 * kTileK, kt1 * kTileK);
+      rowByKeys<D, kPaged, bf16>(a, unit, rows, p0 + q, kt0 * kTileK, kt1 * kTileK);
     return;
   }
 #pragma unroll
@@ -436,7 +437,7 @@ __device__ __forceinline__ void packedAttention(const PackedAttentionArgs& a) {
     }
     // a row that sees no key gives zeros; one whose visible scores are all -inf gives NaN
     const float inv = lim[qb] > 0 ? 1.f / lsum[qb][0] : 0.f;
-    uint16_t* orow = outRow<D>(a, b, kvh, group, p) + g * 4;
+    uint16_t* orow = outRow<D, uint16_t>(a, b, kvh, group, p) + g * 4;
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) {
       const uint32_t lo = packBf16x2(o[qb][dt][0] * inv, o[qb][dt][1] * inv);
@@ -444,6 +445,155 @@ __device__ __forceinline__ void packedAttention(const PackedAttentionArgs& a) {
       *gp(reinterpret_cast<uint2*>(orow + dt * 16)) = uint2{lo, hi};
     }
   }
+}
+
+// ---- fp32, contiguous keys and values --------------------------------------------------------------
+// The same rows and tiles with v_mfma_f32_16x16x4_f32 (lane l = 16 g + r supplies A[r][g] and
+// B[g][r] and receives D[4 g + i][r]): scores S^T = K Q^T with lane group g on
+// the g-th quarter of d, one 16-row block per wave. A lane's scores, keys 4 g + i of each 16-key block, are the B operand of
+// O^T += V^T P^T as they stand (step i takes key 4 g + i from every group), so the probabilities
+// stay in fp32 registers; V keeps its [key][d] layout, 16 consecutive d per operand row. K and V rows
+// are D + 4 floats apart: the rows of a K fragment and the four keys of a V fragment start on
+// different banks. Bound by the fp32 matrix instruction (a sixteenth of the bf16 rate) and the
+// longest rows: 2 x 500 tokens, 14 / 2 heads, head_dim 64, causal 30 us, 150 with one wave per row and
+// a scalar dot.
+template <int D>
+__device__ __forceinline__ void packedAttentionF32(const PackedAttentionArgs& a) {
+  constexpr int kPitch = D + 4, kRowChunks = D / 4, kPer = kTileK * kRowChunks / kThreads;
+  constexpr int DT = D / 16, DC = D / 16;  // 16-wide d blocks of O; 4-float chunks per lane group
+  __shared__ __attribute__((aligned(16))) float Ks[kTileK * kPitch];
+  __shared__ __attribute__((aligned(16))) float Vs[kTileK * kPitch];
+  const int t = threadIdx.x, lane = t % kWave, wave = t / kWave;
+  const int r = lane % 16, g = lane / 16;
+  const int group = a.q_heads / a.kv_heads, rows = a.seq_q * group;
+  const uint32_t lin = blockIdx.x + gridDim.x * blockIdx.y;
+  const int unit = static_cast<int>(lin % gridDim.y);
+  const int b = unit / a.kv_heads, kvh = unit - b * a.kv_heads;
+  const int p0 = (gridDim.x - 1 - lin / gridDim.y) * 64, pw = p0 + wave * 16;
+  const bool active = pw < rows;  // uniform over the wave
+  auto query = [&](int p) { return (p < rows ? p : rows - 1) / group; };
+  const int pr = pw + r < rows ? pw + r : rows - 1;  // clamped: not stored
+  const int i0 = pr / group;
+  f32x4 qf[DC];  // d = g * (D / 4) + 4 c + j
+  {
+    const int h = kvh * group + pr - i0 * group;
+    const float* qp = static_cast<const float*>(a.q) +
+                      ((static_cast<int64_t>(b) * a.q_heads + h) * a.seq_q + i0) * D + g * (D / 4);
+#pragma unroll
+    for (int c = 0; c < DC; ++c) qf[c] = *gp(reinterpret_cast<const f32x4*>(qp + c * 4));
+  }
+  const int lim = visibleKeys<false>(a, 0, i0);
+  const int wg_keys = visibleKeys<false>(a, 0, query(p0 + 63));
+  const int wg_full = visibleKeys<false>(a, 0, query(p0));
+  const int wave_full = visibleKeys<false>(a, 0, query(pw));
+  const int tiles = (wg_keys + kTileK - 1) / kTileK;
+
+  const int64_t base = static_cast<int64_t>(unit) * a.keys * D;
+  f32x4 kr[kPer], vr[kPer];
+  auto fetch = [&](int kt) {
+    const int k0 = kt * kTileK;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      const int c = t + i * kThreads;
+      const int64_t at = base + static_cast<int64_t>(k0) * D + c * 4;
+      const bool in = k0 + c / kRowChunks < a.keys;
+      kr[i] = in ? *gp(reinterpret_cast<const f32x4*>(static_cast<const float*>(a.k) + at))
+                 : f32x4{0.f, 0.f, 0.f, 0.f};
+      vr[i] = in ? *gp(reinterpret_cast<const f32x4*>(static_cast<const float*>(a.v) + at))
+                 : f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+  };
+  f32x4 o[DT];  // O^T: d = 16 dt + 4 g + i, row pw + r
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m_run = -INFINITY, l_run = 0.f;
+  int special = 0;
+  if (tiles > 0) fetch(0);
+  for (int kt = 0; kt < tiles; ++kt) {
+    const int k0 = kt * kTileK;
+    __syncthreads();  // the previous tile is no longer read
+    bool bad = false;
+#pragma unroll
+    for (int i = 0; i < kPer; ++i) {
+      const int c = t + i * kThreads, at = (c / kRowChunks) * kPitch + (c % kRowChunks) * 4;
+      *reinterpret_cast<f32x4*>(&Ks[at]) = kr[i];
+      *reinterpret_cast<f32x4*>(&Vs[at]) = vr[i];
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        bad = bad || (__float_as_uint(vr[i][j]) & 0x7F800000u) == 0x7F800000u;
+    }
+    // infinite or NaN values in a tile that some row sees in part: as in packedAttention
+    if (k0 + kTileK > wg_full)  // uniform
+      special |= __syncthreads_or(bad);
+    else
+      __syncthreads();
+    if (kt + 1 < tiles) fetch(kt + 1);
+    if (!active) continue;
+    f32x4 s[4];
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) {
+      s[kk] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int c = 0; c < DC; ++c) {
+        const f32x4 kf =
+            *reinterpret_cast<const f32x4*>(&Ks[(kk * 16 + r) * kPitch + g * (D / 4) + c * 4]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          s[kk] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[j], qf[c][j], s[kk], 0, 0, 0);
+      }
+    }
+    if (k0 + kTileK > wave_full) {  // uniform over the wave
+      const int key0 = k0 + g * 4;
+#pragma unroll
+      for (int kk = 0; kk < 4; ++kk)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          s[kk][i] = key0 + kk * 16 + i < lim ? s[kk][i] : -INFINITY;
+    }
+    float tmax = -INFINITY;
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) tmax = fmaxf(tmax, s[kk][i]);
+    const float tm = rowsMax(tmax) * a.scale_log2;
+    const bool grow = tm > m_run + kRescaleLog2;  // false while tm = -inf
+    if (__builtin_amdgcn_ballot_w64(grow)) {
+      const float alpha = grow ? __builtin_amdgcn_exp2f(m_run - tm) : 1.f;  // 0 from -inf
+      m_run = grow ? tm : m_run;
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) o[dt] *= alpha;
+      l_run *= alpha;
+    }
+    const float ref = m_run == -INFINITY ? 0.f : m_run;
+    float sum = 0.f;
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        s[kk][i] = __builtin_amdgcn_exp2f(fmaf(s[kk][i], a.scale_log2, -ref));
+        sum += s[kk][i];
+      }
+    l_run += sum;  // this lane group's keys; the groups are added at the end
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt)
+          o[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+              Vs[(kk * 16 + g * 4 + i) * kPitch + dt * 16 + r], s[kk][i], o[dt], 0, 0, 0);
+  }
+  if (special != 0) {  // uniform
+    for (int q = wave; q < 64 && p0 + q < rows; q += kThreads / kWave)
+      rowByKeys<D, false, float>(a, unit, rows, p0 + q, 0, tiles * kTileK);
+    return;
+  }
+  const float l = rowsSum(l_run);
+  if (pw + r >= rows) return;
+  const float inv = lim > 0 ? 1.f / l : 0.f;
+  float* orow = outRow<D, float>(a, b, kvh, group, pw + r) + g * 4;
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt) *gp(reinterpret_cast<f32x4*>(orow + dt * 16)) = o[dt] * inv;
 }
 
 // Combines the key splits: D / 4 lanes per row, 16 bytes of every split's sums each.
@@ -469,7 +619,7 @@ __device__ __forceinline__ void packedMerge(const PackedAttentionArgs& a, int un
   const int unit = static_cast<int>(row / rows), p = static_cast<int>(row % rows);
   const int b = unit / a.kv_heads, kvh = unit % a.kv_heads;
   const float inv = visibleKeys<kPaged>(a, pastOf<kPaged>(a, b), p / group) > 0 ? 1.f / l : 0.f;
-  *gp(reinterpret_cast<uint2*>(outRow<D>(a, b, kvh, group, p) + d)) =
+  *gp(reinterpret_cast<uint2*>(outRow<D, uint16_t>(a, b, kvh, group, p) + d)) =
       uint2{packBf16x2(acc[0] * inv, acc[1] * inv), packBf16x2(acc[2] * inv, acc[3] * inv)};
 }
 
@@ -488,6 +638,16 @@ DK_PACKED(packed_attention_paged_d128, 128, 1, true)
 DK_PACKED(packed_attention_paged_d128_r128, 128, 2, true)
 DK_PACKED(packed_attention_dense_d128, 128, 1, false)
 DK_PACKED(packed_attention_dense_d128_r128, 128, 2, false)
+
+// Grid {ceil(rows / 64), B Hkv}.
+extern "C" __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2)))
+    packed_attention_f32_d64(PackedAttentionArgs a) {
+  packedAttentionF32<64>(a);
+}
+extern "C" __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2)))
+    packed_attention_f32_d128(PackedAttentionArgs a) {
+  packedAttentionF32<128>(a);
+}
 
 // Grid {ceil(B Hq Sq / (1024 / D))}; units = B Hkv.
 extern "C" __global__ void __launch_bounds__(kThreads)

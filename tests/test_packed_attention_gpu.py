@@ -119,3 +119,37 @@ def test_dense_head_dim_128(sq, sk, hq, hkv, causal):
         assert (out[:, :, :sq - sk] == 0).all()
         out, q = out[:, :, sq - sk:], q[:, :, sq - sk:]
     check(out, ops.attention(to_np(q), to_np(k), to_np(v), causal=causal))
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("sq,sk,hq,hkv,causal", [(16, 16, 4, 4, True), (18, 100, 28, 4, True),
+                                                 (77, 77, 7, 1, True), (40, 130, 6, 2, False),
+                                                 (130, 65, 2, 2, True)])
+def test_dense_f32(d, sq, sk, hq, hkv, causal):
+    """fp32 throughout: the scores' and sums' roundings, about sqrt(d) and sqrt(keys) ulps."""
+    import dli
+
+    g = torch.Generator().manual_seed(21)
+    q, k, v = (torch.randn(2, h, s, d, generator=g).to(DEV)
+               for h, s in ((hq, sq), (hkv, sk), (hkv, sk)))
+    out = run_attention({"q": q, "k": k, "v": v}, {"causal": causal}, dli.Engine().load_plugin())
+    if causal and sq > sk:  # queries before the first key: zeros
+        assert (out[:, :, :sq - sk] == 0).all()
+        out, q = out[:, :, sq - sk:], q[:, :, sq - sk:]
+    ref = ops.attention(to_np(q), to_np(k), to_np(v), causal=causal)
+    assert np.linalg.norm(to_np(out) - ref) <= 1e-6 * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("d", [64, 128])
+def test_dense_f32_never_reads_hidden_values(d):
+    import dli
+
+    g = torch.Generator().manual_seed(22)
+    q, k, v = (torch.randn(1, h, 50, d, generator=g).to(DEV) for h in (4, 2, 2))
+    engine = dli.Engine().load_plugin()
+    clean = run_attention({"q": q, "k": k, "v": v}, {"causal": True}, engine)
+    v[:, :, -1, ::2], v[:, :, -1, 1::2] = float("inf"), float("nan")
+    out = run_attention({"q": q, "k": k, "v": v}, {"causal": True}, engine)
+    err = (out[:, :, :-1] - clean[:, :, :-1]).norm()
+    assert err <= 1e-6 * clean[:, :, :-1].norm()
+    assert torch.isinf(out[:, :, -1, ::2]).all() and torch.isnan(out[:, :, -1, 1::2]).all()
