@@ -48,6 +48,70 @@ __device__ void relu_impl(const void* x, void* out, int64_t total) {
   DK_GRID_STRIDE(i, total) { st(po + i, fmaxf(ld(px + i), 0.0f)); }
 }
 
+// ---- 16-byte forms ---------------------------------------------------------------------------------
+// The same arithmetic per element on 16-byte chunks (aligned tensors, a whole number of chunks): the
+// element forms above issue a 2-byte load per element and a 64-bit modulo per broadcast index, and
+// reached 2.7 TB/s (silu of 38 M bf16 57 us, mul 62 us) where a copy from memory reaches 4.8; these take
+// 27 and 35 us.
+template <typename T>
+struct Chunk16 {
+  static constexpr int kN = 16 / sizeof(T);
+  typedef uint32_t Raw __attribute__((ext_vector_type(4)));
+  T e[kN];
+  static __device__ __forceinline__ Chunk16 load(const T* p) {
+    return __builtin_bit_cast(Chunk16, *gp(reinterpret_cast<const Raw*>(p)));
+  }
+  __device__ __forceinline__ void store(T* p) const {
+    *gp(reinterpret_cast<Raw*>(p)) = __builtin_bit_cast(Raw, *this);
+  }
+};
+
+template <typename T, class Op>
+__device__ __forceinline__ void unary16(const void* x, void* out, int64_t chunks, Op op) {
+  using C = Chunk16<T>;
+  DK_GRID_STRIDE(i, chunks) {
+    C v = C::load(static_cast<const T*>(x) + i * C::kN);
+#pragma unroll
+    for (int k = 0; k < C::kN; ++k) st(&v.e[k], op(ld(&v.e[k])));
+    v.store(static_cast<T*>(out) + i * C::kN);
+  }
+}
+
+// b repeats every b_chunks chunks (below 2^32 chunks in all; b_chunks = chunks: no repeat)
+template <typename T, class Op>
+__device__ __forceinline__ void binary16(const void* a, const void* b, void* out, int64_t chunks,
+                                         int64_t b_chunks, Op op) {
+  using C = Chunk16<T>;
+  const bool same = b_chunks == chunks;
+  DK_GRID_STRIDE(i, chunks) {
+    const int64_t j = same ? i : static_cast<uint32_t>(i) % static_cast<uint32_t>(b_chunks);
+    C v = C::load(static_cast<const T*>(a) + i * C::kN);
+    const C w = C::load(static_cast<const T*>(b) + j * C::kN);
+#pragma unroll
+    for (int k = 0; k < C::kN; ++k) st(&v.e[k], op(ld(&v.e[k]), ld(&w.e[k])));
+    v.store(static_cast<T*>(out) + i * C::kN);
+  }
+}
+
+template <typename T>
+__device__ void add16_impl(const void* a, const void* b, void* out, int64_t chunks,
+                           int64_t b_chunks) {
+  binary16<T>(a, b, out, chunks, b_chunks, [](float x, float y) { return x + y; });
+}
+template <typename T>
+__device__ void mul16_impl(const void* a, const void* b, void* out, int64_t chunks,
+                           int64_t b_chunks) {
+  binary16<T>(a, b, out, chunks, b_chunks, [](float x, float y) { return x * y; });
+}
+template <typename T>
+__device__ void silu16_impl(const void* x, void* out, int64_t chunks) {
+  unary16<T>(x, out, chunks, [](float v) { return v / (1.0f + __expf(-v)); });
+}
+template <typename T>
+__device__ void relu16_impl(const void* x, void* out, int64_t chunks) {
+  unary16<T>(x, out, chunks, [](float v) { return fmaxf(v, 0.0f); });
+}
+
 // batch_norm2d/kernel.py:6-28 — (x - mean) * rsqrt(var + eps) * w + b, channel = (i / spatial) % C
 template <typename T>
 __device__ void batch_norm2d_impl(const void* x, const void* w, const void* b, const void* mean,
@@ -195,6 +259,51 @@ __device__ void rotate_tensor(const T* x, T* out, int64_t vectors, int64_t heads
   }
 }
 
+// Whole rows (2 pairs = head_dim) in 16-byte chunks, q's chunks and then k's in one index range of 32
+// bits: the same arithmetic, table rows read as vectors.
+template <typename T>
+__device__ void rotary16_impl(const void* q, const void* k, const float* cosT, const float* sinT,
+                              void* out_q, void* out_k, int64_t batch, int64_t q_heads,
+                              int64_t k_heads, int64_t seq, int64_t head_dim, int64_t max_pos,
+                              int64_t start_pos, const void* positions, int pos64) {
+  using C = Chunk16<T>;
+  constexpr int kPairs = C::kN / 2;
+  const uint32_t row = static_cast<uint32_t>(head_dim) / C::kN, s = static_cast<uint32_t>(seq);
+  const uint32_t q_chunks = static_cast<uint32_t>(batch * q_heads) * s * row;
+  const uint32_t chunks = q_chunks + static_cast<uint32_t>(batch * k_heads) * s * row;
+  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < chunks;
+       i += gridDim.x * blockDim.x) {
+    const bool is_q = i < q_chunks;
+    const uint32_t at = is_q ? i : i - q_chunks;
+    const uint32_t heads = static_cast<uint32_t>(is_q ? q_heads : k_heads);
+    const uint32_t vec = at / row, part = at - vec * row;  // vec = (b * heads + h) * seq + t
+    const uint32_t bh = vec / s;
+    int64_t pos = start_pos + (vec - bh * s);
+    if (positions != nullptr) pos += loadIndex(positions, pos64, bh / heads);
+    const T* const px = static_cast<const T*>(is_q ? q : k) + static_cast<int64_t>(at) * C::kN;
+    T* const po = static_cast<T*>(is_q ? out_q : out_k) + static_cast<int64_t>(at) * C::kN;
+    C v = C::load(px);
+    if (pos >= 0 && pos < max_pos) {
+      const int64_t t = pos * (head_dim / 2) + part * kPairs;
+      float cs[kPairs], sn[kPairs];
+#pragma unroll
+      for (int p = 0; p < kPairs; p += 2) {
+        typedef float f32x2 __attribute__((ext_vector_type(2)));
+        const f32x2 c2 = *gp(reinterpret_cast<const f32x2*>(cosT + t + p));
+        const f32x2 s2 = *gp(reinterpret_cast<const f32x2*>(sinT + t + p));
+        cs[p] = c2.x, cs[p + 1] = c2.y, sn[p] = s2.x, sn[p + 1] = s2.y;
+      }
+#pragma unroll
+      for (int p = 0; p < kPairs; ++p) {
+        const float x0 = ld(&v.e[2 * p]), x1 = ld(&v.e[2 * p + 1]);
+        st(&v.e[2 * p], x0 * cs[p] - x1 * sn[p]);
+        st(&v.e[2 * p + 1], x0 * sn[p] + x1 * cs[p]);
+      }
+    }
+    v.store(po);
+  }
+}
+
 template <typename T>
 __device__ void rotary_impl(const void* q, const void* k, const float* cosT, const float* sinT,
                             void* out_q, void* out_k, int64_t batch, int64_t q_heads,
@@ -273,6 +382,21 @@ DK_FLOAT_KERNELS(mul, 256, (const void* a, const void* b, void* out, int64_t tot
                  (a, b, out, total, width))
 DK_FLOAT_KERNELS(silu, 256, (const void* x, void* out, int64_t total), (x, out, total))
 DK_FLOAT_KERNELS(relu, 256, (const void* x, void* out, int64_t total), (x, out, total))
+DK_FLOAT_KERNELS(add16, 256,
+                 (const void* a, const void* b, void* out, int64_t chunks, int64_t b_chunks),
+                 (a, b, out, chunks, b_chunks))
+DK_FLOAT_KERNELS(mul16, 256,
+                 (const void* a, const void* b, void* out, int64_t chunks, int64_t b_chunks),
+                 (a, b, out, chunks, b_chunks))
+DK_FLOAT_KERNELS(silu16, 256, (const void* x, void* out, int64_t chunks), (x, out, chunks))
+DK_FLOAT_KERNELS(relu16, 256, (const void* x, void* out, int64_t chunks), (x, out, chunks))
+DK_FLOAT_KERNELS(rotary16, 256,
+                 (const void* q, const void* k, const float* cosT, const float* sinT, void* out_q,
+                  void* out_k, int64_t batch, int64_t q_heads, int64_t k_heads, int64_t seq,
+                  int64_t head_dim, int64_t max_pos, int64_t start_pos, const void* positions,
+                  int pos64),
+                 (q, k, cosT, sinT, out_q, out_k, batch, q_heads, k_heads, seq, head_dim, max_pos,
+                  start_pos, positions, pos64))
 DK_FLOAT_KERNELS(batch_norm2d, 256,
                  (const void* x, const void* w, const void* b, const void* mean, const void* var,
                   void* out, int64_t total, int64_t channels, int64_t spatial, float eps),

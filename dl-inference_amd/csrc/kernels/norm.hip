@@ -48,14 +48,14 @@ __device__ void rms_norm_impl(const void* x, const void* weight, void* out, int6
   }
 }
 
-// bf16 rows with hidden % 8 == 0 and hidden <= 64 * 8 * kRowChunks (4096), 16-byte aligned: one wave
+// bf16 rows with hidden % 8 == 0 and hidden <= 4096, 16-byte aligned: one wave
 // per row (4 rows per 256-thread block, grid-stride over rows), the row held in registers as
 // 16-byte chunks (chunk c of the row in lane c % 64), sum of squares reduced inside the wave
 // (no LDS, no barrier), 16-byte loads and stores. Per element the same arithmetic as the
 // block-per-row kernel: x * inv * w with inv = 1 / sqrt(mean(x^2) + eps), rounded once.
-constexpr int kRowChunks = 8;
-
-__device__ void rms_norm_rows_bf16(const uint16_t* x, const uint16_t* weight, uint16_t* out,
+// kRowChunks: chunks per lane, 2 (hidden <= 1024, fewer registers and so more rows in flight) or 8.
+template <int kRowChunks>
+__device__ __forceinline__ void rms_norm_rows_bf16(const uint16_t* x, const uint16_t* weight, uint16_t* out,
                                    int64_t rows, int hidden, float eps) {
   const int lane = threadIdx.x % kWave;
   const int chunks = hidden / 8;
@@ -64,15 +64,21 @@ __device__ void rms_norm_rows_bf16(const uint16_t* x, const uint16_t* weight, ui
     const uint16_t* row = x + r * hidden;
     uint32_t v[kRowChunks][4];
     float sq = 0.f;
+    // every chunk is requested before the first is used (a branch around each load made a row a
+    // chain of up to 8 round trips: 34 rows of 3584 7.3 us, 4.2 now); past the row: its last chunk
 #pragma unroll
     for (int c = 0; c < kRowChunks; ++c) {
+      if (c * kWave >= chunks) break;  // uniform
       const int i = lane + c * kWave;
-      if (i < chunks) {
-        const uint4 w = *gp(reinterpret_cast<const uint4*>(row + i * 8));
-        v[c][0] = w.x;
-        v[c][1] = w.y;
-        v[c][2] = w.z;
-        v[c][3] = w.w;
+      const uint4 w = *gp(reinterpret_cast<const uint4*>(row + (i < chunks ? i : chunks - 1) * 8));
+      v[c][0] = w.x;
+      v[c][1] = w.y;
+      v[c][2] = w.z;
+      v[c][3] = w.w;
+    }
+#pragma unroll
+    for (int c = 0; c < kRowChunks; ++c) {
+      if (lane + c * kWave < chunks) {
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
           const float lo = __uint_as_float(v[c][k] << 16), hi = __uint_as_float(v[c][k] & 0xFFFF0000u);
@@ -106,7 +112,12 @@ __device__ void rms_norm_rows_bf16(const uint16_t* x, const uint16_t* weight, ui
 extern "C" __global__ void __launch_bounds__(256)
     rms_norm_rows_bf16_k(const uint16_t* x, const uint16_t* weight, uint16_t* out, int64_t rows,
                          int hidden, float eps) {
-  rms_norm_rows_bf16(x, weight, out, rows, hidden, eps);
+  rms_norm_rows_bf16<2>(x, weight, out, rows, hidden, eps);
+}
+extern "C" __global__ void __launch_bounds__(256)
+    rms_norm_wide_rows_bf16_k(const uint16_t* x, const uint16_t* weight, uint16_t* out,
+                              int64_t rows, int hidden, float eps) {
+  rms_norm_rows_bf16<8>(x, weight, out, rows, hidden, eps);
 }
 
 DK_FLOAT_KERNELS(rms_norm, 256,
