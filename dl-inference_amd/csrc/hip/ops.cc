@@ -187,6 +187,15 @@ PlanF32 planF32(int64_t rows, int64_t cols, int64_t k, bool vec, bool linear, in
   }
   return p;
 }
+// A conv on the 16-byte / buffer forms: whole 4-wide chunks of weight rows, a window of less than 32
+// positions (bits of a mask), and the images under a tile's 64 pixels within a buffer's 4 GB.
+bool convVec(int64_t n, int64_t c, int64_t h, int64_t w, int64_t patch, int64_t window,
+             int64_t out_pixels) {
+  int64_t images = 63 / out_pixels + 2;
+  if (images > n) images = n;
+  return patch % 4 == 0 && window < 32 && images * c * h * w < (int64_t{1} << 30);
+}
+
 // parts that a workspace holds
 int64_t partsHeldF32(const void* workspace, size_t bytes, int64_t rows, int64_t cols) {
   const auto held = static_cast<int64_t>(bytes / sizeof(float)) / (rows * cols);
@@ -554,7 +563,9 @@ size_t dli_hip_conv2d_workspace(int dtype, int64_t n, int64_t in_c, int64_t out_
       out_h <= 0 || out_w <= 0)
     return 0;
   const int64_t pixels = n * out_h * out_w, patch = in_c * kernel_h * kernel_w;
-  return partBytesF32(planF32(out_c, pixels, patch, patch % 4 == 0, false, kMaxPartsF32), out_c, pixels);
+  // (the image size is not known here; what it decides is met by images of gigabytes only)
+  const bool vec = patch % 4 == 0 && kernel_h * kernel_w < 32;
+  return partBytesF32(planF32(out_c, pixels, patch, vec, false, kMaxPartsF32), out_c, pixels);
 }
 
 int dli_hip_conv2d_act(int dtype, const void* x, const void* weight, const void* bias, void* out,
@@ -599,7 +610,8 @@ int dli_hip_conv2d_act(int dtype, const void* x, const void* weight, const void*
                     i32(out_c), i32(out_h), i32(out_w), i32(stride_h), i32(stride_w), i32(pad_h),
                     i32(pad_w), relu, tab);
     }
-    const bool vec = patch % 4 == 0 && aligned16(weight);
+    const bool vec = convVec(n, in_c, h, w, patch, kernel_h * kernel_w, out_h * out_w) &&
+                     aligned16(weight);
     const PlanF32 p = planF32(out_c, pixels, patch, vec, false,
                               partsHeldF32(workspace, workspace_bytes, out_c, pixels));
     if ((out_c + 63) / 64 <= kMaxGridY) {

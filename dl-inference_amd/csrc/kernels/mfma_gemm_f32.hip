@@ -23,7 +23,8 @@
 // pixels x 1728 159 / 68 + 5; distance from float64 there 7.1e-7 / 2.5e-7 (K = 4864).
 //
 //  _m16: 16 rows of A against 64 of B (a decode-sized x); _stream: nontemporal weight loads.
-//  _scalar: rows that are not 16-byte aligned or K % 4 != 0 (4-byte loads).
+//  _scalar: rows that are not 16-byte aligned or K % 4 != 0 (4-byte loads); convs of windows or images
+//        that the gather through a buffer does not hold.
 #include <type_traits>
 
 #include "common.h"
@@ -119,16 +120,22 @@ struct KRows : AlongRows<ROWS> {
 };
 
 // Input patch of a zero-padded NCHW conv: row = output pixel (n, oy, ox), k = (c, ky, kx) over
-// k_base + [0, K). prepare() tabulates (c * H * W + ky * W + kx, ky, kx) for the k of a slice, and
-// an element is a table read, two bounds checks and one gather. 32-bit index math (the host checks
-// that every index fits).
-template <int ROWS>
+// k_base + [0, K). prepare() tabulates the k of a slice, and an element is a table read and one gather.
+// 32-bit index math (the host checks that every index fits).
+// kBuffer (KH * KW < 32, the images of a tile below 4 GB): the table holds (byte offset, ky * KW + kx)
+// and the pixel a mask of the window positions outside the image; an element is one bit extract, an
+// or that sends what is masked out of the buffer's range (which reads as 0) and a buffer load, 4
+// vector instructions. Without it two range checks, two selects and 64-bit addresses, about 13: the
+// convolutions are bound by vector instructions (57% of the CU cycles with these).
+template <int ROWS, bool kBuffer>
 struct ConvPatch : AlongRows<ROWS> {
   static constexpr bool kTable = true;
   const float* x;
   int rows, K, k_base, C, H, W, KH, KW, OH, OW, SH, SW, PH, PW;
   int iy0, ix0, base, t;
+  unsigned outside;  // kBuffer: bit ky * KW + kx: that position lies outside; bit 31: past K
   bool valid;
+  __amdgpu_buffer_rsrc_t images;
   __device__ __forceinline__ ConvPatch(const float* x, int rows, int K, int k_base, int C, int H,
                                        int W, int KH, int KW, int OH, int OW, int SH, int SW,
                                        int PH, int PW)
@@ -139,10 +146,30 @@ struct ConvPatch : AlongRows<ROWS> {
     const int pixel = static_cast<int>(r0) + t % ROWS;
     valid = pixel < rows;
     const int ox = pixel % OW, q = pixel / OW;
-    const int oy = q % OH, n = q / OH;
+    const int oy = q % OH;
+    int n = q / OH;
     iy0 = oy * SH - PH;
     ix0 = ox * SW - PW;
-    base = n * C * H * W + iy0 * W + ix0;
+    if constexpr (kBuffer) {
+      // offsets from the tile's first image
+      const int n0 = static_cast<int>(r0) / (OH * OW), last = (rows - 1) / (OH * OW);
+      const int64_t chw = static_cast<int64_t>(C) * H * W;
+      const int64_t bytes = (last + 1 - n0) * chw * 4;
+      n -= n0;
+      images = __builtin_amdgcn_make_buffer_rsrc(
+          const_cast<float*>(x + n0 * chw), 0,
+          static_cast<int>(bytes < 0xFFFFFFFFll ? bytes : 0xFFFFFFFFll), 0x00027000);
+      outside = 0x80000000u;
+      for (int ky = 0, bit = 0; ky < KH; ++ky)
+        for (int kx = 0; kx < KW; ++kx, ++bit) {
+          const bool in = valid && static_cast<unsigned>(iy0 + ky) < static_cast<unsigned>(H) &&
+                          static_cast<unsigned>(ix0 + kx) < static_cast<unsigned>(W);
+          outside |= (in ? 0u : 1u) << bit;
+        }
+      base = static_cast<int>(static_cast<unsigned>(n * C * H * W + iy0 * W + ix0) * 4u);
+    } else {
+      base = n * C * H * W + iy0 * W + ix0;
+    }
   }
   __device__ __forceinline__ void prepare(int64_t k0, int t, int2* tab) const {
     const int k = static_cast<int>(k0) + t;
@@ -150,7 +177,11 @@ struct ConvPatch : AlongRows<ROWS> {
       const int kk = k_base + k, khw = KH * KW;
       const int c = kk / khw, rem = kk - c * khw;
       const int ky = rem / KW, kx = rem - ky * KW;
-      tab[t] = int2{k < K ? (c * H + ky) * W + kx : -1, (ky << 16) | kx};
+      const int at = (c * H + ky) * W + kx;
+      if constexpr (kBuffer)
+        tab[t] = k < K ? int2{static_cast<int>(static_cast<unsigned>(at) * 4u), rem} : int2{0, 31};
+      else
+        tab[t] = int2{k < K ? at : -1, (ky << 16) | kx};
     }
   }
   template <bool kWhole>
@@ -160,11 +191,18 @@ struct ConvPatch : AlongRows<ROWS> {
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const int2 e = tab[c0 + j];
-      const unsigned iy = iy0 + (static_cast<unsigned>(e.y) >> 16), ix = ix0 + (e.y & 0xFFFF);
-      const bool in = valid && e.x >= 0 && iy < static_cast<unsigned>(H) &&
-                      ix < static_cast<unsigned>(W);
-      const float g = gp(x)[in ? base + e.x : 0];
-      v[j] = in ? g : 0.f;
+      if constexpr (kBuffer) {
+        const int out = __builtin_amdgcn_sbfe(static_cast<int>(outside), e.y, 1);  // -1: masked
+        const int off = static_cast<int>(static_cast<unsigned>(base) + static_cast<unsigned>(e.x));
+        v[j] = __uint_as_float(
+            __builtin_amdgcn_raw_buffer_load_b32(images, off | out, 0, 0));
+      } else {
+        const unsigned iy = iy0 + (static_cast<unsigned>(e.y) >> 16), ix = ix0 + (e.y & 0xFFFF);
+        const bool in = valid && e.x >= 0 && iy < static_cast<unsigned>(H) &&
+                        ix < static_cast<unsigned>(W);
+        const float g = gp(x)[in ? base + e.x : 0];
+        v[j] = in ? g : 0.f;
+      }
     }
     return v;
   }
@@ -524,7 +562,7 @@ DK_MATMUL(mfma_matmul_f32_scalar, 1, false)
     const int pixels = N * OH * OW;                                                             \
     DK_PART(K)                                                                                  \
     const RowsK<64, VEC, false> A{weight + kb, OC, kl, K};                                      \
-    const ConvPatch<64> B(x, pixels, static_cast<int>(kl), static_cast<int>(kb), C, H, W, KH,   \
+    const ConvPatch<64, VEC> B(x, pixels, static_cast<int>(kl), static_cast<int>(kb), C, H, W, KH,   \
                           KW, OH, OW, SH, SW, PH, PW);                                          \
     const RowMajorOut parts{part + static_cast<int64_t>(blockIdx.z) * OC * pixels, nullptr,     \
                             pixels, 0};                                                         \

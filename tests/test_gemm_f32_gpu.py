@@ -92,7 +92,8 @@ def test_matmul_f32_forms():
     (1, 64, 16, 16, 192, 3, 1, 1), (3, 192, 8, 8, 384, 3, 1, 1),  # K groups and parts
     (40, 64, 8, 8, 256, 3, 1, 1),  # parts of one group
     (64, 16, 16, 16, 192, 3, 1, 1),  # one group, one part
-    (2, 5, 9, 7, 33, 3, 2, 1), (2, 7, 11, 11, 10, 5, 2, 2), (3, 12, 5, 5, 65, 1, 1, 0)])
+    (2, 5, 9, 7, 33, 3, 2, 1), (2, 7, 11, 11, 10, 5, 2, 2), (3, 12, 5, 5, 65, 1, 1, 0),
+    (70, 4, 3, 3, 20, 3, 1, 0), (2, 4, 12, 12, 20, 7, 1, 3), (5, 8, 6, 6, 70, 5, 1, 2)])
 def test_conv2d_f32_forms(n, c, h, w, oc, kern, stride, pad):
     x, k, b = rand((n, c, h, w), 15), rand((oc, c, kern, kern), 16, 0.1), rand((oc,), 17)
     attrs = {"stride": [stride, stride], "padding": [pad, pad], "activation": "relu"}
