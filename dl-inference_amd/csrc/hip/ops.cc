@@ -154,7 +154,8 @@ struct PlanF32 {
 // instructions; where the tiles alone are fewer, K parts make up for it, or, where the parts' traffic
 // would cost more, a second K group in the workgroup. In us: conv 384 x 4096 pixels x 1728 (384
 // tiles) 104 in one part, 68 + 5 for the sum in two; 256 x 4096 x 3456 (256 tiles) 108 with two
-// groups, 87 + 5 in three parts of one; linear 1000 x 896 x 4864 (224 tiles) 65 with two groups, 68
+// groups, 87 + 5 in three parts of one (these with gathers that branch; as they run now 55 + 6 and
+// 68 + 5); linear 1000 x 896 x 4864 (224 tiles) 65 with two groups, 68
 // to 72 in parts; 1000 x 896 x 896 17 with two groups, 21 with one, 23 in two parts; a conv of 3
 // images (24 tiles) 12 + 4 with two groups and 11 to 16 parts, 14 + 4 with one.
 constexpr int64_t kMaxPartsF32 = 16;

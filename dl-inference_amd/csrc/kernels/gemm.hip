@@ -3,8 +3,9 @@
 //  gemm_tiled_<t>   any dtype/shape: 64x64 output tile per 256-thread block, k in steps of 16
 //                   through LDS, 4x4 outputs per thread, fp32 accumulation.
 //                   linear/kernel.py:6-44 (w is [n, k]) and matmul/kernel.py:6-40 (b is [k, n]).
-//  skinny_linear_<MB>  bf16 weight streaming for m <= 16 * MB rows (decode): MFMA core from
-//                   skinny.h, bias epilogue, bf16 or fp32 output.
+//  skinny_linear_<t>_m<MB>, skinny_linear_<t>_w16_m<MB>  bf16 / f16 weight streaming for
+//                   m <= 16 * MB rows (decode), 4 or 16 waves: MFMA core from skinny.h, bias
+//                   epilogue, 16-bit or fp32 output.
 #include "common.h"
 #include "skinny.h"
 

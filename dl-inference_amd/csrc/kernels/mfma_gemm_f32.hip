@@ -19,8 +19,8 @@
 // the parts in order. Every output is a fixed-order sum: results do not depend on timing.
 //
 // Measured in us, before (fp32 instruction, 4-byte loads) and now: linear 1000 x 4864 x 896 153 / 66,
-// 1000 x 896 x 4864 132 / 67, 64 x 4096 x 16384 113 / 80, 3 x 4096 x 16384 103 / 65; conv 384 x 4096
-// pixels x 1728 159 / 68 + 5; distance from float64 there 7.1e-7 / 2.5e-7 (K = 4864).
+// 1000 x 896 x 4864 132 / 67, 64 x 4096 x 16384 113 / 77, 3 x 4096 x 16384 103 / 52; conv 384 x 4096
+// pixels x 1728 159 / 55 + 6; distance from float64 there 7.1e-7 / 2.5e-7 (K = 4864).
 //
 //  _m16: 16 rows of A against 64 of B (a decode-sized x); _stream: nontemporal weight loads.
 //  _scalar: rows that are not 16-byte aligned or K % 4 != 0 (4-byte loads); convs of windows or images
