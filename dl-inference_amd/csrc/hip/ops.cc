@@ -248,13 +248,21 @@ int unary(FloatKernels& kernels, FloatKernels& wide, const char* op, int dtype, 
 // Rows (queries x heads of a KV group) per workgroup: 128, or 64 for units of at most 64 rows.
 int64_t packedTile(int64_t rows) { return rows > 64 ? 128 : 64; }
 
-// Key splits for `blocks` row tiles over all (sequence, KV head) pairs: about two workgroups per
-// CU, each with at least two 64-key tiles of the cache's capacity.
+// Key splits for `blocks` row tiles over all (sequence, KV head) pairs and a cache of T 64-key tiles:
+// at most two workgroups per CU, and as many as the shorter walk (T / n tiles of 1 to 2.4 us) pays for
+// the partial results (their traffic and merge grow with n): n^2 <= 3 T, or, where the row tiles
+// alone occupy half of the CUs, T / 6. Measured in us, T / 2 splits (the rule before) and these:
+// 3 queries of 28 / 4 heads of 128 over 4000 keys 25.3 / 21.3 (13 splits), 4 x 10 over 3000 30 / 25.2,
+// 14 / 2 heads of 64 over 4000 22.5 / 17.8, over 1000 12.2 / 10.8; 2 x 300 queries of 28 / 4 heads
+// (136 row tiles) over 64 keys 30.9 / 21.8 (unsplit), over 150 31.4 / 24.7, over 600 36.4 / 35.7.
 int64_t packedSplits(int64_t blocks, int64_t capacity) {
-  const int64_t by_tiles = (capacity + dk::kPackedTileK - 1) / dk::kPackedTileK / 2;
-  int64_t splits = blocks > 0 ? 512 / blocks : 1;
-  if (splits > by_tiles) splits = by_tiles;
-  return splits < 1 ? 1 : (splits > 64 ? 64 : splits);
+  const int64_t tiles = (capacity + dk::kPackedTileK - 1) / dk::kPackedTileK;
+  const int64_t most = blocks > 0 ? 512 / blocks : 1;
+  int64_t splits = 1;
+  while (splits < most && splits < 64 &&
+         (blocks >= 128 ? 6 * (splits + 1) <= tiles : (splits + 1) * (splits + 1) <= 3 * tiles))
+    ++splits;
+  return splits;
 }
 
 size_t packedPartialBytes(int64_t rows, int64_t head_dim, int64_t splits) {
