@@ -324,7 +324,8 @@ __device__ __forceinline__ void gemm16(const uint16_t* a, const uint16_t* b, int
     constexpr int kRowStep = kThreads / (BN / 8);
     if (kRuns < kThreads && row0 >= BM) return;  // more threads than runs
     const int64_t gcol = c0 + c8;
-    if (Epi::kVectorOnly || (vec && gcol + 8 <= Cn)) {
+    // (vector-only epilogues have Cn % 8 == 0: a run is inside the columns or past them)
+    if (Epi::kVectorOnly ? gcol < Cn : vec && gcol + 8 <= Cn) {
       const auto cd = epi.column(gcol);
       typename Epi::Run rd[kPer];
 #pragma unroll
@@ -532,7 +533,8 @@ struct SwiGluOut {
 // outside the table copied unchanged); results go to q [B, Hq, S, D], k and v [B, Hkv, S, D]
 // (rotary/kernel.py:6-35, and the reshape + transpose nodes a prompt needs). Vector form only:
 // the host requires D % 8 == 0 and 16-byte aligned pointers (cos/sin too), so every 8-column
-// run lies in one head and reads 16 bytes of each table row.
+// run lies in one head (or past the last column, where gemm16 skips it) and reads 16 bytes of each
+// table row.
 struct QkvHeadsOut {
   static constexpr bool kPairs = false;
   static constexpr bool kVectorOnly = true;

@@ -165,6 +165,39 @@ def test_qkv_rope_heads(B, S, H, Hq, Hkv, D, start, max_pos):
     assert_close(out["v"], heads(vr, Hkv), "bfloat16")
 
 
+@pytest.mark.parametrize("B,S,H,Hq,Hkv,D", [
+    (2, 5, 64, 3, 1, 8),          # 40 columns of a 64-wide tile, two K groups
+    (3, 40, 72, 5, 2, 40),        # 360 columns: 40 past the last 64-wide tile's start
+    (1, 30, 64, 425, 2, 40),      # one row tile over 269 column tiles (128-wide slices)
+    (2, 400, 128, 13, 3, 120),    # 64-wide tiles, one K group
+    (4, 1400, 64, 5, 1, 64),      # 448 columns, 128 x 128 tiles: half of the last one is past them
+    (4, 1400, 64, 5, 1, 56)])     # 392 columns, 128 x 128 tiles: 8 columns in the last one
+def test_qkv_rope_heads_columns_past_the_last_tile(B, S, H, Hq, Hkv, D):
+    """(Hq + 2 Hkv) D need not fill its last tile: nothing is read or written past the operands
+    (guard words after each output stay) and head 0 of the next sequence keeps its values."""
+    from dli import hip
+
+    n, m = (Hq + 2 * Hkv) * D, B * S
+    x, w, b = rand((m, H), 63), rand((n, H), 64, 0.05), rand((n,), 65, 0.1)
+    cos, sin = rope_tables(S, D)
+    guard, spare = 12345.0, 4096
+    outs = [torch.full((B * h * S * D + spare,), guard, dtype=torch.bfloat16, device=DEV)
+            for h in (Hq, Hkv, Hkv)]
+    hip.call("dli_hip_qkv_rope_heads", x.data_ptr(), w.data_ptr(), b.data_ptr(), cos.data_ptr(),
+             sin.data_ptr(), S, *(o.data_ptr() for o in outs), B, S, H, Hq, Hkv, D, 0,
+             hip.current_stream())
+    torch.cuda.synchronize()
+    lin = R((x.cpu().double() @ w.cpu().double().T + b.cpu().double()).numpy()).reshape(B, S, n)
+    heads = lambda a, h: a.reshape(B, S, h, D).transpose(0, 2, 1, 3)
+    parts = np.split(lin, [Hq * D, (Hq + Hkv) * D], -1)
+    for o, part, h, rotated in zip(outs, parts, (Hq, Hkv, Hkv), (True, True, False)):
+        ref = heads(part, h)
+        if rotated:
+            ref = R(ops.rotary(ref, to_np(cos), to_np(sin), start_pos=0))
+        assert_close(o[:-spare].view(B, h, S, D), ref, "bfloat16")
+        assert (o[-spare:] == o[-1]).all() and float(o[-1]) == float(torch.tensor(guard).bfloat16())
+
+
 @pytest.mark.parametrize("B,N,K,splits,bias", CASES + [(16, 4096, 1024, 1, True),
                                                       (16, 4096, 1024, 2, True),
                                                       # n > 1024 at 33-64 rows: the tiled GEMM,
