@@ -32,6 +32,7 @@ TensorMap Engine::run(const Graph& graph, TensorMap tensors) {
 }
 
 TensorMap Engine::run(const Graph& graph, TensorMap tensors, const RunOptions& options) {
+  const StreamScope scope(stream_);
   ExecutionContext context;
   context.kv_cache = &kv_cache_;
   context.stream = stream_;

@@ -153,8 +153,9 @@ Tensor Tensor::zeros(DType dtype, std::vector<std::int64_t> shape) {
 
 Tensor Tensor::cuda(DType dtype, std::vector<std::int64_t> shape, int device_id) {
   validateShape(shape);
-  return Tensor(
-      std::make_shared<Impl>(at::empty(shape, optionsFor(dtype, DeviceType::Cuda, device_id))));
+  at::Tensor tensor = at::empty(shape, optionsFor(dtype, DeviceType::Cuda, device_id));
+  StreamScope::use(tensor, device_id);
+  return Tensor(std::make_shared<Impl>(std::move(tensor)));
 }
 
 Tensor Tensor::externalCuda(DType dtype, std::vector<std::int64_t> shape, void* data,

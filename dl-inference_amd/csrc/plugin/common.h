@@ -101,6 +101,24 @@ class PersistentWorkspace {
   std::vector<Tensor> retired_;
 };
 
+// Scratch of one call from the caching allocator, of any content and given back on return: partial
+// results of kernels that also run without them. Empty where the call may not take any
+// (StreamScope::allowsScratch).
+class CallScratch {
+ public:
+  CallScratch(std::size_t bytes, int device_id) {
+    if (bytes > 0 && StreamScope::allowsScratch(device_id))
+      buffer_ = Tensor::cuda(DType::Float32,
+                             {static_cast<std::int64_t>((bytes + sizeof(float) - 1) / sizeof(float))},
+                             device_id);
+  }
+  void* data() { return buffer_.defined() ? buffer_.deviceData() : nullptr; }
+  std::size_t bytes() const { return buffer_.defined() ? buffer_.nbytes() : 0; }
+
+ private:
+  Tensor buffer_;
+};
+
 template <typename Op>
 void add(OperatorRegistry* registry) {
   registry->registerFactory(Op().type(), [] { return std::make_unique<Op>(); });

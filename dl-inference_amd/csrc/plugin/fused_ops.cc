@@ -171,15 +171,11 @@ class LinearResidualOp final : public Operator {
       throw std::invalid_argument("linear_residual bias size mismatch");
     const auto splits = static_cast<int>(attrs.value_or<std::int64_t>("splits", 1));
     *out[0] = Tensor::cuda(DType::BFloat16, res.shape(), x.deviceId());
-    if (m > 64) {  // a prompt: K parts of the tiled GEMM, scratch from the caching allocator
-      const std::size_t bytes = dli_hip_linear_residual_rows_workspace(m, n, k);
-      Tensor ws;
-      if (bytes > 0)
-        ws = Tensor::cuda(DType::Float32, {static_cast<std::int64_t>(bytes / sizeof(float))},
-                          x.deviceId());
+    if (m > 64) {  // a prompt: K parts of the tiled GEMM
+      CallScratch ws(dli_hip_linear_residual_rows_workspace(m, n, k), x.deviceId());
       check(dli_hip_linear_residual_rows(ptr(x), ptr(w), in.size() == 4 ? ptr(*in[3]) : nullptr,
-                                         ptr(res), ptr(*out[0]), m, n, k,
-                                         bytes > 0 ? ptr(ws) : nullptr, bytes, ctx.stream),
+                                         ptr(res), ptr(*out[0]), m, n, k, ws.data(), ws.bytes(),
+                                         ctx.stream),
             type());
       return;
     }

@@ -137,14 +137,10 @@ class LinearOp final : public Operator {
     *out[0] = allocLike(out_dtype, withLast(in[0]->shape(), n), *in[0]);
     const int act = activationAttr(attrs, type());
     const int dt = hipDtype(in[0]->dtype());
-    // split-K scratch for fp32 shapes with few output tiles (from the caching allocator)
-    const std::size_t ws_bytes = dli_hip_linear_workspace(dt, m, n, k);
-    Tensor ws;
-    if (ws_bytes > 0)
-      ws = allocLike(DType::Float32, {static_cast<std::int64_t>(ws_bytes / sizeof(float))}, *in[0]);
+    CallScratch ws(dli_hip_linear_workspace(dt, m, n, k), in[0]->deviceId());  // K parts
     check(dli_hip_linear_act(dt, hipDtype(out_dtype), ptr(*in[0]), ptr(*in[1]),
                              has_bias ? ptr(*in[2]) : nullptr, ptr(*out[0]), m, n, k, act,
-                             ws_bytes > 0 ? ptr(ws) : nullptr, ws_bytes, ctx.stream),
+                             ws.data(), ws.bytes(), ctx.stream),
           type());
   }
 };
@@ -285,15 +281,13 @@ class AttentionOp final : public Operator {
     const void* pos = positions ? ptr(*positions) : nullptr;
     const int pos_dt = positions ? hipDtype(positions->dtype()) : DLI_I64;
     if (Sq > 1) {
-      const std::size_t bytes =
-          dli_hip_chunk_attention_workspace(dt, B, Hq, Sq, D, e.capacity());
-      Tensor ws;  // partial results of the key splits (from the caching allocator)
-      if (bytes > 0)
-        ws = allocLike(DType::Float32, {static_cast<std::int64_t>(bytes / sizeof(float))}, q);
+      // partial results of the key splits
+      CallScratch ws(dli_hip_chunk_attention_workspace(dt, B, Hq, Sq, D, e.capacity()),
+                     q.deviceId());
       check(dli_hip_chunk_attention(dt, ptr(q), ptr(e.key_pool), ptr(e.value_pool), table,
                                     ptr(*out[0]), B, Hq, Hkv, Sq, D, e.block_size, e.max_blocks,
-                                    past, pos, pos_dt, causal ? 1 : 0, scale,
-                                    bytes > 0 ? ptr(ws) : nullptr, bytes, ctx.stream),
+                                    past, pos, pos_dt, causal ? 1 : 0, scale, ws.data(), ws.bytes(),
+                                    ctx.stream),
             type());
       return;
     }
@@ -402,13 +396,10 @@ class Conv2dOp final : public Operator {
     const int act = activationAttr(attrs, type());
     *out[0] = allocLike(x.dtype(), {n, oc, oh, ow}, x);
     const int dt = hipDtype(x.dtype());
-    const std::size_t ws_bytes = dli_hip_conv2d_workspace(dt, n, c, oc, kh, kw, oh, ow);
-    Tensor ws;
-    if (ws_bytes > 0)
-      ws = allocLike(DType::Float32, {static_cast<std::int64_t>(ws_bytes / sizeof(float))}, x);
+    CallScratch ws(dli_hip_conv2d_workspace(dt, n, c, oc, kh, kw, oh, ow), x.deviceId());
     check(dli_hip_conv2d_act(dt, ptr(x), ptr(w), has_bias ? ptr(*in[2]) : nullptr, ptr(*out[0]),
                              n, c, h, wd, oc, kh, kw, oh, ow, stride[0], stride[1], pad[0],
-                             pad[1], act, ws_bytes > 0 ? ptr(ws) : nullptr, ws_bytes, ctx.stream),
+                             pad[1], act, ws.data(), ws.bytes(), ctx.stream),
           type());
   }
 };

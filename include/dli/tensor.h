@@ -78,6 +78,28 @@ class Tensor {
   void* external_device_ptr_ = nullptr;
 };
 
+// The stream that this thread's device work goes to while the scope lives (Engine::run opens one).
+// The caching allocator hands a freed block out again in the order of torch's current stream, so
+// where `stream` is another one, every tensor that Tensor::cuda makes is recorded on it: its block
+// is reused only once the work queued on `stream` at the time of the free is done.
+class StreamScope {
+ public:
+  explicit StreamScope(void* stream);
+  ~StreamScope();
+  StreamScope(const StreamScope&) = delete;
+  StreamScope& operator=(const StreamScope&) = delete;
+
+  // Whether a call may take scratch that it gives back on return: not where the scope's stream is
+  // being captured and is not torch's current one. The graph would then keep the address of a block
+  // that belongs to no capture, and an event recorded for the block would end up in the graph.
+  static bool allowsScratch(int device_id);
+  static void use(const at::Tensor& tensor, int device_id);
+
+ private:
+  void* previous_;
+  bool active_;
+};
+
 bool sameShape(const Tensor& lhs, const Tensor& rhs);
 std::size_t contiguousOffset(const std::vector<std::int64_t>& shape,
                              const std::vector<std::int64_t>& indices);
