@@ -269,13 +269,19 @@ size_t packedPartialBytes(int64_t rows, int64_t head_dim, int64_t splits) {
   return static_cast<size_t>(rows * splits * (head_dim + 2)) * sizeof(float);
 }
 
+// The flash and packed kernels mask scores and take their maximum before the scale is multiplied in
+// (one fma per probability), which needs a positive one: with another scale a key that a row does not
+// see, at -inf, would come out as +inf or NaN. The row kernels scale q first and take any.
+bool scaleAfterMask(float scale) { return scale > 0.f && std::isfinite(scale); }
+
 // Forms that the packed kernels take (others run on the generic kernels).
 bool packedForm(int dtype, int64_t batch, int64_t q_heads, int64_t kv_heads, int64_t seq_q,
-                int64_t keys, const void* q, const void* k, const void* v, const void* out) {
+                int64_t keys, float scale, const void* q, const void* k, const void* v,
+                const void* out) {
   const int64_t limit = int64_t{1} << 30;
   return (dtype == DLI_BF16 || dtype == DLI_F32) && batch * kv_heads <= 65535 && keys > 0 && keys < limit &&
-         seq_q < limit && seq_q * (q_heads / kv_heads) < limit && aligned16(q) && aligned16(k) &&
-         aligned16(v) && aligned16(out);
+         seq_q < limit && seq_q * (q_heads / kv_heads) < limit && scaleAfterMask(scale) &&
+         aligned16(q) && aligned16(k) && aligned16(v) && aligned16(out);
 }
 
 }  // namespace
@@ -767,7 +773,7 @@ int dli_hip_rotary(int dtype, const void* q, const void* k, const float* cos_tab
                 pos64);
 }
 
-// attention with out as [B, Hq, Sq, D] (out_bshd 0) or [B, Sq, Hq, D] (1, flash path only)
+// attention with out as [B, Hq, Sq, D] (out_bshd 0) or [B, Sq, Hq, D] (1, the flash kernel's forms)
 static int attentionImpl(int dtype, const void* q, const void* k, const void* v, void* out,
                   int64_t batch, int64_t q_heads, int64_t kv_heads, int64_t seq_q, int64_t seq_k,
                   int64_t head_dim, int causal, float scale, int out_bshd, void* stream) {
@@ -783,9 +789,11 @@ static int attentionImpl(int dtype, const void* q, const void* k, const void* v,
     return badArg("attention", "NULL pointer");
   // bf16 with head_dim 64 (prefill): flash-style MFMA kernel, 128 queries per workgroup (64 for
   // query sequences of at most 64)
-  if (dtype == DLI_BF16 && head_dim == 64 && seq_k > 0 && batch * q_heads <= 65535 &&
-      seq_q < (int64_t{1} << 30) && seq_k < (int64_t{1} << 30) &&
-      aligned16(q) && aligned16(k) && aligned16(v) && aligned16(out)) {
+  const bool flash = dtype == DLI_BF16 && head_dim == 64 && seq_k > 0 &&
+                     batch * q_heads <= 65535 && seq_q < (int64_t{1} << 30) &&
+                     seq_k < (int64_t{1} << 30) && aligned16(q) && aligned16(k) && aligned16(v) &&
+                     aligned16(out);
+  if (flash && scaleAfterMask(scale)) {
     const float log2e = 1.4426950408889634f;
     const int64_t tile_q = seq_q > 64 ? 128 : 64;
     return launch(tile_q == 128 ? k_flash_attention_q32 : k_flash_attention,
@@ -799,7 +807,7 @@ static int attentionImpl(int dtype, const void* q, const void* k, const void* v,
   // fp32 with head_dim 64 or 128: the same on the fp32 matrix instruction.
   const bool f32 = dtype == DLI_F32;
   if (!out_bshd && (head_dim == 128 || (f32 && head_dim == 64)) && seq_q >= 16 &&
-      packedForm(dtype, batch, q_heads, kv_heads, seq_q, seq_k, q, k, v, out)) {
+      packedForm(dtype, batch, q_heads, kv_heads, seq_q, seq_k, scale, q, k, v, out)) {
     dk::PackedAttentionArgs a{};
     a.q = q;
     a.k = k;
@@ -820,12 +828,12 @@ static int attentionImpl(int dtype, const void* q, const void* k, const void* v,
                   {blocksFor(unit_rows, tile), static_cast<unsigned>(batch * kv_heads)}, {256}, 0,
                   stream, a);
   }
-  if (out_bshd)
+  if (out_bshd && !flash)
     return badArg("attention", "a [B, S, H, D] output needs bf16, head_dim 64, seq_k > 0 and "
                                "16-byte aligned tensors (the flash kernel)");
   if (rows > 0x7fffffff) return badArg("attention", "too many query rows");
   return launch(*ka, {static_cast<unsigned>(rows)}, {64}, 0, stream, q, k, v, out, batch, q_heads,
-                kv_heads, seq_q, seq_k, head_dim, causal, scale);
+                kv_heads, seq_q, seq_k, head_dim, causal, scale, out_bshd);
 }
 
 int dli_hip_attention(int dtype, const void* q, const void* k, const void* v, void* out,
@@ -912,7 +920,7 @@ static int pagedAttention(int dtype, const void* q, const void* key_pool, const 
   // several queries per sequence: the packed-row MFMA kernels (64-key tiles inside cache blocks)
   if (dtype == DLI_BF16 && seq_q > 1 && (head_dim == 64 || head_dim == 128) &&
       block_size % dk::kPackedTileK == 0 && block_size < (int64_t{1} << 30) && max_blocks < (int64_t{1} << 30) &&
-      packedForm(dtype, batch, q_heads, kv_heads, seq_q, max_blocks * block_size, q, key_pool,
+      packedForm(dtype, batch, q_heads, kv_heads, seq_q, max_blocks * block_size, scale, q, key_pool,
                  value_pool, out)) {
     const int64_t unit_rows = seq_q * (q_heads / kv_heads), tile = packedTile(unit_rows);
     const int64_t units = batch * kv_heads, blocks = (unit_rows + tile - 1) / tile;

@@ -98,7 +98,7 @@ __device__ void attendRow(const T* qrow, T* orow, const KV& kv, int64_t b, int64
 template <typename T>
 __device__ void attention_impl(const void* q_, const void* k_, const void* v_, void* out_,
                                int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq, int64_t Sk,
-                               int64_t D, int causal, float scale) {
+                               int64_t D, int causal, float scale, int out_bshd) {
   __shared__ float q_lds[256];
   __shared__ float p_lds[kWave];
   const int64_t row = blockIdx.x;  // ((b * Hq + h) * Sq + i)
@@ -112,7 +112,8 @@ __device__ void attention_impl(const void* q_, const void* k_, const void* v_, v
     const int64_t limit = (Sk - Sq) + i + 1;
     kv_len = limit < Sk ? (limit > 0 ? limit : 0) : Sk;
   }
-  attendRow(static_cast<const T*>(q_) + row * D, static_cast<T*>(out_) + row * D, kv, b, kvh,
+  const int64_t out_row = out_bshd ? (b * Sq + i) * Hq + h : row;
+  attendRow(static_cast<const T*>(q_) + row * D, static_cast<T*>(out_) + out_row * D, kv, b, kvh,
             kv_len, D, scale, q_lds, p_lds);
 }
 
@@ -263,8 +264,9 @@ extern "C" __global__ void __launch_bounds__(256)
 
 DK_FLOAT_KERNELS(attention, 64,
                  (const void* q, const void* k, const void* v, void* out, int64_t B, int64_t Hq,
-                  int64_t Hkv, int64_t Sq, int64_t Sk, int64_t D, int causal, float scale),
-                 (q, k, v, out, B, Hq, Hkv, Sq, Sk, D, causal, scale))
+                  int64_t Hkv, int64_t Sq, int64_t Sk, int64_t D, int causal, float scale,
+                  int out_bshd),
+                 (q, k, v, out, B, Hq, Hkv, Sq, Sk, D, causal, scale, out_bshd))
 DK_FLOAT_KERNELS(paged_attention, 64,
                  (const void* q, const void* k_pool, const void* v_pool,
                   const int32_t* block_table, void* out, int64_t B, int64_t Hq, int64_t Hkv,

@@ -164,3 +164,33 @@ def test_dense_f32_never_reads_hidden_values(d):
     err = (out[:, :, :-1] - clean[:, :, :-1]).norm()
     assert err <= 1e-6 * clean[:, :, :-1].norm()
     assert torch.isinf(out[:, :, -1, ::2]).all() and torch.isnan(out[:, :, -1, 1::2]).all()
+
+
+@pytest.mark.parametrize("scale", [0.0, -0.1, 0.3])
+@pytest.mark.parametrize("dtype,d,layout", [
+    (torch.bfloat16, 128, "bhsd"), (torch.float32, 64, "bhsd"), (torch.float32, 128, "bhsd"),
+    (torch.bfloat16, 64, "bhsd"), (torch.bfloat16, 64, "bshd")])
+def test_dense_scale_of_any_sign(dtype, d, layout, scale):
+    import dli
+
+    g = torch.Generator().manual_seed(31)
+    q, k, v = (torch.randn(2, h, s, d, generator=g).to(dtype).to(DEV)
+               for h, s in ((6, 20), (2, 90), (2, 90)))
+    out = run_attention({"q": q, "k": k, "v": v},
+                        {"causal": True, "scale": scale, "output_layout": layout},
+                        dli.Engine().load_plugin())
+    out = out.transpose(1, 2) if layout == "bshd" else out
+    check(out, ops.attention(to_np(q), to_np(k), to_np(v), causal=True, scale=scale))
+
+
+@pytest.mark.parametrize("scale", [0.0, -0.1, 0.3])
+@pytest.mark.parametrize("d", [64, 128])
+def test_paged_chunk_scale_of_any_sign(d, scale):
+    past = [70, 200]
+    engine, inputs, hist_k, hist_v = paged_case(6, 2, d, 7, past, True)
+    out = run_attention(inputs, {"causal": True, "kv_cache": "L", "scale": scale}, engine)
+    q, k, v = inputs["q"], inputs["k"], inputs["v"]
+    for b, n in enumerate(past):
+        keys = np.concatenate([to_np(hist_k[b:b + 1, :, :n]), to_np(k[b:b + 1])], 2)
+        vals = np.concatenate([to_np(hist_v[b:b + 1, :, :n]), to_np(v[b:b + 1])], 2)
+        check(out[b:b + 1], ops.attention(to_np(q[b:b + 1]), keys, vals, causal=True, scale=scale))
