@@ -74,12 +74,14 @@ __device__ __forceinline__ int vtPos(int key) {
   return (key & 32) + ((key >> 2) & 3) * 8 + ((key >> 4) & 1) * 4 + (key & 3);
 }
 
-// true if one of the 8 bf16 is an infinity or a NaN
-__device__ __forceinline__ bool nonFinite(const U128& w) {
+// True if a sum is an infinity or a NaN. An infinite or NaN value always makes it so, but the matrix
+// product may give a NaN where the row's own arithmetic has an infinity or a finite result: the key may
+// be one that the row does not see (probability 0), and one that it sees meets the terms of p = hi + lo
+// with either sign. A workgroup with such a sum redoes its rows key by key.
+__device__ __forceinline__ bool nonFinite(const f32x4& v) {
   bool bad = false;
 #pragma unroll
-  for (int k = 0; k < 4; ++k)
-    bad = bad || (w[k] & 0x7F80u) == 0x7F80u || (w[k] & 0x7F800000u) == 0x7F800000u;
+  for (int k = 0; k < 4; ++k) bad = bad || (__float_as_uint(v[k]) & 0x7F800000u) == 0x7F800000u;
   return bad;
 }
 
@@ -198,9 +200,8 @@ __device__ __forceinline__ void packedAttention(const PackedAttentionArgs& a) {
     for (int c = 0; c < DK; ++c) qf[qb][c] = gload16(qp + c * 32);
     lim[qb] = visibleKeys<kPaged>(a, past, i);
   }
-  // keys some row of the workgroup sees; keys every row of the workgroup / of this wave sees
+  // keys some row of the workgroup sees; keys every row of this wave sees
   const int wg_keys = visibleKeys<kPaged>(a, past, query(p0 + kTileQ - 1));
-  const int wg_full = visibleKeys<kPaged>(a, past, query(p0));
   const int wave_full = visibleKeys<kPaged>(a, past, query(pw));
 
   const int all_tiles = (wg_keys + kTileK - 1) / kTileK;
@@ -300,24 +301,13 @@ __device__ __forceinline__ void packedAttention(const PackedAttentionArgs& a) {
   }
   const U128 ones{0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u};  // bf16 1.0 x 8
 
-  int special = 0;
   if (kt0 < kt1) fetch(kt0);
   for (int kt = kt0; kt < kt1; ++kt) {
     const int k0 = kt * kTileK;
     if (k0 + kTileK > wg_keys) zeroPast(k0);
     __syncthreads();  // the previous tile is no longer read
     stash();
-    // A row that does not see a key has probability 0 for it, which an infinite or NaN value
-    // would turn into a NaN in the MFMA. Tiles that some row sees in part are checked for such
-    // values; a workgroup that meets one redoes its rows key by key at the end.
-    if (k0 + kTileK > wg_full) {  // uniform
-      bool bad = false;
-#pragma unroll
-      for (int i = 0; i < kPer; ++i) bad = bad || nonFinite(vr[i]);
-      special |= __syncthreads_or(bad);
-    } else {
-      __syncthreads();
-    }
+    __syncthreads();
     if (kt + 1 < kt1) fetch(kt + 1);
     if (!active) continue;
 
@@ -415,7 +405,12 @@ __device__ __forceinline__ void packedAttention(const PackedAttentionArgs& a) {
       }
   }
 
-  if (special != 0) {  // uniform
+  bool bad = false;
+#pragma unroll
+  for (int qb = 0; qb < QB; ++qb)
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) bad = bad || nonFinite(o[qb][dt]);
+  if (__syncthreads_or(bad)) {
     for (int q = wave; q < kTileQ && p0 + q < rows; q += kThreads / kWave)
       rowByKeys<D, kPaged, bf16>(a, unit, rows, p0 + q, kt0 * kTileK, kt1 * kTileK);
     return;
@@ -484,7 +479,6 @@ __device__ __forceinline__ void packedAttentionF32(const PackedAttentionArgs& a)
   }
   const int lim = visibleKeys<false>(a, 0, i0);
   const int wg_keys = visibleKeys<false>(a, 0, query(p0 + 63));
-  const int wg_full = visibleKeys<false>(a, 0, query(p0));
   const int wave_full = visibleKeys<false>(a, 0, query(pw));
   const int tiles = (wg_keys + kTileK - 1) / kTileK;
 
@@ -507,26 +501,17 @@ __device__ __forceinline__ void packedAttentionF32(const PackedAttentionArgs& a)
 #pragma unroll
   for (int dt = 0; dt < DT; ++dt) o[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
   float m_run = -INFINITY, l_run = 0.f;
-  int special = 0;
   if (tiles > 0) fetch(0);
   for (int kt = 0; kt < tiles; ++kt) {
     const int k0 = kt * kTileK;
     __syncthreads();  // the previous tile is no longer read
-    bool bad = false;
 #pragma unroll
     for (int i = 0; i < kPer; ++i) {
       const int c = t + i * kThreads, at = (c / kRowChunks) * kPitch + (c % kRowChunks) * 4;
       *reinterpret_cast<f32x4*>(&Ks[at]) = kr[i];
       *reinterpret_cast<f32x4*>(&Vs[at]) = vr[i];
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        bad = bad || (__float_as_uint(vr[i][j]) & 0x7F800000u) == 0x7F800000u;
     }
-    // infinite or NaN values in a tile that some row sees in part: as in packedAttention
-    if (k0 + kTileK > wg_full)  // uniform
-      special |= __syncthreads_or(bad);
-    else
-      __syncthreads();
+    __syncthreads();
     if (kt + 1 < tiles) fetch(kt + 1);
     if (!active) continue;
     f32x4 s[4];
@@ -583,7 +568,10 @@ __device__ __forceinline__ void packedAttentionF32(const PackedAttentionArgs& a)
           o[dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(
               Vs[(kk * 16 + g * 4 + i) * kPitch + dt * 16 + r], s[kk][i], o[dt], 0, 0, 0);
   }
-  if (special != 0) {  // uniform
+  bool bad = false;
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt) bad = bad || nonFinite(o[dt]);
+  if (__syncthreads_or(bad)) {
     for (int q = wave; q < 64 && p0 + q < rows; q += kThreads / kWave)
       rowByKeys<D, false, float>(a, unit, rows, p0 + q, 0, tiles * kTileK);
     return;

@@ -194,3 +194,43 @@ def test_paged_chunk_scale_of_any_sign(d, scale):
         keys = np.concatenate([to_np(hist_k[b:b + 1, :, :n]), to_np(k[b:b + 1])], 2)
         vals = np.concatenate([to_np(hist_v[b:b + 1, :, :n]), to_np(v[b:b + 1])], 2)
         check(out[b:b + 1], ops.attention(to_np(q[b:b + 1]), keys, vals, causal=True, scale=scale))
+
+
+def check_spoiled(run, clean, v, seen):
+    """Infinities of both signs and a NaN at `seen` of the values: the heads that read them give them
+    back, other dimensions keep their values."""
+    v[seen + (slice(0, 1),)], v[seen + (slice(5, 6),)] = float("inf"), float("-inf")
+    v[seen + (slice(9, 10),)] = float("nan")
+    out = run()
+    assert (out[..., 0] == float("inf")).all() and (out[..., 5] == float("-inf")).all()
+    assert torch.isnan(out[..., 9]).all()
+    rest = [d for d in range(out.shape[-1]) if d not in (0, 5, 9)]
+    err = (out[..., rest].double() - clean[..., rest].double()).norm()
+    assert err <= REL * clean[..., rest].double().norm()
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("sq,past", [(5, 200), (70, 130), (3, 4000)])
+def test_paged_chunk_infinite_value_of_a_cached_key(d, sq, past):
+    """A key that every row sees, in a tile without hidden keys (and in one key split of several)."""
+    engine, inputs, _, _ = paged_case(14, 2, d, sq, [past], True)
+    attrs = {"causal": True, "kv_cache": "L"}
+    clean = run_attention(inputs, attrs, engine)
+    entry = engine.kv_cache_entry("L")
+    blk = int(entry["block_table"][0, 0])
+    values = entry["value_pool"].transpose(2, 3)  # [block, head, slot, d]
+    check_spoiled(lambda: run_attention(inputs, attrs, engine), clean, values,
+                  (blk, slice(None), 3))
+
+
+@pytest.mark.parametrize("dtype,d", [(torch.bfloat16, 128), (torch.float32, 64),
+                                     (torch.float32, 128)])
+def test_dense_infinite_value_of_a_seen_key(dtype, d):
+    import dli
+
+    g = torch.Generator().manual_seed(41)
+    q, k, v = (torch.randn(2, h, s, d, generator=g).to(dtype).to(DEV)
+               for h, s in ((6, 40), (2, 200), (2, 200)))
+    engine = dli.Engine().load_plugin()
+    run = lambda: run_attention({"q": q, "k": k, "v": v}, {"causal": True}, engine)
+    check_spoiled(run, run(), v, (slice(None), slice(None), 3))
