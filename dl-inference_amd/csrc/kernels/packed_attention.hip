@@ -15,16 +15,15 @@
 //   1. S^T = K Q^T with v_mfma_f32_16x16x32_bf16: lane l = 16 g + r holds the scores of row r for
 //      keys 4 g + i of each 16-key block;
 //   2. online softmax per row in fp32, base 2, with a lazy rescale of the running output;
-//   3. O^T += V^T P^T. The probabilities are fp32; each is split into two bf16 terms
-//      p = hi + lo (relative error 2^-18, below the fp32 sums' own), and both terms go through
-//      the MFMA, so that nothing is rounded to 16 bits before the output. The row sums come from
-//      the same terms against an all-ones operand.
+//   3. O^T += V^T P^T. The probabilities are fp32; each is the exact sum of three bf16 terms (8
+//      mantissa bits each, cut by truncation), and all three go through the MFMA, so that nothing is
+//      rounded to 16 bits before the output. The row sums are fp32 adds.
 // V^T lies in LDS with the 32 keys of an MFMA step permuted (key 16 h + 4 g + i at 8 g + 4 h + i),
 // which is the order in which a lane's probabilities stand, so a V fragment is one 16-byte read.
 // The 16-byte units of a V^T row are xor-swizzled by d (the 16 rows of a fragment read fall on
 // distinct banks, and the 2-key words of the dense form's transposing stores on few).
 //
-// Bound by the matrix cores (QK once, PV twice for the split) together with the exponentials of
+// Bound by the matrix cores (QK once, PV three times for the split) together with the exponentials of
 // the same waves. Measured against one wave per row with a scalar dot per key (attention.hip):
 //   paged, 2 x 300 new tokens over 3000 and 1500 cached, 28 / 4 heads, head_dim 128: 16.2 ms
 //     before, 70 us now (295 TFLOP/s of attention arithmetic) and 8 us for the merge of 3 splits;
@@ -76,8 +75,8 @@ __device__ __forceinline__ int vtPos(int key) {
 
 // True if a sum is an infinity or a NaN. An infinite or NaN value always makes it so, but the matrix
 // product may give a NaN where the row's own arithmetic has an infinity or a finite result: the key may
-// be one that the row does not see (probability 0), and one that it sees meets the terms of p = hi + lo
-// with either sign. A workgroup with such a sum redoes its rows key by key.
+// be one that the row does not see (probability 0), and one that it sees meets the terms of p with
+// either sign. A workgroup with such a sum redoes its rows key by key.
 __device__ __forceinline__ bool nonFinite(const f32x4& v) {
   bool bad = false;
 #pragma unroll
@@ -290,16 +289,15 @@ __device__ __forceinline__ void packedAttention(const PackedAttentionArgs& a) {
   };
 
   f32x4 o[QB][DT];  // O^T tiles: d = 16 dt + 4 g + i, row pw + 16 qb + r
-  f32x4 lsum[QB];   // row sums (element 0 kept current)
+  float lsum[QB];   // row sums over the lane group's keys
   float m_run[QB];
 #pragma unroll
   for (int qb = 0; qb < QB; ++qb) {
     m_run[qb] = -INFINITY;
-    lsum[qb] = f32x4{0.f, 0.f, 0.f, 0.f};
+    lsum[qb] = 0.f;
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) o[qb][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
-  const U128 ones{0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u};  // bf16 1.0 x 8
 
   if (kt0 < kt1) fetch(kt0);
   for (int kt = kt0; kt < kt1; ++kt) {
@@ -331,7 +329,6 @@ __device__ __forceinline__ void packedAttention(const PackedAttentionArgs& a) {
     __builtin_amdgcn_sched_barrier(0);
     // 2. online softmax per row (keys a row does not see: -inf), reference point in scaled units
     const bool full = k0 + kTileK <= wave_full;  // uniform over the wave: every key visible
-    bf16x8 ph[QB][2], pl[QB][2];
 #pragma unroll
     for (int qb = 0; qb < QB; ++qb) {
       float tmax = -INFINITY;
@@ -357,7 +354,7 @@ __device__ __forceinline__ void packedAttention(const PackedAttentionArgs& a) {
         m_run[qb] = grow ? tm : m_run[qb];
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt) o[qb][dt] *= alpha;
-        lsum[qb][0] *= alpha;
+        lsum[qb] *= alpha;
       }
       const float base = m_run[qb] == -INFINITY ? 0.f : m_run[qb];
 #pragma unroll
@@ -365,44 +362,44 @@ __device__ __forceinline__ void packedAttention(const PackedAttentionArgs& a) {
 #pragma unroll
         for (int i = 0; i < 4; ++i)
           s[qb][kk][i] = __builtin_amdgcn_exp2f(fmaf(s[qb][kk][i], a.scale_log2, -base));
-      // keys of 32-key step kc, lane group g: 4 g + i of blocks 2 kc and 2 kc + 1
-#pragma unroll
-      for (int kc = 0; kc < 2; ++kc) {
-        const bf16x4_t h0 = __builtin_convertvector(s[qb][2 * kc], bf16x4_t);
-        const bf16x4_t h1 = __builtin_convertvector(s[qb][2 * kc + 1], bf16x4_t);
-        const f32x4 d0 = s[qb][2 * kc] - __builtin_convertvector(h0, f32x4);
-        const f32x4 d1 = s[qb][2 * kc + 1] - __builtin_convertvector(h1, f32x4);
-        const bf16x4_t l0 = __builtin_convertvector(d0, bf16x4_t);
-        const bf16x4_t l1 = __builtin_convertvector(d1, bf16x4_t);
-        ph[qb][kc] = bf16x8{h0[0], h0[1], h0[2], h0[3], h1[0], h1[1], h1[2], h1[3]};
-        pl[qb][kc] = bf16x8{l0[0], l0[1], l0[2], l0[3], l1[0], l1[1], l1[2], l1[3]};
-      }
+      const f32x4 part = (s[qb][0] + s[qb][1]) + (s[qb][2] + s[qb][3]);
+      lsum[qb] += (part[0] + part[1]) + (part[2] + part[3]);
     }
     __builtin_amdgcn_sched_barrier(0);
-    // 3. O^T += V^T P^T, 32 keys per step; each V^T fragment serves both terms of every row block
+    // 3. O^T += V^T P^T, 32 keys per step; each V^T fragment serves every term of every row block
 #pragma unroll
-    for (int kc = 0; kc < 2; ++kc)
+    for (int kc = 0; kc < 2; ++kc) {
+      // lane group g: keys 4 g + i of blocks 2 kc and 2 kc + 1; the largest term first. Cut off
+      // instead of rounded, a term is one byte permute of two values (2 x 300 queries over 3000
+      // keys, head_dim 64: 55 us, 61 with rounded terms)
+      bf16x8 pt[3][QB];
+#pragma unroll
+      for (int qb = 0; qb < QB; ++qb)
+#pragma unroll
+        for (int u = 0; u < 3; ++u) {
+          U128 w;
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {  // keys 2 j and 2 j + 1 of the lane's 8
+            f32x4& x = s[qb][2 * kc + j / 2];
+            const int i = 2 * (j % 2);
+            const uint32_t lo = __float_as_uint(x[i]), hi = __float_as_uint(x[i + 1]);
+            w[j] = __builtin_amdgcn_perm(hi, lo, 0x07060302u);  // the upper halves
+            x[i] -= __uint_as_float(lo & 0xFFFF0000u);
+            x[i + 1] -= __uint_as_float(hi & 0xFFFF0000u);
+          }
+          pt[u][qb] = asBf16x8(w);
+        }
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt) {
         const U128 va = *reinterpret_cast<const U128*>(&Vt[vtAt<kPaged>(dt * 16 + r, kc * 32 + g * 8)]);
 #pragma unroll
-        for (int qb = 0; qb < QB; ++qb)
-          o[qb][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(asBf16x8(va), ph[qb][kc],
-                                                              o[qb][dt], 0, 0, 0);
+        for (int u = 2; u >= 0; --u)
 #pragma unroll
-        for (int qb = 0; qb < QB; ++qb)
-          o[qb][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(asBf16x8(va), pl[qb][kc],
-                                                              o[qb][dt], 0, 0, 0);
+          for (int qb = 0; qb < QB; ++qb)
+            o[qb][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(asBf16x8(va), pt[u][qb],
+                                                                o[qb][dt], 0, 0, 0);
       }
-#pragma unroll
-    for (int kc = 0; kc < 2; ++kc)
-#pragma unroll
-      for (int qb = 0; qb < QB; ++qb) {
-        lsum[qb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(asBf16x8(ones), ph[qb][kc], lsum[qb],
-                                                           0, 0, 0);
-        lsum[qb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(asBf16x8(ones), pl[qb][kc], lsum[qb],
-                                                           0, 0, 0);
-      }
+    }
   }
 
   bool bad = false;
@@ -417,13 +414,14 @@ __device__ __forceinline__ void packedAttention(const PackedAttentionArgs& a) {
   }
 #pragma unroll
   for (int qb = 0; qb < QB; ++qb) {
+    const float l = rowsSum(lsum[qb]);
     const int p = pw + qb * 16 + r;
     if (p >= rows) continue;
     if (a.splits > 1) {
       const int64_t at = partIndex(a, unit, rows, p);
       if (g == 0) {
         gp(a.part_ml)[at * 2] = m_run[qb];
-        gp(a.part_ml)[at * 2 + 1] = lsum[qb][0];
+        gp(a.part_ml)[at * 2 + 1] = l;
       }
 #pragma unroll
       for (int dt = 0; dt < DT; ++dt)
@@ -431,7 +429,7 @@ __device__ __forceinline__ void packedAttention(const PackedAttentionArgs& a) {
       continue;
     }
     // a row that sees no key gives zeros; one whose visible scores are all -inf gives NaN
-    const float inv = lim[qb] > 0 ? 1.f / lsum[qb][0] : 0.f;
+    const float inv = lim[qb] > 0 ? 1.f / l : 0.f;
     uint16_t* orow = outRow<D, uint16_t>(a, b, kvh, group, p) + g * 4;
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) {

@@ -234,3 +234,43 @@ def test_dense_infinite_value_of_a_seen_key(dtype, d):
     engine = dli.Engine().load_plugin()
     run = lambda: run_attention({"q": q, "k": k, "v": v}, {"causal": True}, engine)
     check_spoiled(run, run(), v, (slice(None), slice(None), 3))
+
+
+@pytest.mark.parametrize("d,paged", [(128, False), (64, True), (128, True)])
+def test_probabilities_keep_fp32(d, paged):
+    """Two keys of almost the same probability p with values 1 and -1: the output is their
+    difference, about 2^-13 p, over the row sum. An fp32 probability is off by about 2 ulps, 2^-23 p,
+    so the difference by 2^-9 of itself, like the rounding of the output; probabilities of 17 or 18
+    bits are off by up to 2^-5 of it."""
+    import dli
+
+    batch, hkv, sq, sk, delta = 8, 4, 16, 200, 2.0 ** -13
+    c = torch.linspace(0.05, 0.95, batch * hkv).view(batch, hkv).to(torch.bfloat16).to(DEV)
+    q = torch.zeros(batch, 2 * hkv, sq, d, dtype=torch.bfloat16, device=DEV)
+    q[..., :2] = 1
+    k = torch.zeros(batch, hkv, sk, d, dtype=torch.bfloat16, device=DEV)
+    k[..., 0] = -100  # probability 0
+    k[:, :, 9, 0] = 0  # the row maximum
+    k[:, :, 70, 0] = k[:, :, 71, 0] = -c
+    k[:, :, 71, 1] = -delta
+    v = torch.zeros_like(k)
+    v[:, :, 70], v[:, :, 71] = 1, -1
+    engine, attrs = dli.Engine().load_plugin(), {"scale": 1.0}
+    if paged:
+        past = sk - sq
+        engine.configure_kv_cache(block_size=64, max_seq_len=sk)
+        engine.reserve_kv_cache("L", "bfloat16", batch, hkv, d)
+        entry = engine.kv_cache_entry("L")
+        for j in range(past):
+            blocks = entry["block_table"][:, j // 64].long()
+            entry["key_pool"][blocks, :, j % 64] = k[:, :, j]
+            entry["value_pool"][blocks, :, :, j % 64] = v[:, :, j]
+        out = run_attention({"q": q, "k": k[:, :, past:].contiguous(),
+                             "v": v[:, :, past:].contiguous(),
+                             "positions": torch.full((batch,), past, device=DEV)},
+                            {**attrs, "kv_cache": "L"}, engine)
+    else:
+        out = run_attention({"q": q, "k": k, "v": v}, attrs, engine)
+    pa, pb = torch.exp(-c.double()), torch.exp(-c.double() - delta)
+    ref = ((pa - pb) / (1 + pa + pb)).repeat_interleave(2, 1)[:, :, None, None]
+    assert ((out.double() - ref).abs() <= 2.0 ** -7 * ref).all()
