@@ -217,8 +217,9 @@ struct ConvPatch : AlongRows<ROWS> {
 // one: the large sum is then rounded once per 32 products (with one accumulator for all six, 5 to 6
 // times, which showed: 3.9e-7 from float64 over the CNN against 2.2e-7 with the fp32 instruction).
 // An infinity or NaN among the operands, or a sum past the fp32 range, makes a result of the tile
-// non-finite; such a tile is computed again with the fp32 instruction, whose rules for them hold.
-// (Terms below the bf16 normal range, of operands below 2^-110, may count as zero.)
+// non-finite; such a tile is computed again with the fp32 instruction, whose rules for them hold. So is
+// a tile with operands below 2^-110, whose last bits lie below the smallest bf16 (2^-133): they are
+// what is left in the lower half of the third term.
 //
 // Staging splits a chunk once for the waves that share it. LDS holds an operand's slice as planes of
 // 16-byte runs (8 k of one term), one plane per term and run g of the 32 k, row r of a plane at
@@ -234,7 +235,11 @@ __device__ __forceinline__ int runAt(int row, int g) {
   return (g * ROWS + (row ^ mask)) * 16;
 }
 
-__device__ __forceinline__ void split3(const f32x4& v, uint2 (&t)[3]) {
+// lost: the or of the third terms, whose lower halves are what the bf16 terms drop (the upper halves:
+// noise). The asm statements are empty: they keep the ors where the values are made. Gathered for all
+// chunks at the end of a step, the ors held the values in registers and made 4096^3 6% slower, 500 x 896 x
+// 4864 (_g2) 11%; like this 1% and 6%.
+__device__ __forceinline__ void split3(const f32x4& v, uint2 (&t)[3], uint32_t& lost) {
   uint32_t h[4], m[4], l[4];
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
@@ -248,6 +253,10 @@ __device__ __forceinline__ void split3(const f32x4& v, uint2 (&t)[3]) {
                  __builtin_amdgcn_perm(u[3], u[2], 0x07060302u)};
   };
   t[0] = pack(h), t[1] = pack(m), t[2] = pack(l);
+  lost |= l[0] | l[1];
+  asm("" : "+v"(lost));
+  lost |= l[2] | l[3];
+  asm("" : "+v"(lost));
 }
 
 // WR x WC: the 4 waves of a group over the tile.
@@ -278,6 +287,10 @@ __device__ __forceinline__ void gemmF32(ASrc A, BSrc B, int64_t R, int64_t Cn, i
   A.begin(r0, t);
   B.begin(c0, t);
   f32x4 acc[TM][TN], low[TM][TN];  // the products of the first terms; the others
+  // what the bf16 terms drop (split3): one chain of ors per chunk where registers allow, so that none
+  // waits for another chunk's load
+  constexpr int kLostA = G == 1 ? 1 : CA, kLostB = G == 1 ? 1 : CB;
+  uint32_t lost_a[kLostA] = {}, lost_b[kLostB] = {};
   const int fr = lane % 16, fk = lane / 16;
 
   // acc = the tile's products over the group's slices; exact: with the fp32 instruction
@@ -298,12 +311,12 @@ __device__ __forceinline__ void gemmF32(ASrc A, BSrc B, int64_t R, int64_t Cn, i
 #pragma unroll
       for (int i = 0; i < CB; ++i) rb[i] = B.template chunk<kWhole>(i, k0, tab);
     };
-    auto put = [&](auto rows, float* base, int row, int col, const f32x4& v) {
+    auto put = [&](auto rows, float* base, int row, int col, const f32x4& v, uint32_t& lost) {
       if constexpr (kExact) {
         *reinterpret_cast<f32x4*>(&base[row * kPitch + col]) = v;
       } else {
         uint2 term[3];
-        split3(v, term);
+        split3(v, term, lost);
         constexpr int kRows = decltype(rows)::value;
         char* const p = reinterpret_cast<char*>(base) + runAt<kRows>(row, col / 8) + (col & 4) * 2;
 #pragma unroll
@@ -316,12 +329,14 @@ __device__ __forceinline__ void gemmF32(ASrc A, BSrc B, int64_t R, int64_t Cn, i
       if (kAllA || t < BM * kChunks) {
 #pragma unroll
         for (int i = 0; i < CA; ++i)
-          put(std::integral_constant<int, BM>{}, as, ASrc::row(t, i), ASrc::col(t, i), ra[i]);
+          put(std::integral_constant<int, BM>{}, as, ASrc::row(t, i), ASrc::col(t, i), ra[i],
+              lost_a[i % kLostA]);
       }
       if (kAllB || t < BN * kChunks) {
 #pragma unroll
         for (int i = 0; i < CB; ++i)
-          put(std::integral_constant<int, BN>{}, bs, BSrc::row(t, i), BSrc::col(t, i), rb[i]);
+          put(std::integral_constant<int, BN>{}, bs, BSrc::row(t, i), BSrc::col(t, i), rb[i],
+              lost_b[i % kLostB]);
       }
     };
     auto multiply = [&](int b) {
@@ -425,6 +440,10 @@ __device__ __forceinline__ void gemmF32(ASrc A, BSrc B, int64_t R, int64_t Cn, i
 #pragma unroll
     for (int j = 0; j < TN; ++j) acc[i][j] += low[i][j];
   bool bad = false;
+#pragma unroll
+  for (int i = 0; i < kLostA; ++i) bad = bad || (lost_a[i] & 0xFFFFu) != 0;
+#pragma unroll
+  for (int i = 0; i < kLostB; ++i) bad = bad || (lost_b[i] & 0xFFFFu) != 0;
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll

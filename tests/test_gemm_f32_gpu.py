@@ -64,6 +64,37 @@ def test_linear_f32_magnitudes(m, scale):
     check_linear(x, w, b)
 
 
+# exponents of the operands; the last bits of a normal value below 2^-110 lie below the smallest bf16
+# (2^-133), and below 2^-126 values are subnormal
+@pytest.mark.parametrize("m", [4, 40, 100, 300])
+@pytest.mark.parametrize("low,high", [(-108, 60), (-114, 60), (-120, 0), (-126, 60), (-132, 100),
+                                      (-140, 100)])
+def test_f32_products_of_tiny_operands(m, low, high):
+    if low + high < -100:  # results of 2^-120: their own roundings are subnormal steps of 2^-149
+        high += 60
+    x, w = rand((m, 256), 18) * 2.0 ** low, rand((80, 256), 19) * 2.0 ** high
+    tiny = x.double().abs().max()
+    assert 0 < tiny < 2.0 ** (low + 4)
+    check_linear(x, w, torch.zeros(80, device="cuda"))
+    check_linear(w, x, torch.zeros(m, device="cuda"))
+    check_linear(x[:, :251].contiguous(), w[:, :251].contiguous(), torch.zeros(80, device="cuda"))
+    close(run("matmul", {"a": x, "b": w.t().contiguous()}, {}), x.double() @ w.double().t(),
+          x.double().abs() @ w.double().abs().t(), 256)
+    # one tiny value among ordinary ones, in a column of w that is 2^100
+    x, w = rand((m, 64), 20), rand((80, 64), 21)
+    x[:, 5], w[:, 5] = x[:, 5] * 2.0 ** low, 2.0 ** 100
+    check_linear(x, w, torch.zeros(80, device="cuda"))
+
+
+@pytest.mark.parametrize("n,c,kern", [(3, 16, 3), (2, 3, 7)])
+def test_conv2d_f32_of_tiny_operands(n, c, kern):
+    x, k = rand((n, c, 12, 12), 22) * 2.0 ** -125, rand((70, c, kern, kern), 23) * 2.0 ** 60
+    out = run("conv2d", {"x": x, "w": k}, {"padding": [1, 1]})
+    ref, terms = (F.conv2d(p.double().cpu(), q.double().cpu(), padding=1).cuda()
+                  for p, q in ((x, k), (x.abs(), k.abs())))
+    close(out, ref, terms, c * kern * kern)
+
+
 @pytest.mark.parametrize("m", [4, 40, 100, 300])
 def test_linear_f32_infinities_and_nan(m):
     """Infinite and NaN operands, and sums past the fp32 range, give what fp32 arithmetic gives; the
