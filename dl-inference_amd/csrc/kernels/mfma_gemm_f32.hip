@@ -8,7 +8,7 @@
 //                        B = the input patch of each output pixel, gathered from NCHW x while
 //                        staging (never materialised); out NCHW
 //
-// The products run on the bf16 matrix cores as sums of three terms (below), six instructions at
+// The products run on the bf16 matrix cores as sums of three terms (below), eight instructions at
 // sixteen times the rate of the fp32 one, so a 64 x 64 tile is bound by staging as much as by the
 // matrix cores (of the CU cycles of 1000 x 4864 x 896: splitting and addresses 55%, LDS 41%, matrix
 // cores 40%): one tile size, fine enough that a few hundred tiles spread over 256 CUs. What overlaps
@@ -212,10 +212,16 @@ struct ConvPatch : AlongRows<ROWS> {
 // The products run on the bf16 matrix cores, which are 16 times as fast as the fp32 ones: an fp32
 // value is the exact sum of three bf16 terms, x = h + m + l (8 mantissa bits each, cut by
 // truncation, so that h never overflows), and
-//   x y = l h' + h l' + m m' + m h' + h m' + h h'  (+ m l' + l m' + l l', below 2^-23 x y, left out)
-// is six v_mfma_f32_16x16x32_bf16, h h' into one fp32 accumulator and the small products into another
-// one: the large sum is then rounded once per 32 products (with one accumulator for all six, 5 to 6
-// times, which showed: 3.9e-7 from float64 over the CNN against 2.2e-7 with the fp32 instruction).
+//   x y = l m' + m l' + l h' + h l' + m m' + m h' + h m' + h h'  (+ l l', below 2^-30 x y, left out)
+// is eight v_mfma_f32_16x16x32_bf16, h h' into one fp32 accumulator and the small products into another
+// one: the large sum is then rounded once per 32 products (with one accumulator for all, as often as
+// there are products, which showed: 3.9e-7 from float64 over the CNN against 2.2e-7 with the fp32
+// instruction). The two smallest products reach 2^-21 x y and always have its sign; without them one
+// product was off by up to 8 half-ulps (K = 1: 6.0e-8 in the 2-norm, 2.5e-8 with the fp32 instruction
+// and with these two). Distance from float64 over random normal operands, the fp32 instruction / here:
+// K = 4 3.9e-8 / 2.6e-8, K = 32 1.0e-7 / 3.9e-8, K = 256 2.8e-7 / 6.3e-8, K = 4864 3.2e-7 / 1.1e-7. They
+// cost 12 to 14% where the matrix cores bind (4096^3 841 -> 968 us, 1272 with the fp32 instruction), 1 to
+// 8% elsewhere.
 // An infinity or NaN among the operands, or a sum past the fp32 range, makes a result of the tile
 // non-finite; such a tile is computed again with the fp32 instruction, whose rules for them hold. So is
 // a tile with operands below 2^-110, whose last bits lie below the smallest bf16 (2^-133): they are
@@ -380,9 +386,9 @@ __device__ __forceinline__ void gemmF32(ASrc A, BSrc B, int64_t R, int64_t Cn, i
           for (int j = 0; j < TN; ++j)
             bt[j][q] = *reinterpret_cast<const U128*>(bp + q * 64 * BN + j * 256);
         }
-        constexpr int kTerms[5][2] = {{2, 0}, {0, 2}, {1, 1}, {1, 0}, {0, 1}};
+        constexpr int kTerms[7][2] = {{2, 1}, {1, 2}, {2, 0}, {0, 2}, {1, 1}, {1, 0}, {0, 1}};
 #pragma unroll
-        for (int q = 0; q < 5; ++q)
+        for (int q = 0; q < 7; ++q)
 #pragma unroll
           for (int i = 0; i < TM; ++i)
 #pragma unroll

@@ -64,6 +64,26 @@ def test_linear_f32_magnitudes(m, scale):
     check_linear(x, w, b)
 
 
+@pytest.mark.parametrize("m,n,k", [(4, 70, 1), (4, 70, 4), (40, 70, 2), (100, 65, 4), (100, 65, 3),
+                                   (300, 600, 12), (900, 1200, 4)])
+@pytest.mark.parametrize("worst", [False, True])
+def test_short_f32_products_keep_every_term(m, n, k, worst):
+    """Products of one sign: h h' and the small terms are rounded once each and once more together, at
+    most 2^-24 of the sum of the products apiece, the small terms' 2^-7 of that. Without m l' and
+    l m' an operand of 1.0000 1111 1111 1111 1111 (`worst`) loses 2^-21 of every product."""
+    x, w = (1 + torch.rand(s, generator=torch.Generator().manual_seed(i)).cuda()
+            for i, s in ((24, (m, k)), (25, (n, k))))
+    if worst:
+        x[:], w[:] = (torch.tensor(0x3F80FFFF, dtype=torch.int32).view(torch.float32).item(),) * 2
+    ref = x.double() @ w.double().t()
+    bound = (2 + 2.0 ** -6) * 2.0 ** -24 * ref
+    for out in (run("linear", {"x": x, "w": w}, {}),
+                run("matmul", {"a": x, "b": w.t().contiguous()}, {}),
+                run("conv2d", {"x": x.t().reshape(1, k, 1, m).contiguous(), "w": w.view(n, k, 1, 1)},
+                    {}).view(n, m).t()):
+        assert ((out.double() - ref).abs() <= bound).all()
+
+
 # exponents of the operands; the last bits of a normal value below 2^-110 lie below the smallest bf16
 # (2^-133), and below 2^-126 values are subnormal
 @pytest.mark.parametrize("m", [4, 40, 100, 300])
