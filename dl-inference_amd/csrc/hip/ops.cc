@@ -211,6 +211,18 @@ size_t partBytesF32(const PlanF32& p, int64_t rows, int64_t cols) {
 
 constexpr int64_t kMaxGridY = 65535;
 
+// fp32 linear and matmul: 64-row tiles in grid.y, in two launches past what that holds (the rows of the
+// 128-row tiles that these calls had).
+constexpr int64_t kGridRowsF32 = 64 * kMaxGridY, kMaxRowsF32 = 2 * kGridRowsF32;
+template <class Launch>
+int byRowsF32(const void* x, void* out, int64_t m, int64_t n, int64_t k, const Launch& go) {
+  for (int64_t r = 0; r < m; r += kGridRowsF32)
+    if (int rc = go(static_cast<const float*>(x) + r * k, static_cast<float*>(out) + r * n,
+                    m - r < kGridRowsF32 ? m - r : kGridRowsF32))
+      return rc;
+  return 0;
+}
+
 // elements of a 16-byte chunk of a float dtype
 int64_t chunkOf(int dtype) { return dtype == DLI_F32 ? 4 : 8; }
 
@@ -682,18 +694,21 @@ int dli_hip_linear_act(int dtype, int out_dtype, const void* x, const void* w, c
   if (x == nullptr || w == nullptr || out == nullptr) return badArg("linear", "NULL pointer");
   const int out_f32 = out_dtype == DLI_F32 ? 1 : 0;
   const int relu = activation == DLI_ACT_RELU ? 1 : 0;
-  if (dtype == DLI_F32 && (m + 63) / 64 <= kMaxGridY) {
-    const bool vec = k > 0 && k % 4 == 0 && aligned16(x) && aligned16(w);
-    const PlanF32 p =
-        planF32(m, n, k, vec, true, partsHeldF32(workspace, workspace_bytes, m, n));
-    const int rc = launch(k_f32_linear[p.form],
-                          {static_cast<unsigned>((n + 63) / 64),
-                           static_cast<unsigned>((m + p.tile_rows - 1) / p.tile_rows),
-                           static_cast<unsigned>(p.parts)},
-                          {p.threads}, 0, stream, x, w, bias, out, workspace, m, n, k, p.per, relu);
-    if (rc != 0 || p.parts == 1) return rc;
-    return launch(k_splitk_reduce, {strideBlocks((m * n + 3) / 4)}, {256}, 0, stream, workspace,
-                  bias, out, m, n, static_cast<int>(p.parts), relu);
+  if (dtype == DLI_F32 && m <= kMaxRowsF32) {
+    return byRowsF32(x, out, m, n, k, [&](const void* xr, void* outr, int64_t rows) {
+      const bool vec = k > 0 && k % 4 == 0 && aligned16(xr) && aligned16(w);
+      const PlanF32 p =
+          planF32(rows, n, k, vec, true, partsHeldF32(workspace, workspace_bytes, rows, n));
+      const int rc = launch(k_f32_linear[p.form],
+                            {static_cast<unsigned>((n + 63) / 64),
+                             static_cast<unsigned>((rows + p.tile_rows - 1) / p.tile_rows),
+                             static_cast<unsigned>(p.parts)},
+                            {p.threads}, 0, stream, xr, w, bias, outr, workspace, rows, n, k, p.per,
+                            relu);
+      if (rc != 0 || p.parts == 1) return rc;
+      return launch(k_splitk_reduce, {strideBlocks((rows * n + 3) / 4)}, {256}, 0, stream,
+                    workspace, bias, outr, rows, n, static_cast<int>(p.parts), relu);
+    });
   }
   int rc;
   const bool h16 = dtype == DLI_BF16 || dtype == DLI_F16;
@@ -727,12 +742,14 @@ int dli_hip_matmul(int dtype, const void* a, const void* b, void* out, int64_t m
   if (m < 0 || n < 0 || k < 0) return badArg("matmul", "negative size");
   if (m == 0 || n == 0) return 0;
   if (a == nullptr || b == nullptr || out == nullptr) return badArg("matmul", "NULL pointer");
-  if (dtype == DLI_F32 && (m + 63) / 64 <= kMaxGridY) {
-    const bool vec = k > 0 && k % 4 == 0 && aligned16(a);
-    const PlanF32 p = planF32(m, n, k, vec, false, 1);
-    return launch(k_f32_matmul[p.form],
-                  {static_cast<unsigned>((n + 63) / 64), static_cast<unsigned>((m + 63) / 64)},
-                  {p.threads}, 0, stream, a, b, out, m, n, k);
+  if (dtype == DLI_F32 && m <= kMaxRowsF32) {
+    return byRowsF32(a, out, m, n, k, [&](const void* ar, void* outr, int64_t rows) {
+      const bool vec = k > 0 && k % 4 == 0 && aligned16(ar);
+      const PlanF32 p = planF32(rows, n, k, vec, false, 1);
+      return launch(k_f32_matmul[p.form],
+                    {static_cast<unsigned>((n + 63) / 64), static_cast<unsigned>((rows + 63) / 64)},
+                    {p.threads}, 0, stream, ar, b, outr, rows, n, k);
+    });
   }
   DeviceKernel* kt = k_gemm.pick(dtype);
   if (kt == nullptr) return badDtype("matmul", dtype);

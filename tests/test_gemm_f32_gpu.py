@@ -153,3 +153,17 @@ def test_conv2d_f32_forms(n, c, h, w, oc, kern, stride, pad):
                            padding=pad).cuda()
                   for p, q, r in ((x, k, b), (x.abs(), k.abs(), b.abs())))
     close(out, ref.clamp_min(0), terms, c * kern * kern)
+
+
+def test_f32_rows_past_one_grid():
+    """More than 64 x 65535 rows go in two launches; more than 128 x 65535 are refused."""
+    m, n, k = 64 * 65535 + 70, 3, 4
+    x, w, b = rand((m, k), 26), rand((n, k), 27), rand((n,), 28)
+    check_linear(x, w, b, relu=True)
+    close(run("matmul", {"a": x, "b": w.t().contiguous()}, {}), x.double() @ w.double().t(),
+          x.double().abs() @ w.double().abs().t(), k)
+    x = torch.zeros(128 * 65535 + 1, k, device="cuda")
+    with pytest.raises(ValueError, match="m too large"):
+        run("linear", {"x": x, "w": w}, {})
+    with pytest.raises(ValueError, match="m too large"):
+        run("matmul", {"a": x, "b": w.t().contiguous()}, {})
