@@ -260,6 +260,21 @@ int unary(FloatKernels& kernels, FloatKernels& wide, const char* op, int dtype, 
 // Rows (queries x heads of a KV group) per workgroup: 128, or 64 for units of at most 64 rows.
 int64_t packedTile(int64_t rows) { return rows > 64 ? 128 : 64; }
 
+// The same without key splits (contiguous keys): 64 also while that leaves CUs without a second
+// workgroup, since a tile of 128 rows walks the same keys at almost twice the time of each. In us with
+// 128 / 64 rows, 28 / 4 heads of 128: 16 x 16 8.8 / 6.4 (the row kernel 6.5), 2 x 64 x 64 9.0 / 6.5, 500 x
+// 500 27.9 / 20.0, 16 queries over 4096 keys 174 / 124; 1000 x 1000 (438 tiles of 64 rows) 49.6 with 128.
+int64_t denseTile(int64_t rows, int64_t units) {
+  return (rows + 63) / 64 * units <= 256 ? 64 : packedTile(rows);
+}
+
+// fp32 attention of few keys and few query rows times keys stays on the row kernel: the packed kernel's
+// tiles cost a short prompt what 64 keys cost. In us packed / row, 28 / 4 heads: head_dim 64 16 x 16 6.3 /
+// 4.5, 40 x 40 (44800) 6.4 / 6.0, 48 x 48 (64512) 6.4 / 6.5, 8 x 16 x 16 (57344) 6.5 / 7.0; head_dim 128
+// 16 x 16 9.8 / 6.0, 40 x 40 10.2 / 8.5, 8 x 16 x 16 10.1 / 10.7; 4 / 4 heads of 128 96 x 96 15.0 / 13.5,
+// 16 x 128 14.7 / 15.9.
+bool rowKernelF32(int64_t rows, int64_t keys) { return keys <= 96 && rows * keys <= 49152; }
+
 // Key splits for `blocks` row tiles over all (sequence, KV head) pairs and a cache of T 64-key tiles:
 // at most two workgroups per CU, and as many as the shorter walk (T / n tiles of 1 to 2.4 us) pays for
 // the partial results (their traffic and merge grow with n): n^2 <= 3 T, or, where the row tiles
@@ -824,6 +839,7 @@ static int attentionImpl(int dtype, const void* q, const void* k, const void* v,
   // fp32 with head_dim 64 or 128: the same on the fp32 matrix instruction.
   const bool f32 = dtype == DLI_F32;
   if (!out_bshd && (head_dim == 128 || (f32 && head_dim == 64)) && seq_q >= 16 &&
+      !(f32 && rowKernelF32(rows, seq_k)) &&
       packedForm(dtype, batch, q_heads, kv_heads, seq_q, seq_k, scale, q, k, v, out)) {
     dk::PackedAttentionArgs a{};
     a.q = q;
@@ -838,7 +854,7 @@ static int attentionImpl(int dtype, const void* q, const void* k, const void* v,
     a.splits = 1;
     a.scale_log2 = scale * 1.4426950408889634f;
     const int64_t unit_rows = seq_q * (q_heads / kv_heads);
-    const int64_t tile = f32 ? 64 : packedTile(unit_rows);
+    const int64_t tile = f32 ? 64 : denseTile(unit_rows, batch * kv_heads);
     DeviceKernel& kern = f32 ? (head_dim == 64 ? k_packed_f32_64 : k_packed_f32_128)
                              : (tile == 128 ? k_packed_dense128_r128 : k_packed_dense128);
     return launch(kern,

@@ -274,3 +274,26 @@ def test_probabilities_keep_fp32(d, paged):
     pa, pb = torch.exp(-c.double()), torch.exp(-c.double() - delta)
     ref = ((pa - pb) / (1 + pa + pb)).repeat_interleave(2, 1)[:, :, None, None]
     assert ((out.double() - ref).abs() <= 2.0 ** -7 * ref).all()
+
+
+# the lines of the dense rules: fp32 query rows x keys of 49152 (row kernel) and above, 96 keys and more; bf16 with 256
+# 64-row tiles and more (128-row tiles)
+@pytest.mark.parametrize("dtype,d,batch,hq,hkv,sq,sk", [
+    (torch.float32, 64, 2, 8, 2, 32, 96), (torch.float32, 64, 2, 8, 2, 33, 96),
+    (torch.float32, 128, 1, 3, 1, 16, 96), (torch.float32, 128, 1, 3, 1, 16, 97),
+    (torch.bfloat16, 128, 4, 64, 32, 64, 70), (torch.bfloat16, 128, 4, 64, 32, 65, 70)])
+def test_dense_rule_lines(dtype, d, batch, hq, hkv, sq, sk):
+    import dli
+
+    g = torch.Generator().manual_seed(51)
+    q, k, v = (torch.randn(batch, h, s, d, generator=g).to(dtype).to(DEV)
+               for h, s in ((hq, sq), (hkv, sk), (hkv, sk)))
+    out = run_attention({"q": q, "k": k, "v": v}, {"causal": True}, dli.Engine().load_plugin())
+    group = hq // hkv
+    mask = torch.ones(sq, sk, dtype=torch.bool, device=DEV).tril(sk - sq)
+    for h in range(hq):
+        score = torch.matmul(q[:, h].double(), k[:, h // group].double().transpose(1, 2).contiguous())
+        p = torch.softmax((score / d ** 0.5).masked_fill(~mask, -np.inf), -1)
+        ref = torch.matmul(p, v[:, h // group].double())
+        err = (out[:, h].double() - ref).norm()
+        assert err <= (1e-6 if dtype == torch.float32 else REL) * ref.norm()
