@@ -282,9 +282,12 @@ bool rowKernelF32(int64_t rows, int64_t keys) { return keys <= 96 && rows * keys
 // 3 queries of 28 / 4 heads of 128 over 4000 keys 25.3 / 21.3 (13 splits), 4 x 10 over 3000 30 / 25.2,
 // 14 / 2 heads of 64 over 4000 22.5 / 17.8, over 1000 12.2 / 10.8; 2 x 300 queries of 28 / 4 heads
 // (136 row tiles) over 64 keys 30.9 / 21.8 (unsplit), over 150 31.4 / 24.7, over 600 36.4 / 35.7.
+// Up to 4 tiles the merge costs more than any split gives (unsplit / split by the root): 2 queries of 14 /
+// 2 heads of 64 over 2 tiles 5.1 / 7.0, 4 tiles 7.0 / 8.4, 6 tiles 9.0 / 8.9; 2 x 100 of 28 / 4 heads of
+// 128 over 2 tiles 11.4 / 14.7, 4 tiles 15.9 / 19.0, 6 tiles 20.5 / 20.9.
 int64_t packedSplits(int64_t blocks, int64_t capacity) {
   const int64_t tiles = (capacity + dk::kPackedTileK - 1) / dk::kPackedTileK;
-  const int64_t most = blocks > 0 ? 512 / blocks : 1;
+  const int64_t most = blocks > 0 && tiles > 4 ? 512 / blocks : 1;
   int64_t splits = 1;
   while (splits < most && splits < 64 &&
          (blocks >= 128 ? 6 * (splits + 1) <= tiles : (splits + 1) * (splits + 1) <= 3 * tiles))

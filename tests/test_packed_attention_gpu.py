@@ -91,11 +91,12 @@ def test_paged_chunk_large_blocks_and_spare_capacity():
                 True)
 
 
-# the lines of the split rule: few row tiles (1, 2, 3 splits, then the most that 64 tiles give), and
-# 128 of them (1 and 2 splits)
+# the lines of the split rule: few row tiles (unsplit up to 4 key tiles, 3 splits of 5, then the most
+# that 64 tiles give), and 128 of them (1 and 2 splits)
 @pytest.mark.parametrize("d", [64, 128])
 @pytest.mark.parametrize("batch,hq,hkv,past,tiles", [
     (1, 4, 2, 50, 1), (1, 4, 2, 100, 2), (1, 4, 2, 180, 3), (1, 4, 2, 4000, 64),
+    (1, 4, 2, 253, 4), (1, 4, 2, 254, 5),
     (4, 64, 32, 40, 11), (4, 64, 32, 700, 12)])
 def test_paged_chunk_split_rule(d, batch, hq, hkv, past, tiles):
     case = paged_case(hq, hkv, d, 3, [past] * batch, True, capacity=64 * tiles)
