@@ -71,6 +71,7 @@ FloatKernels k_argmax("elementwise", "argmax");
 DeviceKernel k_argmax_rows_v4("elementwise", "argmax_f32_rows_v4");
 FloatKernels k_rms_norm("norm", "rms_norm");
 DeviceKernel k_rms_norm_rows("norm", "rms_norm_rows_bf16_k");
+DeviceKernel k_rms_norm_mid_rows("norm", "rms_norm_mid_rows_bf16_k");
 DeviceKernel k_rms_norm_wide_rows("norm", "rms_norm_wide_rows_bf16_k");
 DeviceKernel k_kv_append_tiles("attention", "kv_append_tiles_bf16_k");
 FloatKernels k_gemm("gemm", "gemm_tiled");
@@ -507,7 +508,10 @@ int dli_hip_rms_norm(int dtype, const void* x, const void* weight, void* out, in
       aligned16(weight) && aligned16(out)) {
     const int64_t groups = (rows + 3) / 4;
     const unsigned blocks = static_cast<unsigned>(groups < 65535 ? groups : 65535);
-    return launch(hidden <= 1024 ? k_rms_norm_rows : k_rms_norm_wide_rows, {blocks}, {256}, 0, stream, x, weight, out, rows,
+    DeviceKernel& kernel = hidden <= 1024   ? k_rms_norm_rows
+                           : hidden <= 2048 ? k_rms_norm_mid_rows
+                                            : k_rms_norm_wide_rows;
+    return launch(kernel, {blocks}, {256}, 0, stream, x, weight, out, rows,
                   static_cast<int>(hidden), eps);
   }
   const unsigned blocks = static_cast<unsigned>(rows < 65535 ? rows : 65535);

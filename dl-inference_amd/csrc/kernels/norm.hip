@@ -53,10 +53,12 @@ __device__ void rms_norm_impl(const void* x, const void* weight, void* out, int6
 // 16-byte chunks (chunk c of the row in lane c % 64), sum of squares reduced inside the wave
 // (no LDS, no barrier), 16-byte loads and stores. Per element the same arithmetic as the
 // block-per-row kernel: x * inv * w with inv = 1 / sqrt(mean(x^2) + eps), rounded once.
-// kRowChunks: chunks per lane, 2 (hidden <= 1024, fewer registers and so more rows in flight) or 8.
+// kRowChunks: chunks per lane, 2 (hidden <= 1024), 4 (<= 2048) or 8: fewer registers, and so more rows
+// in flight (8192 rows of 1032 with 8 chunks 9.5 us, with 4 7.5; of 1536 10.6 and 9.7).
 template <int kRowChunks>
-__device__ __forceinline__ void rms_norm_rows_bf16(const uint16_t* x, const uint16_t* weight, uint16_t* out,
-                                   int64_t rows, int hidden, float eps) {
+__device__ __forceinline__ void rms_norm_rows_bf16(const uint16_t* x, const uint16_t* weight,
+                                                   uint16_t* out, int64_t rows, int hidden,
+                                                   float eps) {
   const int lane = threadIdx.x % kWave;
   const int chunks = hidden / 8;
   for (int64_t r = static_cast<int64_t>(blockIdx.x) * 4 + threadIdx.x / kWave; r < rows;
@@ -65,7 +67,7 @@ __device__ __forceinline__ void rms_norm_rows_bf16(const uint16_t* x, const uint
     uint32_t v[kRowChunks][4];
     float sq = 0.f;
     // every chunk is requested before the first is used (a branch around each load made a row a
-    // chain of up to 8 round trips: 34 rows of 3584 7.3 us, 4.2 now); past the row: its last chunk
+    // chain of up to 8 round trips: 32 rows of 3584 4.8 us, 4.2 now); past the row: its last chunk
 #pragma unroll
     for (int c = 0; c < kRowChunks; ++c) {
       if (c * kWave >= chunks) break;  // uniform
@@ -113,6 +115,11 @@ extern "C" __global__ void __launch_bounds__(256)
     rms_norm_rows_bf16_k(const uint16_t* x, const uint16_t* weight, uint16_t* out, int64_t rows,
                          int hidden, float eps) {
   rms_norm_rows_bf16<2>(x, weight, out, rows, hidden, eps);
+}
+extern "C" __global__ void __launch_bounds__(256)
+    rms_norm_mid_rows_bf16_k(const uint16_t* x, const uint16_t* weight, uint16_t* out,
+                             int64_t rows, int hidden, float eps) {
+  rms_norm_rows_bf16<4>(x, weight, out, rows, hidden, eps);
 }
 extern "C" __global__ void __launch_bounds__(256)
     rms_norm_wide_rows_bf16_k(const uint16_t* x, const uint16_t* weight, uint16_t* out,

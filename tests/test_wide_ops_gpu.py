@@ -106,3 +106,15 @@ def test_kv_append_places_every_token(d, block, cap, s):
         entry = engine.kv_cache_entry("L")
         for name in expect:
             assert torch.equal(entry[name], expect[name]), (name, positions)
+
+
+# a row in one wave: 2, 4 and 8 chunks of 8 per lane, whole and with a rest
+@pytest.mark.parametrize("rows,hidden", [(5, 1024), (5, 1032), (2, 1536), (9, 2048), (5, 2056),
+                                         (3, 4088), (4, 4096), (70000, 1032)])
+def test_rms_norm_rows(rows, hidden):
+    x, w = rand((rows, hidden), "bfloat16", 9), rand((hidden,), "bfloat16", 10)
+    out = run("rms_norm", {"x": x, "w": w}, {"eps": 1e-6})[0].double()
+    xd = x.double()
+    ref = xd * torch.rsqrt((xd * xd).mean(-1, keepdim=True) + 1e-6) * w.double()
+    # the output's rounding, half a step; the fp32 sum and root are far below
+    assert ((out - ref).abs() <= 0.51 * ULP["bfloat16"] * ref.abs()).all()
