@@ -38,7 +38,8 @@ def check_linear(x, w, b, relu=False):
 
 
 @pytest.mark.parametrize("m,n,k", [
-    (1, 64, 4), (16, 65, 32), (16, 4096, 1024), (3, 10, 4096), (5, 896, 4864),  # 16-row tiles
+    (1, 64, 4), (16, 65, 32), (100, 65, 28),  # one slice: one group
+    (16, 65, 36), (1, 64, 64), (16, 4096, 1024), (3, 10, 4096), (5, 896, 4864),  # 16-row tiles
     (17, 63, 36), (64, 4096, 1024), (64, 10, 4096), (40, 130, 4100),  # one row tile
     (65, 64, 64), (77, 128, 896), (256, 1024, 100), (200, 896, 2000),  # K groups, parts
     (1000, 1100, 260), (513, 2050, 32),  # one group
