@@ -181,9 +181,6 @@ PlanF32 planF32(int64_t rows, int64_t cols, int64_t k, bool vec, bool linear, in
   p.threads = 256u * groups;
   // at least two slices per group (six where a workgroup has one)
   int64_t s = (many ? 768 : 256) / tiles;
-  // 16 rows over a long K: two workgroups per CU in turn even out the weights' stream (3 x 4096 x
-  // 16384 52 us, 65 in half as many parts; at K = 4096 19 against 16)
-  if (p.form == kM16 && s > 0 && slices / s >= 128) s *= 2;
   const int64_t least = many ? 6 : 2 * groups;
   if (s > slices / least) s = slices / least;
   if (s > max_parts) s = max_parts;

@@ -168,3 +168,18 @@ def test_f32_rows_past_one_grid():
         run("linear", {"x": x, "w": w}, {})
     with pytest.raises(ValueError, match="m too large"):
         run("matmul", {"a": x, "b": w.t().contiguous()}, {})
+
+
+# 16 slices per group and part, every one whole: the walks start at different slices; one column less:
+# all at the first
+@pytest.mark.parametrize("m,n,k", [(3, 2047, 16384), (16, 2048, 16384), (3, 2047, 16380)])
+def test_linear_f32_few_rows_over_a_long_k(m, n, k):
+    g = torch.Generator(device="cuda").manual_seed(29)
+    x, w, b = (torch.randn(s, generator=g, device="cuda") for s in ((m, k), (n, k), (n,)))
+    check_linear(x, w, b)
+    x[1, k - 5] = float("inf")  # the tiles again with the fp32 instruction
+    out = run("linear", {"x": x, "w": w, "b": b}, {})
+    assert torch.equal(out[1], float("inf") * w[:, k - 5])
+    rest = [0] + list(range(2, m))
+    close(out[rest], x[rest].double() @ w.double().t() + b.double(),
+          x[rest].double().abs() @ w.double().abs().t() + b.double().abs(), k)
