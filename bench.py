@@ -567,7 +567,7 @@ def bench_linear(args):
         "vs_baseline": None, "dtype": "f32", "data": "synthetic",
         "config": {"workload": "single linear layer fp32, x [64,1024] ~N(0,1), W [4096,1024] and "
                                "b [4096] ~U(-1/32,1/32), y = x W^T + b"},
-        "roofline": {"bound": "mfma", "kernel": "dli_hip_linear_act fp32 (16x16x4 f32 MFMA)",
+        "roofline": {"bound": "mfma", "kernel": "dli_hip_linear_act fp32 (three-term products, 16x16x32 bf16 MFMA)",
                      "achieved": round(tflops, 2), "peak": FP32_MFMA_PEAK_TFLOPS,
                      "unit": "TFLOP/s", "frac": round(tflops / FP32_MFMA_PEAK_TFLOPS, 4),
                      "traffic": None, "avg_us": round(us, 2), "flops_per_launch": flops,

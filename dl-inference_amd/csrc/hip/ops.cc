@@ -153,12 +153,11 @@ struct PlanF32 {
 //
 // Three workgroups of one K group (_g1) fit a CU and overlap each other's loads, staging and matrix
 // instructions; where the tiles alone are fewer, K parts make up for it, or, where the parts' traffic
-// would cost more, a second K group in the workgroup. In us: conv 384 x 4096 pixels x 1728 (384
-// tiles) 104 in one part, 68 + 5 for the sum in two; 256 x 4096 x 3456 (256 tiles) 108 with two
-// groups, 87 + 5 in three parts of one (these with gathers that branch; as they run now 55 + 6 and
-// 68 + 5); linear 1000 x 896 x 4864 (224 tiles) 65 with two groups, 68
-// to 72 in parts; 1000 x 896 x 896 17 with two groups, 21 with one, 23 in two parts; a conv of 3
-// images (24 tiles) 12 + 4 with two groups and 11 to 16 parts, 14 + 4 with one.
+// would cost more, a second K group in the workgroup. In us, parts with their sum: conv 384 x 4096 pixels
+// x 1728 (384 tiles) 65 in one part, 55 in two; 256 x 4096 x 3456 (256 tiles) 73 with two groups, 69 in
+// three parts of one; linear 1000 x 896 x 4864 (224 tiles) 76 with two groups, 97 with one, 79 in parts;
+// 1000 x 896 x 896 17 with two groups, 21 with one, 24 in parts; convs of 3 images (12 to 24 tiles) are
+// even: 13.5 with two groups and 12.8 with one for 384 x 192 x 1728, 15.4 either way for 256 x 192 x 3456.
 constexpr int64_t kMaxPartsF32 = 16;
 PlanF32 planF32(int64_t rows, int64_t cols, int64_t k, bool vec, bool linear, int64_t max_parts) {
   PlanF32 p{kG1, 256, 64, 1, k};

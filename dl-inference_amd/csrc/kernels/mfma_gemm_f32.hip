@@ -10,17 +10,17 @@
 //
 // The products run on the bf16 matrix cores as sums of three terms (below), eight instructions at
 // sixteen times the rate of the fp32 one, so a 64 x 64 tile is bound by staging as much as by the
-// matrix cores (of the CU cycles of 1000 x 4864 x 896: splitting and addresses 55%, LDS 41%, matrix
-// cores 40%): one tile size, fine enough that a few hundred tiles spread over 256 CUs. What overlaps
+// matrix cores (over 1000 x 4864 x 896: vector instructions 47%, LDS 32%, matrix cores 41% busy; at 4096^3
+// the products run at 1140 TFLOP/s of bf16, near what a library product reaches): one tile size, fine enough that a few hundred tiles spread over 256 CUs. What overlaps
 // loads, staging and products are three workgroups per CU or, when the tiles are few, G = 2 groups of
 // 256 threads that share a tile's K (_g2). Each group stages 32-wide K slices through LDS buffers of
 // its own, two slices in flight in registers, and the epilogue adds the groups' tiles in group order.
 // grid.z > 1 splits K further into a workspace (part); splitk_reduce_f32 / conv_splitk_reduce_f32 add
 // the parts in order. Every output is a fixed-order sum: results do not depend on timing.
 //
-// Measured in us, before (fp32 instruction, 4-byte loads) and now: linear 1000 x 4864 x 896 153 / 66,
-// 1000 x 896 x 4864 132 / 67, 64 x 4096 x 16384 113 / 77, 3 x 4096 x 16384 103 / 52; conv 384 x 4096
-// pixels x 1728 159 / 55 + 6; distance from float64 there 7.1e-7 / 2.5e-7 (K = 4864).
+// Measured in us, before (fp32 instruction, 4-byte loads) and now: linear 1000 x 4864 x 896 153 / 73,
+// 1000 x 896 x 4864 132 / 76, 8192 x 4864 x 896 700 / 514, 4096^3 1297 / 965, 3 x 4096 x 16384 103 / 45;
+// conv 384 x 4096 pixels x 1728 159 / 55 (with the sum of its parts), 256 x 6272 pixels x 2304 200 / 84.
 //
 //  _m16: 16 rows of A against 64 of B (a decode-sized x); _stream: nontemporal weight loads.
 //  _scalar: rows that are not 16-byte aligned or K % 4 != 0 (4-byte loads); convs of windows or images

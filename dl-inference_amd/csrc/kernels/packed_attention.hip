@@ -1,7 +1,8 @@
-// Attention of several query tokens per sequence on the matrix cores, over the paged KV cache
-// (a conversation's next turn, a prompt fed in chunks) or over contiguous keys and values
-// (prefill, head_dim 128): softmax(q k^T * scale [+ causal mask]) v (attention/kernel.py:6-62),
-// bf16 in and out, the masking of attention.hip.
+// Attention of several query tokens per sequence on the matrix cores: softmax(q k^T * scale [+ causal
+// mask]) v (attention/kernel.py:6-62), the masking of attention.hip, scale > 0. bf16 in and out, over the
+// paged KV cache (a conversation's next turn, a prompt fed in chunks; head_dim 64 and 128) or over
+// contiguous keys and values (prefill, head_dim 128); fp32 over contiguous keys and values (head_dim 64
+// and 128) in the form at the end of this file. What follows is the bf16 form.
 //
 // Rows: the group = Hq / Hkv query heads that share a KV head are packed with the queries into
 // one row index, row p = query p / group of head p % group, so a staged K / V tile serves every
@@ -26,7 +27,8 @@
 // Bound by the matrix cores (QK once, PV three times for the split) together with the exponentials of
 // the same waves. Measured against one wave per row with a scalar dot per key (attention.hip):
 //   paged, 2 x 300 new tokens over 3000 and 1500 cached, 28 / 4 heads, head_dim 128: 16.2 ms
-//     before, 70 us now (295 TFLOP/s of attention arithmetic) and 8 us for the merge of 3 splits;
+//     before, 74 us now (280 TFLOP/s of attention arithmetic; MFMA 22%, VALU 24% busy) and 8.7 us for
+//     the merge of 3 splits;
 //   dense causal, 2 x 1000 tokens, 28 / 4 heads, head_dim 128: 1.83 ms before, 60 us now.
 // Distance from float64 over these: 1.7e-3 (the rounding of the bf16 output) before and now.
 #include "packed_attention.h"

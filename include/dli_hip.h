@@ -194,18 +194,18 @@ size_t dli_hip_conv2d_workspace(int dtype, int64_t n, int64_t in_c, int64_t out_
 
 /* out[m, n] = sum_k x[m, k] * w[n, k] (+ bias[n]) (linear/kernel.py:6-44;
  * linear/template.cc:23-32). x, w, bias share `dtype`; out_dtype is dtype or DLI_F32.
- * bias may be NULL. fp32 accumulation. MFMA: fp32 always (16x16x4 f32); bf16 as a weight
- * stream for m <= 64 (K % 64 == 0), else as tiled bf16 MFMA (K % 8 == 0, 16-byte aligned). */
+ * bias may be NULL. fp32 accumulation. MFMA: fp32 always (three bf16 terms per operand, exact;
+ * m <= 8388480); bf16 and f16 as a weight stream of few rows (K % 64 == 0), else tiled (K % 8 == 0,
+ * 16-byte aligned). */
 int dli_hip_linear(int dtype, int out_dtype, const void* x, const void* w, const void* bias,
                    void* out, int64_t m, int64_t n, int64_t k, void* stream);
 
 /* dli_hip_linear followed by `activation` (DLI_ACT_*), fused into the epilogue on the tiled
  * MFMA paths. No counterpart in the reference (linear and relu are separate nodes there); the
  * plugin uses it for every linear node (attribute activation = "relu" to fuse). A workspace of
- * dli_hip_linear_workspace(dtype, m, n, k) bytes (no zeroing needed) lets fp32 shapes with few
- * output tiles and a long K, and bf16 shapes with 33-64 rows (or 9-32 rows and n >= 8192, which
- * run on the tiled GEMM) and few output tiles, split K over more workgroups, summing the splits
- * in a fixed order; with workspace NULL or smaller, fewer or no splits. */
+ * dli_hip_linear_workspace(dtype, m, n, k) bytes (no zeroing needed) lets shapes with few output
+ * tiles and a long K (fp32, and bf16 and f16 on the tiled GEMM) split K over more workgroups,
+ * summing the splits in a fixed order; with workspace NULL or smaller, fewer or no splits. */
 int dli_hip_linear_act(int dtype, int out_dtype, const void* x, const void* w, const void* bias,
                        void* out, int64_t m, int64_t n, int64_t k, int activation,
                        void* workspace, size_t workspace_bytes, void* stream);
@@ -399,7 +399,7 @@ int dli_hip_gate_up_silu(const void* hidden, const void* norm_weight, const void
  * head_dim]. One tiled MFMA GEMM with the RoPE and the head layout in its epilogue. Replaces
  * q/k/v_proj, the three reshapes, the three [B,S,H,D] -> [B,H,S,D] transposes and
  * rotary_embedding of a prompt layer (export.py:280-349; rotary/kernel.py:6-35). head_dim % 8
- * == 0, hidden_size % 8 == 0, pointers (except cos/sin) 16-byte aligned. */
+ * == 0, hidden_size % 8 == 0, pointers 16-byte aligned. */
 int dli_hip_qkv_rope_heads(const void* x, const void* w_qkv, const void* b_qkv, const float* cos,
                            const float* sin, int64_t max_pos, void* q_out, void* k_out,
                            void* v_out, int64_t batch, int64_t seq, int64_t hidden_size,

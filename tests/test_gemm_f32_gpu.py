@@ -24,8 +24,8 @@ def run(op, inputs, attrs):
 
 
 def close(out, ref, terms, k):
-    """Each product within 2^-22 of its value (what the split leaves out, the output's rounding) and
-    at most one rounding of the partial sums per product."""
+    """Each product within 2^-24 of its value (what the split leaves out is below 2^-30), at most one
+    rounding of the partial sums per product, and those of the parts, the bias and the output."""
     assert ((out.double() - ref).abs() <= (k + 4) * 2.0 ** -23 * terms).all()
     assert (out.double() - ref).norm() <= 1e-6 * terms.norm()
 
